@@ -325,6 +325,9 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
     UP(h.sph, sph);
     UP(h.csg, csg);
     UP(h.csg_children, csg_children);
+    UP(h.csg_slots, csg_slots);
+    UP(h.csg_tests, csg_tests);
+    UP(h.placed, placed);
     UP(h.csg_leaves, csg_leaves);
     UP(h.csg_leaf_range, csg_leaf_range);
     UP(h.shade_tris, shade_tris);
@@ -428,6 +431,17 @@ extern "C" int pvx_scene_get_stats(const pvx_scene *s, pvx_scene_stats *out) {
     return PVX_OK;
 }
 
+// Rays per wavefront of a launch of n rays on a grid of `grid` blocks: 64,
+// halved while the grid still holds every wavefront at once.  A wavefront
+// runs every path that any of its rays takes, so below a full grid fewer rays
+// each end sooner (plain radiosity of the 5,000-box room, whose rounds gather
+// some ten thousand rays: 53 ms with 64 rays per wavefront, 45 ms so).
+static uint32_t rays_per_wave(size_t n, uint32_t grid) {
+    uint32_t r = 64;
+    while (r > 1 && n <= (size_t)grid * (kBlock / 64) * (r / 2)) r /= 2;
+    return r;
+}
+
 // One closest-hit launch with an explicit traversal variant and grid.
 // variant: PVX_TRAVERSAL_DEFAULT (by scene content and ray kind), _WIDE_WW,
 // _WIDE_STEP (4-wide tree; triangle/sphere scenes) or _BINARY (binary tree,
@@ -438,10 +452,17 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
                           hipStream_t st, uint32_t variant, uint32_t grid, int32_t *spill = nullptr) {
     int r;
     if (!spill && (r = scene_spill(s, st, &spill))) return r;
-    uint32_t nblocks = (uint32_t)std::min<size_t>(grid, (n + kBlock - 1) / kBlock);
+    const uint32_t level = kernel_level(s->view);
+    // Walks of any primitive kind whose stack fits in LDS need no spill area
+    // per resident thread, so the launch covers all rays and the hardware
+    // hands out the wavefronts as others end: a ray's cost varies a hundredfold
+    // there (10,000-leaf CSG field, 921,600 rays: 1.89 ms on the persistent
+    // grid, 1.67 ms so).
+    if (!s->use_kd && level >= 2 && s->host.depth + 1 <= (uint32_t)kStackLds) grid = 0x7FFFFFFFu;
+    const uint32_t wave_rays = !s->use_kd && level >= 1 ? rays_per_wave(n, s->grid) : 64u;
+    uint32_t nblocks = (uint32_t)std::min<size_t>(grid, (n + 4 * wave_rays - 1) / (4 * wave_rays));
     const bool flags = s->view.any_flags != 0 && (ray_kind != PVX_RAY_PRIMARY || kinds);
     TraceKernel k{kWalkStep4, flags, kCount, false};
-    const uint32_t level = kernel_level(s->view);
     if (s->use_kd)
         k.walk = kWalkKd;
     else if (level >= 3)
@@ -463,6 +484,7 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
     ta.kind = ray_kind;
     ta.kinds = kinds;
     ta.n = (uint32_t)n;
+    ta.wave_rays = wave_rays;
     ta.hits = hits;
     ta.spill = spill;
     ta.node_visits = nv;
@@ -608,6 +630,7 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     const uint32_t grid = grid_blocks ? grid_blocks : next ? s->grid : 2 * s->grid;
     const uint32_t nb = (uint32_t)std::min<size_t>(grid, ((size_t)n_rays + kBlock - 1) / kBlock);
     TraceArgs ta{};
+    ta.wave_rays = 64;
     ta.sv = s->view;
     ta.n = n_rays;
     ta.spill = spill;
@@ -812,6 +835,7 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
                                         : kWalkStep4,
                         flags, kCount, true};
     TraceArgs ta{};
+    ta.wave_rays = 64;
     ta.views = views;
     ta.chunks = chunks;
     ta.clocks = clk;

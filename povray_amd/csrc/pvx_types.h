@@ -41,6 +41,7 @@ enum PrimKind : uint32_t {
     kPrimQuadric = 9,    // quadric (outside the BVH)
     kPrimPolygon = 10,   // polygon, by reference
     kPrimRevolution = 11,// lathe or sor, by reference
+    kPrimCsgLeaf = 12,   // one leaf of a bounded CSG object (its csg_children slot)
 };
 
 struct alignas(16) Node {
@@ -124,9 +125,27 @@ struct SphRec {
     double pad[3];
 };
 struct RefRec {
-    uint32_t index; // index into the kind's shape array
-    uint32_t pad[13];
+    uint32_t index;     // index into the kind's shape array; kPrimCsgLeaf: the csg_children slot
+    uint32_t type;      // object type; kPrimCsgLeaf: the leaf's
+    uint32_t shape;     // index into that type's shape array
+    float lo[3], hi[3]; // the record's FP32 box, as the tree's leaves bound it
+    uint32_t rec;       // boxes and tori: index into placed, else kNoRec
+    uint32_t rflags;    // ... and its kPlaced* flags
+    uint32_t pad[3];
 };
+constexpr uint32_t kNoRec = 0xFFFFFFFFu;
+
+// A box or torus with its placement in one record, so that a test waits for
+// one load after its primitive's instead of two (shape record, then matrix):
+// the upper 4 x 3 of the inverse (rows of xforms[].inv) and c1, c2 (box) or
+// R, r (torus).
+constexpr uint32_t kPlacedXf = 1u;    // has a transform
+constexpr uint32_t kPlacedSturm = 2u; // torus solved by Sturm sequences
+struct alignas(16) PlacedRec {
+    double inv[12];
+    double q[6];
+};
+static_assert(sizeof(PlacedRec) == 144, "placed record is 144 B");
 
 struct alignas(16) PrimRec {
     union {
@@ -251,6 +270,27 @@ struct CsgChild {
     uint32_t node; // CSG node that owns this slot
 };
 
+// One operand test of a CSG filter program and where to go after it: an
+// index into csg_tests, kCsgUp (this node's filter passed) or kCsgDrop.
+// what: object type | PVX_FLAG_INVERTED set << 8 | kPlaced* flags << 16.
+constexpr uint32_t kCsgUp = 0xFFFFFFFFu, kCsgDrop = 0xFFFFFFFEu;
+struct CsgTest {
+    uint32_t what;
+    uint32_t index; // boxes and tori: placed record; else the shape's index
+    uint32_t next_in, next_out;
+};
+// A CSG operand: the filter program of its node (`start`; the operand's own
+// tests [skip, skip_to) are left out), the operand that stands for that node
+// in the next enclosing intersection or merge (`up`, -1 at the root), and the
+// operand's own shape.  Programs are per node, so their total size is linear
+// in the tree.
+struct CsgSlot {
+    uint32_t start, skip, skip_to;
+    int32_t up;
+    uint32_t type, shape, rec, rflags;
+};
+static_assert(sizeof(CsgSlot) == 32, "CSG slot is 32 B");
+
 // Smooth-normal data of a mesh triangle (Mesh_Triangle_Struct fields used by
 // Mesh::Normal / Smooth_Mesh_Normal, core/shape/mesh.cpp:380-420, 2366-2394),
 // indices into the scene-wide vertex / normal arrays.
@@ -322,6 +362,9 @@ struct SceneView {
     const double *sph; // sphere array (cx, cy, cz, r) per sphere, for CSG leaves
     const CsgNode *csg;
     const CsgChild *csg_children;
+    const CsgSlot *csg_slots;        // per csg_children slot
+    const CsgTest *csg_tests;        // the filter programs
+    const PlacedRec *placed;         // boxes and tori with their placement
     const uint32_t *csg_leaves;      // leaf slots of each CSG root, contiguous
     const uint32_t *csg_leaf_range;  // 2 per CSG node: [begin, end) into csg_leaves
     const ShadeTri *shade_tris;      // per mesh triangle (global index)

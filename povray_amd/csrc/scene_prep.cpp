@@ -1018,6 +1018,101 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         out.csg_leaf_range[2 * i + 1] = (uint32_t)out.csg_leaves.size();
     }
 
+    // --- boxes and tori with their placement --------------------------------
+    std::vector<uint32_t> box_rec(out.boxes.size(), kNoRec), torus_rec(out.tori.size(), kNoRec);
+    // (record, flags) of a box or torus; kNoRec for other types
+    auto placed = [&](uint32_t type, uint32_t index) -> std::pair<uint32_t, uint32_t> {
+        if (type != PVX_BOX && type != PVX_TORUS) return {kNoRec, 0u};
+        const bool box = type == PVX_BOX;
+        const int32_t xf = box ? out.boxes[index].xf : out.tori[index].xf;
+        const uint32_t flags = (xf >= 0 ? kPlacedXf : 0u) | (!box && out.tori[index].sturm ? kPlacedSturm : 0u);
+        uint32_t &rec = (box ? box_rec : torus_rec)[index];
+        if (rec == kNoRec) {
+            rec = (uint32_t)out.placed.size();
+            PlacedRec r;
+            std::memset(&r, 0, sizeof r);
+            if (xf >= 0)
+                for (int k = 0; k < 4; k++)
+                    for (int a = 0; a < 3; a++) r.inv[3 * k + a] = out.xforms[xf].inv[4 * k + a];
+            if (box)
+                for (int a = 0; a < 3; a++) {
+                    r.q[a] = out.boxes[index].c1[a];
+                    r.q[3 + a] = out.boxes[index].c2[a];
+                }
+            else {
+                r.q[0] = out.tori[index].R;
+                r.q[1] = out.tori[index].r;
+            }
+            out.placed.push_back(r);
+        }
+        return {rec, flags};
+    };
+
+    // --- CSG filter programs (CsgTest) ----------------------------------------
+    // A node's program is written back to front: `emit` puts the tests of one
+    // operand before those already there and returns where they start, given
+    // where to go when p is inside it and when it is not.
+    out.csg_slots.resize(d.n_csg_children);
+    std::vector<uint32_t> node_start(d.n_csg, kCsgUp);
+    for (uint32_t i = 0; i < d.n_csg; i++) {
+        const CsgNode &n = out.csg[i];
+        if (n.op == PVX_CSG_UNION) continue;
+        std::vector<CsgTest> rev; // reversed; entry k of m is at base + m - 1 - k
+        // labels below kCsgDrop count entries of `rev` from its end of program
+        std::function<uint32_t(uint32_t, uint32_t, uint32_t)> emit = [&](uint32_t slot, uint32_t in,
+                                                                          uint32_t no) -> uint32_t {
+            const CsgChild &c = out.csg_children[slot];
+            if (c.type == PVX_CSG) {
+                const CsgNode &m = out.csg[c.index];
+                const bool all = m.op == PVX_CSG_INTERSECTION; // intersection: every operand; union, merge: any
+                uint32_t at = all ? in : no;                   // after the last operand
+                for (uint32_t k = m.count; k-- > 0;) at = all ? emit(m.first + k, at, no) : emit(m.first + k, in, at);
+                return at;
+            }
+            const auto pr = placed(c.type, c.index);
+            rev.push_back(CsgTest{c.type | ((c.flags & PVX_FLAG_INVERTED) ? 1u << 8 : 0u) | pr.second << 16,
+                                  pr.first != kNoRec ? pr.first : c.index, in, no});
+            return (uint32_t)rev.size() - 1;
+        };
+        uint32_t at = kCsgUp;
+        std::vector<uint32_t> seg(n.count + 1, kCsgUp); // where each operand's tests start
+        for (uint32_t k = n.count; k-- > 0;) {
+            at = n.op == PVX_CSG_MERGE ? emit(n.first + k, kCsgDrop, at) : emit(n.first + k, at, kCsgDrop);
+            seg[k] = at;
+        }
+        const uint32_t base = (uint32_t)out.csg_tests.size(), m = (uint32_t)rev.size();
+        auto label = [&](uint32_t l) { return l >= kCsgDrop ? l : base + (m - 1 - l); };
+        for (uint32_t k = m; k-- > 0;) {
+            CsgTest t = rev[k];
+            t.next_in = label(t.next_in);
+            t.next_out = label(t.next_out);
+            out.csg_tests.push_back(t);
+        }
+        node_start[i] = label(at);
+        for (uint32_t k = 0; k < n.count; k++) {
+            out.csg_slots[n.first + k].skip = label(seg[k]);
+            out.csg_slots[n.first + k].skip_to = label(seg[k + 1]);
+        }
+    }
+    for (uint32_t i = 0; i < d.n_csg; i++) {
+        const CsgNode &n = out.csg[i];
+        int32_t up = n.parent_slot; // past the unions, which filter nothing
+        while (up >= 0 && out.csg[out.csg_children[up].node].op == PVX_CSG_UNION)
+            up = out.csg[out.csg_children[up].node].parent_slot;
+        for (uint32_t k = 0; k < n.count; k++) {
+            CsgSlot &s = out.csg_slots[n.first + k];
+            const CsgChild &c = out.csg_children[n.first + k];
+            s.start = node_start[i];
+            if (n.op == PVX_CSG_UNION) s.skip = s.skip_to = kCsgUp;
+            s.up = up;
+            s.type = c.type;
+            s.shape = c.index;
+            const auto pr = placed(c.type, c.index);
+            s.rec = pr.first;
+            s.rflags = pr.second;
+        }
+    }
+
     // --- bounds of shapes (FP64, conservative) ------------------------------
     // Two bounds per shape: S bounds its surfaces (where hits can lie), V
     // bounds the region where Inside can be true.  A CSG hit lies on a child
@@ -1106,11 +1201,71 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         return Bnd{S, V};
     };
 
+    // A bounded CSG object of spheres, boxes, tori and cones enters the tree as
+    // one primitive per leaf, each bounded by the leaf's surface inside the
+    // regions of its siblings in the intersections above it: a ray then meets
+    // only the leaves whose box it crosses, nearest first, instead of every
+    // leaf of every object it passes.  Objects with other leaves stay whole
+    // (a disc's box does not bound its half-space, planes and quadrics are
+    // unbounded, lathes and sors depend on being CSG operands).  The boxes
+    // are widened by 1e-4 of their size: a leaf's computed hit may lie off
+    // its surface by the root finder's error (below 1e-6 of the size).
+    struct CsgPart {
+        uint32_t slot;
+        DBox box;
+    };
+    std::function<bool(uint32_t, const DBox &, std::vector<CsgPart> &)> split_csg =
+        [&](uint32_t node, const DBox &clip, std::vector<CsgPart> &parts) -> bool {
+        const CsgNode &n = out.csg[node];
+        for (uint32_t k = 0; k < n.count; k++) {
+            const CsgChild &c = out.csg_children[n.first + k];
+            DBox b = clip;
+            if (n.op == PVX_CSG_INTERSECTION)
+                for (uint32_t j = 0; j < n.count; j++) {
+                    const CsgChild &sib = out.csg_children[n.first + j];
+                    if (j != k) b = meet(b, shape_bnd(sib.type, sib.index, sib.flags).V);
+                }
+            if (c.type == PVX_CSG) {
+                if (!split_csg(c.index, b, parts)) return false;
+                continue;
+            }
+            if (c.type != PVX_SPHERE && c.type != PVX_BOX && c.type != PVX_TORUS && c.type != PVX_CONE) return false;
+            b = meet(b, leaf_box(c.type, c.index));
+            bool empty = false;
+            for (int a = 0; a < 3; a++) {
+                const double pad = 1.0e-4 * std::fabs(b.hi[a] - b.lo[a]) +
+                                   1.0e-6 * std::max(std::fabs(b.lo[a]), std::fabs(b.hi[a]));
+                b.lo[a] -= pad;
+                b.hi[a] += pad;
+                empty = empty || !(b.lo[a] <= b.hi[a]);
+            }
+            if (!empty) parts.push_back(CsgPart{n.first + k, b});
+        }
+        return true;
+    };
+    const bool bvh_accel = !opts || opts->accel == PVX_ACCEL_BVH;
+
     // --- primitives ------------------------------------------------------------
     std::vector<PrimRec> prims;
     std::vector<float> plo, phi;
     auto add_prim = [&](const PrimRec &p, const float *lo, const float *hi) {
         prims.push_back(p);
+        const uint32_t kind = p.kind_axis & 15u;
+        if (kind != kPrimTriangle && kind != kPrimSphere) {
+            RefRec &r = prims.back().ref;
+            for (int k = 0; k < 3; k++) {
+                r.lo[k] = lo[k];
+                r.hi[k] = hi[k];
+            }
+            if (kind != kPrimCsgLeaf) {
+                const pvx_object &ob = d.objects[p.obj];
+                const auto pr = placed(ob.type, ob.index);
+                r.type = ob.type;
+                r.shape = ob.index;
+                r.rec = pr.first;
+                r.rflags = pr.second;
+            }
+        }
         plo.insert(plo.end(), lo, lo + 3);
         phi.insert(phi.end(), hi, hi + 3);
     };
@@ -1167,11 +1322,25 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
                 // an empty surface bound: the object can never be hit
                 break;
             }
+            out.has_complex = 2;
+            std::vector<CsgPart> parts;
+            if (bvh_accel && split_csg(ob.index, DBox::unbounded(), parts)) {
+                for (const CsgPart &part : parts) {
+                    pr.kind_axis = kPrimCsgLeaf;
+                    pr.ref.index = part.slot;
+                    pr.ref.type = out.csg_slots[part.slot].type;
+                    pr.ref.shape = out.csg_slots[part.slot].shape;
+                    pr.ref.rec = out.csg_slots[part.slot].rec;
+                    pr.ref.rflags = out.csg_slots[part.slot].rflags;
+                    to_fbox(part.box, lo, hi);
+                    add_prim(pr, lo, hi);
+                }
+                break;
+            }
             pr.kind_axis = kPrimCsg;
             pr.ref.index = ob.index;
             to_fbox(b, lo, hi);
             add_prim(pr, lo, hi);
-            out.has_complex = 2;
             break;
         }
         case PVX_PLANE:

@@ -41,6 +41,9 @@ struct HostScene {
     std::vector<double> sph; // 4 per sphere: centre, radius
     std::vector<CsgNode> csg;
     std::vector<CsgChild> csg_children;
+    std::vector<CsgSlot> csg_slots;
+    std::vector<CsgTest> csg_tests;
+    std::vector<PlacedRec> placed;
     std::vector<uint32_t> csg_leaves;
     std::vector<uint32_t> csg_leaf_range;
     std::vector<ShadeTri> shade_tris;

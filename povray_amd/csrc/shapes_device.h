@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "poly_device.h"
 #include "pvx_types.h"
 
 namespace pvx {
@@ -34,6 +35,18 @@ __device__ inline D3 xf_dir(const double *m, D3 p) {
     return D3{p.x * m[0] + p.y * m[4] + p.z * m[8],
               p.x * m[1] + p.y * m[5] + p.z * m[9],
               p.x * m[2] + p.y * m[6] + p.z * m[10]};
+}
+
+// The same with a PlacedRec's inverse (the rows' first three columns).
+__device__ inline D3 pl_point(const double *v, D3 p) {
+    return D3{p.x * v[0] + p.y * v[3] + p.z * v[6] + v[9],
+              p.x * v[1] + p.y * v[4] + p.z * v[7] + v[10],
+              p.x * v[2] + p.y * v[5] + p.z * v[8] + v[11]};
+}
+__device__ inline D3 pl_dir(const double *v, D3 p) {
+    return D3{p.x * v[0] + p.y * v[3] + p.z * v[6],
+              p.x * v[1] + p.y * v[4] + p.z * v[7],
+              p.x * v[2] + p.y * v[5] + p.z * v[8]};
 }
 
 // ---------------------------------------------------------------------------
@@ -102,10 +115,10 @@ __device__ inline int sphere_hits(D3 c, double r, D3 o, D3 d, double *out) {
     if (!(thc2 > kEpsilon)) return 0;
     double hc = sqrt(thc2);
     double d1 = tca - hc, d2 = tca + hc;
-    int n = 0;
-    if (d1 > 1.0e-6 && d1 < kMaxDistance) out[n++] = d1;
-    if (d2 > 1.0e-6 && d2 < kMaxDistance) out[n++] = d2;
-    return n;
+    const bool k1 = d1 > 1.0e-6 && d1 < kMaxDistance, k2 = d2 > 1.0e-6 && d2 < kMaxDistance;
+    out[0] = k1 ? d1 : d2; // static places: the hits stay in registers
+    out[1] = d2;
+    return (int)k1 + (int)k2;
 }
 
 __device__ inline bool sphere_inside(D3 c, double r, D3 p, bool inv) { // sphere.cpp:271-303
@@ -133,46 +146,41 @@ __device__ inline bool plane_hit(const PlaneRec &pl, D3 o, D3 d, double &depth) 
 // CLOSE_TOLERANCE side tie-breaking; returns pushed depths (Depth1 only when
 // > DEPTH_TOLERANCE, Depth2 always) and their sides.
 // ---------------------------------------------------------------------------
-__device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, double *out, int *side) {
+__device__ inline int box_hits_at(const double *c1, const double *c2, D3 P, D3 D, double *out, int *side) {
     const double kClose = 1.0e-6;
-    D3 P = o, D = d;
-    if (b.xf >= 0) {
-        P = xf_point(xf[b.xf].inv, o);
-        D = xf_dir(xf[b.xf].inv, d);
-    }
     int smin = 0, smax = 0;
     double t, tmin = 0.0, tmax = kBoundHuge;
     // X: no ties
     if (D.x < -kEpsilon) {
-        t = (b.c1[0] - P.x) / D.x;
+        t = (c1[0] - P.x) / D.x;
         if (t < tmin) return 0;
         if (t <= tmax) { smax = 1; tmax = t; }
-        t = (b.c2[0] - P.x) / D.x;
+        t = (c2[0] - P.x) / D.x;
         if (t >= tmin) {
             if (t > tmax) return 0;
             smin = 2;
             tmin = t;
         }
     } else if (D.x > kEpsilon) {
-        t = (b.c2[0] - P.x) / D.x;
+        t = (c2[0] - P.x) / D.x;
         if (t < tmin) return 0;
         if (t <= tmax) { smax = 2; tmax = t; }
-        t = (b.c1[0] - P.x) / D.x;
+        t = (c1[0] - P.x) / D.x;
         if (t >= tmin) {
             if (t > tmax) return 0;
             smin = 1;
             tmin = t;
         }
-    } else if (P.x < b.c1[0] || P.x > b.c2[0]) {
+    } else if (P.x < c1[0] || P.x > c2[0]) {
         return 0;
     }
     // Y: ties against |D.x|
     if (D.y < -kEpsilon) {
-        t = (b.c1[1] - P.y) / D.y;
+        t = (c1[1] - P.y) / D.y;
         if (t < tmin) return 0;
         if (t <= tmax - kClose) { smax = 3; tmax = t; }
         else if (t <= tmax + kClose) { if (-D.y > fabs(D.x)) smax = 3; }
-        t = (b.c2[1] - P.y) / D.y;
+        t = (c2[1] - P.y) / D.y;
         if (t >= tmin + kClose) {
             if (t > tmax) return 0;
             smin = 4;
@@ -181,11 +189,11 @@ __device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, dou
             if (-D.y > fabs(D.x)) smin = 4;
         }
     } else if (D.y > kEpsilon) {
-        t = (b.c2[1] - P.y) / D.y;
+        t = (c2[1] - P.y) / D.y;
         if (t < tmin) return 0;
         if (t <= tmax - kClose) { smax = 4; tmax = t; }
         else if (t <= tmax + kClose) { if (D.y > fabs(D.x)) smax = 4; }
-        t = (b.c1[1] - P.y) / D.y;
+        t = (c1[1] - P.y) / D.y;
         if (t >= tmin + kClose) {
             if (t > tmax) return 0;
             smin = 3;
@@ -193,19 +201,19 @@ __device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, dou
         } else if (t >= tmin - kClose) {
             if (D.y > fabs(D.x)) smin = 3;
         }
-    } else if (P.y < b.c1[1] || P.y > b.c2[1]) {
+    } else if (P.y < c1[1] || P.y > c2[1]) {
         return 0;
     }
     // Z: ties against the axis of the side chosen so far
     if (D.z < -kEpsilon) {
         double dz = -D.z;
-        t = (b.c1[2] - P.z) / D.z;
+        t = (c1[2] - P.z) / D.z;
         if (t < tmin) return 0;
         if (t <= tmax - kClose) { smax = 5; tmax = t; }
         else if (t <= tmax + kClose) {
             if ((smax == 1 || smax == 2) ? dz > fabs(D.x) : ((smax == 3 || smax == 4) && dz > fabs(D.y))) smax = 5;
         }
-        t = (b.c2[2] - P.z) / D.z;
+        t = (c2[2] - P.z) / D.z;
         if (t >= tmin + kClose) {
             if (t > tmax) return 0;
             smin = 6;
@@ -215,13 +223,13 @@ __device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, dou
         }
     } else if (D.z > kEpsilon) {
         double dz = D.z;
-        t = (b.c2[2] - P.z) / D.z;
+        t = (c2[2] - P.z) / D.z;
         if (t < tmin) return 0;
         if (t <= tmax - kClose) { smax = 6; tmax = t; }
         else if (t <= tmax + kClose) {
             if ((smax == 1 || smax == 2) ? dz > fabs(D.x) : ((smax == 3 || smax == 4) && dz > fabs(D.y))) smax = 6;
         }
-        t = (b.c1[2] - P.z) / D.z;
+        t = (c1[2] - P.z) / D.z;
         if (t >= tmin + kClose) {
             if (t > tmax) return 0;
             smin = 5;
@@ -229,382 +237,37 @@ __device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, dou
         } else if (t >= tmin - kClose) {
             if ((smin == 1 || smin == 2) ? dz > fabs(D.x) : ((smin == 3 || smin == 4) && dz > fabs(D.y))) smin = 5;
         }
-    } else if (P.z < b.c1[2] || P.z > b.c2[2]) {
+    } else if (P.z < c1[2] || P.z > c2[2]) {
         return 0;
     }
     if (tmax < 1.0e-6) return 0;
-    int n = 0;
-    if (tmin > 1.0e-6) {
-        out[n] = tmin;
-        side[n++] = smin;
-    }
-    out[n] = tmax;
-    side[n++] = smax;
-    return n;
+    const bool both = tmin > 1.0e-6;
+    out[0] = both ? tmin : tmax;
+    side[0] = both ? smin : smax;
+    out[1] = tmax;
+    side[1] = smax;
+    return both ? 2 : 1;
 }
 
-__device__ inline bool box_inside(const BoxRec &b, const Xform *xf, D3 p, bool inv) { // box.cpp:535-570
-    D3 q = b.xf >= 0 ? xf_point(xf[b.xf].inv, p) : p;
-    if (q.x < b.c1[0] || q.x > b.c2[0]) return inv;
-    if (q.y < b.c1[1] || q.y > b.c2[1]) return inv;
-    if (q.z < b.c1[2] || q.z > b.c2[2]) return inv;
+__device__ inline int box_hits(const BoxRec &b, const Xform *xf, D3 o, D3 d, double *out, int *side) {
+    D3 P = o, D = d;
+    if (b.xf >= 0) {
+        P = xf_point(xf[b.xf].inv, o);
+        D = xf_dir(xf[b.xf].inv, d);
+    }
+    return box_hits_at(b.c1, b.c2, P, D, out, side);
+}
+
+__device__ inline bool box_inside_at(const double *c1, const double *c2, D3 q, bool inv) { // box.cpp:535-570
+    if (q.x < c1[0] || q.x > c2[0]) return inv;
+    if (q.y < c1[1] || q.y > c2[1]) return inv;
+    if (q.z < c1[2] || q.z > c2[2]) return inv;
     return !inv;
 }
 
-// ---------------------------------------------------------------------------
-// Polynomial roots: core/math/polynomialsolver.cpp (default build branches).
-// sbisect's recursion becomes an explicit interval stack visited
-// left-to-right, which yields the same roots in the same order.
-// ---------------------------------------------------------------------------
-namespace poly {
-constexpr int kMaxIter = 50;
-constexpr double kSmall = 1.0e-10;
-constexpr double kRel = 1.0e-12;
-
-// A polynomial of order <= N, ascending powers (the reference's `polynomial`
-// holds up to MAX_ORDER 35; the shapes here need 4 (torus) and 6 (lathe)).
-template <int N>
-struct PN {
-    int ord;
-    double c[N + 1];
-};
-using P4 = PN<4>;
-
-__device__ inline double eval(double x, int n, const double *c) {
-    double v = c[n];
-    for (int i = n - 1; i >= 0; i--) v = v * x + c[i];
-    return v;
+__device__ inline bool box_inside(const BoxRec &b, const Xform *xf, D3 p, bool inv) {
+    return box_inside_at(b.c1, b.c2, b.xf >= 0 ? xf_point(xf[b.xf].inv, p) : p, inv);
 }
-
-template <int N>
-__device__ inline int modp(const PN<N> &u, const PN<N> &v, PN<N> &r) {
-    r = u;
-    if (v.c[v.ord] < 0.0) {
-        for (int k = u.ord - v.ord - 1; k >= 0; k -= 2) r.c[k] = -r.c[k];
-        for (int k = u.ord - v.ord; k >= 0; k--)
-            for (int j = v.ord + k - 1; j >= k; j--) r.c[j] = -r.c[j] - r.c[v.ord + k] * v.c[j - k];
-    } else {
-        for (int k = u.ord - v.ord; k >= 0; k--)
-            for (int j = v.ord + k - 1; j >= k; j--) r.c[j] -= r.c[v.ord + k] * v.c[j - k];
-    }
-    int k = v.ord - 1;
-    while (k >= 0 && fabs(r.c[k]) < kSmall) {
-        r.c[k] = 0.0;
-        k--;
-    }
-    r.ord = (k < 0) ? 0 : k;
-    return r.ord;
-}
-
-template <int N>
-__device__ inline int buildsturm(int ord, PN<N> *s) {
-    s[0].ord = ord;
-    s[1].ord = ord - 1;
-    double f = fabs(s[0].c[ord] * ord);
-    for (int i = 1; i <= ord; i++) s[1].c[i - 1] = s[0].c[i] * i / f;
-    int k = 2;
-    while (modp(s[k - 2], s[k - 1], s[k])) {
-        f = -fabs(s[k].c[s[k].ord]);
-        for (int j = s[k].ord; j >= 0; j--) s[k].c[j] /= f;
-        k++;
-    }
-    s[k].c[0] = -s[k].c[0];
-    return k;
-}
-
-template <int N>
-__device__ inline int numchanges(int np, const PN<N> *s, double a) {
-    int ch = 0;
-    double lf = eval(a, s[0].ord, s[0].c);
-    for (int k = 1; k <= np; k++) {
-        double f = eval(a, s[k].ord, s[k].c);
-        if (lf == 0.0 || lf * f < 0) ch++;
-        lf = f;
-    }
-    return ch;
-}
-
-template <int N>
-__device__ inline int visible_roots(int np, const PN<N> *s) {
-    int atpos = 0, atzero = 0;
-    double lf = s[0].c[s[0].ord];
-    for (int k = 1; k <= np; k++) {
-        double f = s[k].c[s[k].ord];
-        if (lf == 0.0 || lf * f < 0) atpos++;
-        lf = f;
-    }
-    lf = s[0].c[0];
-    for (int k = 1; k <= np; k++) {
-        double f = s[k].c[0];
-        if (lf == 0.0 || lf * f < 0) atzero++;
-        lf = f;
-    }
-    return atzero - atpos;
-}
-
-__device__ inline int regula_falsa(int order, const double *coef, double a, double b, double *val) {
-    double fa = eval(a, order, coef), fb = eval(b, order, coef), x, fx, lfx;
-    if (fa * fb > 0.0) return 0;
-    if (fabs(fa) < kSmall) { *val = a; return 1; }
-    if (fabs(fb) < kSmall) { *val = b; return 1; }
-    lfx = fa;
-    for (int its = 0; its < kMaxIter; its++) {
-        x = (fb * a - fa * b) / (fb - fa);
-        fx = eval(x, order, coef);
-        if (fabs(x) > kRel) {
-            if (fabs(fx / x) < kRel) { *val = x; return 1; }
-        } else if (fabs(fx) < kRel) {
-            *val = x;
-            return 1;
-        }
-        if (fa < 0) {
-            if (fx < 0) { a = x; fa = fx; if ((lfx * fx) > 0) fb /= 2; }
-            else { b = x; fb = fx; if ((lfx * fx) > 0) fa /= 2; }
-        } else {
-            if (fx < 0) { b = x; fb = fx; if ((lfx * fx) > 0) fa /= 2; }
-            else { a = x; fa = fx; if ((lfx * fx) > 0) fb /= 2; }
-        }
-        if (fabs(b - a) < kRel) { *val = x; return 1; }
-        lfx = fx;
-    }
-    return 0;
-}
-
-// sbisect over an explicit stack.
-template <int N>
-__device__ inline int sbisect(int np, const PN<N> *s, double lo, double hi, int atlo, int athi,
-                              double *roots) {
-    struct Iv {
-        double lo, hi;
-        int atlo, athi;
-    } st[N + 2]; // each pending interval holds at least one of the <= N roots
-    int sp = 0, nr = 0;
-    st[sp++] = Iv{lo, hi, atlo, athi};
-    while (sp > 0) {
-        Iv iv = st[--sp];
-        double mn = iv.lo, mx = iv.hi, mid = 0.0;
-        int amin = iv.atlo, amax = iv.athi;
-        if (amin - amax == 1) {
-            if (regula_falsa(s[0].ord, s[0].c, mn, mx, &roots[nr])) {
-                nr++;
-                continue;
-            }
-            bool done = false;
-            for (int its = 0; its < kMaxIter; its++) {
-                mid = (mn + mx) / 2;
-                int am = numchanges(np, s, mid);
-                if (am < amax || am > amin) { done = true; break; } // no root
-                if (fabs(mid) > kRel) {
-                    if (fabs((mx - mn) / mid) < kRel) { roots[nr++] = mid; done = true; break; }
-                } else if (fabs(mx - mn) < kRel) {
-                    roots[nr++] = mid;
-                    done = true;
-                    break;
-                }
-                if (amin - am == 0) mn = mid; else mx = mid;
-            }
-            if (!done) roots[nr++] = mid;
-            continue;
-        }
-        bool handled = false;
-        for (int its = 0; its < kMaxIter; its++) {
-            mid = (mn + mx) / 2;
-            int am = numchanges(np, s, mid);
-            if (am < amax || am > amin) { handled = true; break; }
-            if (fabs(mid) > kRel) {
-                if (fabs((mx - mn) / mid) < kRel) { roots[nr++] = mid; handled = true; break; }
-            } else if (fabs(mx - mn) < kRel) {
-                roots[nr++] = mid;
-                handled = true;
-                break;
-            }
-            int n1 = amin - am, n2 = am - amax;
-            if (n1 != 0 && n2 != 0) {
-                if (sp + 2 <= N + 2) {
-                    st[sp++] = Iv{mid, mx, am, amax}; // right, visited second
-                    st[sp++] = Iv{mn, mid, amin, am}; // left, visited first
-                }
-                handled = true;
-                break;
-            }
-            if (n1 == 0) mn = mid; else mx = mid;
-        }
-        if (!handled) roots[nr++] = mid;
-    }
-    return nr;
-}
-
-// (an order-N polynomial has at most N roots pending on the interval stack)
-template <int N = 4>
-__device__ inline int polysolve(int order, const double *coeffs, double *roots) {
-    PN<N> s[N + 2];
-    for (int i = 0; i <= order; i++) s[0].c[order - i] = coeffs[i] / coeffs[0];
-    int np = buildsturm(order, s);
-    if (visible_roots(np, s) == 0) return 0;
-    int atmin = numchanges(np, s, 0.0);
-    int atmax = numchanges(np, s, kMaxDistance);
-    if (atmin - atmax == 0) return 0;
-    return sbisect(np, s, 0.0, kMaxDistance, atmin, atmax, roots);
-}
-
-__device__ inline int solve_quadratic(const double *x, double *y) {
-    double a = x[0], b = -x[1], c = x[2];
-    if (a == 0.0) {
-        if (b == 0.0) return 0;
-        y[0] = c / b;
-        return 1;
-    }
-    b /= a;
-    c /= a;
-    a = 1.0;
-    double d = b * b - 4.0 * a * c;
-    if (d > -kSmall && d < kSmall) {
-        y[0] = 0.5 * b / a;
-        return 1;
-    }
-    if (d < 0.0) return 0;
-    d = sqrt(d);
-    double t = 2.0 * a;
-    y[0] = (b + d) / t;
-    y[1] = (b - d) / t;
-    return 2;
-}
-
-__device__ inline int solve_cubic(const double *x, double *y) {
-    double a0 = x[0], a1, a2, a3;
-    if (a0 == 0.0) return solve_quadratic(&x[1], y);
-    if (a0 != 1.0) {
-        a1 = x[1] / a0; a2 = x[2] / a0; a3 = x[3] / a0;
-    } else {
-        a1 = x[1]; a2 = x[2]; a3 = x[3];
-    }
-    double A2 = a1 * a1;
-    double Q = (A2 - 3.0 * a2) / 9.0;
-    double R = (a1 * (A2 - 4.5 * a2) + 13.5 * a3) / 27.0;
-    double Q3 = Q * Q * Q, R2 = R * R, dd = Q3 - R2, an = a1 / 3.0;
-    if (dd >= 0.0) {
-        dd = R / sqrt(Q3);
-        double theta = acos(dd) / 3.0;
-        double sQ = -2.0 * sqrt(Q);
-        y[0] = sQ * cos(theta) - an;
-        y[1] = sQ * cos(theta + 2.0943951023931954923084) - an;
-        y[2] = sQ * cos(theta + 4.1887902047863909846168) - an;
-        return 3;
-    }
-    double sQ = pow(sqrt(R2 - Q3) + fabs(R), 1.0 / 3.0);
-    y[0] = (R < 0) ? (sQ + Q / sQ) - an : -(sQ + Q / sQ) - an;
-    return 1;
-}
-
-__device__ inline int difficult_coeffs(const double *x) { // signed `biggest`, default branch
-    double biggest = 0.0;
-    for (int i = 0; i <= 4; i++)
-        if (fabs(x[i]) > biggest) biggest = x[i];
-    if (biggest == 0.0) return 0;
-    for (int i = 0; i <= 4; i++)
-        if (x[i] != 0.0 && fabs(biggest / x[i]) > 1.0e12) return 1;
-    return 0;
-}
-
-__device__ inline int solve_quartic(const double *x, double *res) {
-    double c1, c2, c3, c4, c0 = x[0];
-    if (c0 != 1.0) {
-        c1 = x[1] / c0; c2 = x[2] / c0; c3 = x[3] / c0; c4 = x[4] / c0;
-    } else {
-        c1 = x[1]; c2 = x[2]; c3 = x[3]; c4 = x[4];
-    }
-    double c12 = c1 * c1;
-    double p = -0.375 * c12 + c2;
-    double q = 0.125 * c12 * c1 - 0.5 * c1 * c2 + c3;
-    double r = -0.01171875 * c12 * c12 + 0.0625 * c12 * c2 - 0.25 * c1 * c3 + c4;
-    double cubic[4] = {1.0, -0.5 * p, -r, 0.5 * r * p - 0.125 * q * q};
-    double roots[3];
-    if (solve_cubic(cubic, roots) <= 0) return 0;
-    double z = roots[0];
-    double d1 = 2.0 * z - p, d2;
-    if (d1 < 0.0) {
-        if (d1 > -kSmall) d1 = 0.0;
-        else return 0;
-    }
-    if (d1 < kSmall) {
-        d2 = z * z - r;
-        if (d2 < 0.0) return 0;
-        d2 = sqrt(d2);
-    } else {
-        d1 = sqrt(d1);
-        d2 = 0.5 * q / d1;
-    }
-    double q1 = d1 * d1, q2 = -0.25 * c1;
-    int i = 0;
-    p = q1 - 4.0 * (z - d2);
-    if (p == 0) {
-        res[i++] = -0.5 * d1 - q2;
-    } else if (p > 0) {
-        p = sqrt(p);
-        res[i++] = -0.5 * (d1 + p) + q2;
-        res[i++] = -0.5 * (d1 - p) + q2;
-    }
-    p = q1 - 4.0 * (z + d2);
-    if (p == 0) {
-        res[i++] = 0.5 * d1 - q2;
-    } else if (p > 0) {
-        p = sqrt(p);
-        res[i++] = 0.5 * (d1 + p) + q2;
-        res[i++] = 0.5 * (d1 - p) + q2;
-    }
-    return i;
-}
-
-// Solve_Polynomial for order 4 (polynomialsolver.cpp:1585-1732), c descending.
-__device__ inline int solve4(const double *c0, double *r, bool sturm, double eps) {
-    int i = 0, n = 4;
-    while (i < n && fabs(c0[i]) < kSmall) i++;
-    n -= i;
-    const double *c = &c0[i];
-    switch (n) {
-    case 0:
-        return 0;
-    case 1:
-        if (c[0] != 0.0) { r[0] = -c[1] / c[0]; return 1; }
-        return 0;
-    case 2:
-        return solve_quadratic(c, r);
-    case 3:
-        if (eps > 0.0 && c[2] != 0.0 && fabs(c[3] / c[2]) < eps) return solve_quadratic(c, r);
-        return sturm ? polysolve(3, c, r) : solve_cubic(c, r);
-    default:
-        if (eps > 0.0 && c[3] != 0.0 && fabs(c[4] / c[3]) < eps)
-            return sturm ? polysolve(3, c, r) : solve_cubic(c, r);
-        if (difficult_coeffs(c)) sturm = true;
-        return sturm ? polysolve(4, c, r) : solve_quartic(c, r);
-    }
-}
-
-// Solve_Polynomial with epsilon 0 for orders up to 6 (the lathe's and sor's
-// calls, lathe.cpp:255-285 and sor.cpp:395), c descending.
-__device__ inline int solve6(int n, const double *c0, double *r, bool sturm) {
-    int i = 0;
-    while (i < n && fabs(c0[i]) < kSmall) i++;
-    n -= i;
-    const double *c = &c0[i];
-    switch (n) {
-    case 0:
-        return 0;
-    case 1:
-        if (c[0] != 0.0) { r[0] = -c[1] / c[0]; return 1; }
-        return 0;
-    case 2:
-        return solve_quadratic(c, r);
-    case 3:
-        return sturm ? polysolve<3>(3, c, r) : solve_cubic(c, r);
-    case 4:
-        if (difficult_coeffs(c)) sturm = true;
-        return sturm ? polysolve<4>(4, c, r) : solve_quartic(c, r);
-    default:
-        return polysolve<6>(n, c, r);
-    }
-}
-} // namespace poly
 
 // Torus::Test_Thick_Cylinder (core/shape/torus.cpp:932-1085)
 __device__ inline bool thick_cylinder(D3 P, D3 D, double h1, double h2, double r1, double r2) {
@@ -653,13 +316,9 @@ __device__ inline bool thick_cylinder(D3 P, D3 D, double h1, double h2, double r
 }
 
 // Torus::Intersect + All_Intersections (torus.cpp:133-160, 241-329).
-__device__ inline int torus_hits(const TorusRec &tr, const Xform *xf, D3 o, D3 d, double *out) {
-    const Xform &x = xf[tr.xf];
-    D3 P = xf_point(x.inv, o);
-    D3 D = xf_dir(x.inv, d);
+__device__ inline int torus_hits_at(double R, double rr, bool sturm, D3 P, D3 D, double (&out)[4]) {
     double len = sqrt(dot3(D, D));
     D = D3{D.x / len, D.y / len, D.z / len};
-    double R = tr.R, rr = tr.r;
     double r1 = (R - rr) * (R - rr);
     if (R < rr) r1 = 0;
     double r2 = (R + rr) * (R + rr);
@@ -682,20 +341,30 @@ __device__ inline int torus_hits(const TorusRec &tr, const Xform *xf, D3 o, D3 d
     c[3] = 4.0 * (k2 * k1 + 2.0 * R2 * PDy2);
     c[4] = k1 * k1 + 4.0 * R2 * (Py2 - rr2);
     double roots[4];
-    int nr = poly::solve4(c, roots, tr.sturm != 0, 1.0e-4);
+    int nr = poly::solve4(c, roots, sturm, 1.0e-4);
     int n = 0;
-    while (nr--) {
-        double dep = (roots[nr] + closer) / len;
-        if (dep > 1.0e-4 && dep < kMaxDistance) out[n++] = dep;
-    }
+#pragma unroll
+    for (int j = 3; j >= 0; j--)
+        if (j < nr) {
+            const double dep = (roots[j] + closer) / len;
+            if (dep > 1.0e-4 && dep < kMaxDistance) poly::put_root(out, n, dep);
+        }
     return n;
 }
 
-__device__ inline bool torus_inside(const TorusRec &tr, const Xform *xf, D3 p, bool inv) { // torus.cpp:364-385
-    D3 P = xf_point(xf[tr.xf].inv, p);
+__device__ inline int torus_hits(const TorusRec &tr, const Xform *xf, D3 o, D3 d, double (&out)[4]) {
+    const Xform &x = xf[tr.xf];
+    return torus_hits_at(tr.R, tr.r, tr.sturm != 0, xf_point(x.inv, o), xf_dir(x.inv, d), out);
+}
+
+__device__ inline bool torus_inside_at(double R, double rr, D3 P, bool inv) { // torus.cpp:364-385
     double r = sqrt(P.x * P.x + P.z * P.z);
-    double r2 = P.y * P.y + (r - tr.R) * (r - tr.R);
-    return (r2 <= tr.r * tr.r) ? !inv : inv;
+    double r2 = P.y * P.y + (r - R) * (r - R);
+    return (r2 <= rr * rr) ? !inv : inv;
+}
+
+__device__ inline bool torus_inside(const TorusRec &tr, const Xform *xf, D3 p, bool inv) {
+    return torus_inside_at(tr.R, tr.r, xf_point(xf[tr.xf].inv, p), inv);
 }
 
 // ---------------------------------------------------------------------------
@@ -1149,15 +818,12 @@ __device__ inline bool rev_inside(const SceneView &sv, uint32_t index, D3 ip, bo
 // ---------------------------------------------------------------------------
 // CSG (core/shape/csg.cpp): point membership with bounded nesting.
 // ---------------------------------------------------------------------------
+// Inside test of one operand that is not itself a CSG node.
 // kRev: lathes and sors may be operands (the walks of scenes without them
 // leave their code out, which keeps those kernels' register budget).
-template <int D, bool kRev = false>
-__device__ bool csg_inside(const SceneView &sv, uint32_t node, D3 p);
-
-template <int D, bool kRev = false>
-__device__ inline bool shape_inside(const SceneView &sv, uint32_t type, uint32_t index,
-                                    uint32_t flags, D3 p) {
-    bool inv = (flags & PVX_FLAG_INVERTED) != 0;
+template <bool kRev = false>
+__device__ inline bool leaf_inside(const SceneView &sv, uint32_t type, uint32_t index, uint32_t flags, D3 p) {
+    const bool inv = (flags & PVX_FLAG_INVERTED) != 0;
     switch (type) {
     case 1: { // sphere
         const double *s = sv.sph + 4 * (size_t)index;
@@ -1179,8 +845,6 @@ __device__ inline bool shape_inside(const SceneView &sv, uint32_t type, uint32_t
         bool in = (t + pl.d) < kEpsilon;
         return inv ? !in : in;
     }
-    case 6:
-        return csg_inside<D, kRev>(sv, index, p);
     case PVX_LATHE:
     case PVX_SOR:
         if constexpr (kRev) return rev_inside(sv, index, p, inv);
@@ -1190,40 +854,61 @@ __device__ inline bool shape_inside(const SceneView &sv, uint32_t type, uint32_t
     }
 }
 
-template <int D, bool kRev>
-__device__ bool csg_inside(const SceneView &sv, uint32_t node, D3 p) {
-    if constexpr (D <= 0) {
-        return false;
-    } else {
-        const CsgNode &n = sv.csg[node];
-        for (uint32_t k = 0; k < n.count; k++) {
-            const CsgChild &c = sv.csg_children[n.first + k];
-            bool in = shape_inside<D - 1, kRev>(sv, c.type, c.index, c.flags, p);
-            if (n.op == 2) { // intersection: CSGIntersection::Inside (csg.cpp:440-454)
-                if (!in) return false;
-            } else if (in) { // union / merge: CSGUnion::Inside (csg.cpp:405-424)
-                return true;
+// Is p inside the operand in csg_children slot `slot` (CSGIntersection::Inside
+// and CSGUnion::Inside, csg.cpp:405-454)?  The operand's subtree is walked
+// through the nodes' parent links with one operand test in the loop body: a
+// recursion over the nesting levels gave every level its own inlined copy of
+// all shape tests (240 registers, and lanes at different levels ran them one
+// after the other).
+template <bool kRev = false>
+__device__ inline bool csg_slot_inside(const SceneView &sv, uint32_t slot, D3 p) {
+    uint32_t cur = slot;
+    for (;;) {
+        const CsgChild c = sv.csg_children[cur];
+        bool in;
+        if (c.type == PVX_CSG) {
+            const CsgNode &n = sv.csg[c.index];
+            if (n.count > 0) {
+                cur = n.first;
+                continue;
             }
+            in = n.op == 2; // no operands: an intersection holds everything
+        } else {
+            in = leaf_inside<kRev>(sv, c.type, c.index, c.flags, p);
         }
-        return n.op == 2;
+        // the result of `cur`: on to its next sibling, or up
+        for (;;) {
+            if (cur == slot) return in;
+            const uint32_t node = sv.csg_children[cur].node;
+            const CsgNode &n = sv.csg[node];
+            const bool last = cur + 1 == n.first + n.count;
+            // an intersection ends at the first operand outside, a union or
+            // merge at the first inside
+            if ((n.op == 2) == in && !last) {
+                cur++;
+                break;
+            }
+            cur = (uint32_t)n.parent_slot; // its result is `in`
+        }
     }
 }
 
-// Hits of one leaf shape (sphere/box/torus/cone/disc/quadric/triangle) in
+// Inside test of a whole object (CSG node `index` or a single shape).
+template <bool kRev = false>
+__device__ inline bool shape_inside(const SceneView &sv, uint32_t type, uint32_t index, uint32_t flags, D3 p) {
+    if (type != PVX_CSG) return leaf_inside<kRev>(sv, type, index, flags, p);
+    const CsgNode &n = sv.csg[index];
+    for (uint32_t k = 0; k < n.count; k++)
+        if (csg_slot_inside<kRev>(sv, n.first + k, p) != (n.op == 2)) return n.op != 2;
+    return n.op == 2;
+}
+
+// Hits of one leaf shape other than a sphere, box or torus in
 // push order (an inverted quadric pushes its two roots the other way round;
 // the set is the same).
-__device__ inline int leaf_hits(const SceneView &sv, uint32_t type, uint32_t index, D3 o, D3 d,
-                                double *out) {
-    int side[2];
+__device__ inline int other_hits(const SceneView &sv, uint32_t type, uint32_t index, D3 o, D3 d,
+                                double (&out)[kMaxLeafHits]) {
     switch (type) {
-    case 1: {
-        const double *s = sv.sph + 4 * (size_t)index;
-        return sphere_hits(d3(s[0], s[1], s[2]), s[3], o, d, out);
-    }
-    case 2:
-        return box_hits(sv.boxes[index], sv.xforms, o, d, out, side);
-    case 3:
-        return torus_hits(sv.tori[index], sv.xforms, o, d, out);
     case 9: {
         int part[4];
         return cone_hits(sv.cones[index], sv.xforms, o, d, out, part);
@@ -1246,6 +931,47 @@ __device__ inline int leaf_hits(const SceneView &sv, uint32_t type, uint32_t ind
     }
 }
 
+__device__ inline int leaf_hits(const SceneView &sv, uint32_t type, uint32_t index, D3 o, D3 d,
+                                double (&out)[kMaxLeafHits]) {
+    switch (type) {
+    case 1: {
+        const double *s = sv.sph + 4 * (size_t)index;
+        return sphere_hits(d3(s[0], s[1], s[2]), s[3], o, d, out);
+    }
+    case 2: {
+        int side[2];
+        return box_hits(sv.boxes[index], sv.xforms, o, d, out, side);
+    }
+    case 3:
+        return torus_hits(sv.tori[index], sv.xforms, o, d, out);
+    default:
+        return other_hits(sv, type, index, o, d, out);
+    }
+}
+
+// Ascending order of the first nh depths.
+__device__ inline void sort_hits(double (&hs)[kMaxLeafHits], int nh) {
+#pragma unroll
+    for (int j = 0; j < kMaxLeafHits; j++)
+        if (j >= nh) hs[j] = HUGE_VAL;
+    auto cx = [&](int a, int b) {
+        const double lo = hs[a] < hs[b] ? hs[a] : hs[b], hi = hs[a] < hs[b] ? hs[b] : hs[a];
+        hs[a] = lo;
+        hs[b] = hi;
+    };
+    cx(0, 1);
+    cx(2, 3);
+    cx(0, 2);
+    cx(1, 3);
+    cx(1, 2);
+}
+
+// hs[j] without an indexed load (the hits stay in registers).
+__device__ inline double pick_hit(const double (&hs)[kMaxLeafHits], int j) {
+    const double a = j & 1 ? hs[1] : hs[0], b = j & 1 ? hs[3] : hs[2];
+    return j & 2 ? b : a;
+}
+
 // Every hit of one leaf shape in push order, as emit(depth, side, d1); `child`:
 // the shape is a CSG operand (IS_CHILD_OBJECT).
 template <bool kRev, class Emit>
@@ -1259,32 +985,40 @@ __device__ inline void leaf_visit(const SceneView &sv, uint32_t type, uint32_t i
     }
     double hs[kMaxLeafHits];
     const int nh = leaf_hits(sv, type, index, o, d, hs);
-    for (int j = 0; j < nh; j++) emit(hs[j], 0, 0.0);
+#pragma unroll 1
+    for (int j = 0; j < nh; j++) emit(pick_hit(hs, j), 0, 0.0);
 }
 
-// Does a hit at depth `dep` on the leaf in csg_children slot `slot` survive
-// every CSG filter between the leaf and the root (CSGIntersection keeps
-// hits inside all siblings, CSGMerge hits inside none, CSGUnion all;
-// csg.cpp:128-375)?
+// Does a hit at ip on the leaf in csg_children slot `slot` survive every CSG
+// filter between the leaf and the root (CSGIntersection keeps hits inside all
+// siblings, CSGMerge hits inside none, CSGUnion all; csg.cpp:128-375)?  Runs
+// the filter programs of the enclosing nodes (CsgSlot, CsgTest).
 template <bool kRev = false>
 __device__ inline bool csg_survives(const SceneView &sv, uint32_t slot, D3 ip) {
-    uint32_t child = slot;
-    for (int level = 0; level < kCsgMaxDepth; level++) {
-        const CsgChild &cc = sv.csg_children[child];
-        const CsgNode &n = sv.csg[cc.node];
-        if (n.op != 1) {
-            bool is_merge = (n.op == 3);
-            for (uint32_t k = 0; k < n.count; k++) {
-                uint32_t sib = n.first + k;
-                if (sib == child) continue;
-                const CsgChild &s = sv.csg_children[sib];
-                bool in = shape_inside<kCsgMaxDepth, kRev>(sv, s.type, s.index, s.flags, ip);
-                if (is_merge ? in : !in) return false;
+    int32_t cur = (int32_t)slot;
+    do {
+        const CsgSlot &c = sv.csg_slots[cur];
+        const uint32_t skip = c.skip, skip_to = c.skip_to;
+        uint32_t pc = c.start;
+        cur = c.up;
+        for (;;) {
+            if (pc == skip) pc = skip_to;
+            if (pc == kCsgUp) break;
+            if (pc == kCsgDrop) return false;
+            const CsgTest t = sv.csg_tests[pc];
+            const uint32_t type = t.what & 0xFFu;
+            const bool inv = (t.what >> 8) & 1u;
+            bool in;
+            if (type == PVX_BOX || type == PVX_TORUS) {
+                const PlacedRec &r = sv.placed[t.index];
+                const D3 q = ((t.what >> 16) & kPlacedXf) ? pl_point(r.inv, ip) : ip;
+                in = type == PVX_BOX ? box_inside_at(r.q, r.q + 3, q, inv) : torus_inside_at(r.q[0], r.q[1], q, inv);
+            } else {
+                in = leaf_inside<kRev>(sv, type, t.index, inv ? (uint32_t)PVX_FLAG_INVERTED : 0u, ip);
             }
+            pc = in ? t.next_in : t.next_out;
         }
-        if (n.parent_slot < 0) return true;
-        child = (uint32_t)n.parent_slot;
-    }
+    } while (cur >= 0);
     return true;
 }
 

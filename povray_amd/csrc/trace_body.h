@@ -27,6 +27,18 @@ __device__ inline float safe_inv(double d) {
     return 1.0f / f;
 }
 
+// Slab test of one referenced primitive's own box, as the nodes test theirs:
+// a leaf's primitives share a node box, and the FP64 tests behind this one
+// cost tens (a box) to thousands (a torus) of instructions.
+__device__ __forceinline__ bool ref_box_hit(const RefRec &r, const RayF &rf, float tb) {
+    const float x0 = fmaf(r.lo[0], rf.ix, -rf.oix), x1 = fmaf(r.hi[0], rf.ix, -rf.oix);
+    const float y0 = fmaf(r.lo[1], rf.iy, -rf.oiy), y1 = fmaf(r.hi[1], rf.iy, -rf.oiy);
+    const float z0 = fmaf(r.lo[2], rf.iz, -rf.oiz), z1 = fmaf(r.hi[2], rf.iz, -rf.oiz);
+    const float tn = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
+    const float tf = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tb));
+    return tn <= tf * 1.000001f;
+}
+
 // Mesh::Intersect for one mesh2 triangle: for a placed mesh the ray moves
 // into the mesh's own space with its direction normalised (mesh.cpp:179-230)
 // and the depth returns to world units divided by that length (test_hit,
@@ -106,8 +118,9 @@ __device__ inline bool csg_closest(const SceneView &sv, uint32_t root, D3 o, D3 
             leaf_visit<true>(sv, c.type, c.index, o, d, true, [&](double dep, int, double) { consider(dep); });
         } else {
             double hs[kMaxLeafHits];
-            int nh = leaf_hits(sv, c.type, c.index, o, d, hs);
-            for (int j = 0; j < nh; j++) consider(hs[j]);
+            const int nh = leaf_hits(sv, c.type, c.index, o, d, hs);
+#pragma unroll 1
+            for (int j = 0; j < nh; j++) consider(pick_hit(hs, j));
         }
     }
     dep_out = best;
@@ -174,8 +187,8 @@ __device__ inline bool simple_closest(const SceneView &sv, uint32_t kind, uint32
     return found;
 }
 
-// kLevel 0: triangles and spheres; 1: also boxes; 2: also tori and CSG; 3: also
-// lathes and sors.
+// kLevel 0: triangles and spheres; 1: also boxes and stand-alone triangles
+// (the levels above: trace_ref_body).
 // kWW: while-while traversal (triangle scenes, camera and bounce rays).
 // kMulti: rays of many scenes in one launch.  `n` is then 64 x the number of
 // chunks; chunk c = {scene, first ray, ray count <= 64} covers the wavefront
@@ -202,7 +215,8 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                                                    uint32_t *__restrict__ prim_tests, int32_t *s_stack,
                                                    const LightGroup *__restrict__ gen_groups = nullptr,
                                                    const LightRec *__restrict__ gen_lights = nullptr,
-                                                   uint32_t gen_S = 1, uint8_t *__restrict__ gen_vis = nullptr) {
+                                                   uint32_t gen_S = 1, uint8_t *__restrict__ gen_vis = nullptr,
+                                                   uint32_t wave_rays = 64) {
     const uint32_t lane = threadIdx.x;
     const uint32_t gtid = blockIdx.x * kBlock + lane;
     int32_t *my_spill = spill + (size_t)gtid * kStackSpill;
@@ -215,7 +229,12 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
         if (clocks && (lane & 63u) == 0) atomicMin(&clocks[0], (unsigned long long)wall_clock64());
     }
 
-    for (uint32_t i = gtid; i < n; i += gridDim.x * kBlock) {
+    // level 1: wave_rays rays per wavefront (rays_per_wave in pvx.hip)
+    const bool part = kLevel == 1 && !kMulti;
+    if (part && (lane & 63u) >= wave_rays) return;
+    const uint32_t i0 = part ? (gtid >> 6) * wave_rays + (lane & 63u) : gtid;
+    const uint32_t istep = part ? gridDim.x * (kBlock / 64) * wave_rays : gridDim.x * kBlock;
+    for (uint32_t i = i0; i < n; i += istep) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
             const uint4 ch = chunks[__builtin_amdgcn_readfirstlane(i >> 6)];
@@ -254,20 +273,11 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             const InfRec inf = sv.inf[k];
             if (kFlags && !precondition(sv.obj_flags[inf.obj], rk)) continue;
             double dep;
-            int32_t prim = 0;
-            bool ok;
-            if (inf.kind == kPrimPlane) {
-                ok = plane_hit(sv.planes[inf.index], o, d, dep) && depth_ok(dep, shadow);
-            } else if (kLevel >= 2) {
-                ok = inf.kind == kPrimQuadric ? quadric_closest(sv.quadrics[inf.index], o, d, shadow, dep)
-                                              : csg_closest<(kLevel >= 3)>(sv, inf.index, o, d, shadow, bt, dep, prim);
-            } else {
-                ok = false;
-            }
-            if (ok && better(dep, inf.obj, prim, bt, bo, bp)) {
+            const bool ok = inf.kind == kPrimPlane && plane_hit(sv.planes[inf.index], o, d, dep) && depth_ok(dep, shadow);
+            if (ok && better(dep, inf.obj, 0, bt, bo, bp)) {
                 bt = dep;
                 bo = inf.obj;
-                bp = prim;
+                bp = 0;
             }
         }
 
@@ -558,6 +568,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                                     bp = 0;
                                 }
                         } else if (kLevel == 1) { // boxes and stand-alone triangles
+                            if (!ref_box_hit(p.ref, rf, tb)) continue;
                             if (pk == kPrimTriangle64) {
                                 double dep;
                                 if (tri_rec_hit(sv.triangles[p.ref.index], o, d, dep) && depth_ok(dep, shadow) &&
@@ -569,27 +580,16 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                             } else {
                                 double hs[2];
                                 int side[2];
-                                int nh = box_hits(sv.boxes[p.ref.index], sv.xforms, o, d, hs, side);
-                                for (int j = 0; j < nh; j++)
-                                    if (depth_ok(hs[j], shadow) && better(hs[j], obj, 0, bt, bo, bp)) {
+                                const int nh = box_hits(sv.boxes[p.ref.index], sv.xforms, o, d, hs, side);
+#pragma unroll
+                                for (int j = 0; j < 2; j++)
+                                    if (j < nh && depth_ok(hs[j], shadow) && better(hs[j], obj, 0, bt, bo, bp)) {
                                         bt = hs[j];
                                         bo = obj;
                                         bp = 0;
                                     }
                             }
-                        } else if (kLevel >= 2) {
-                            double dep;
-                            int32_t prim = 0;
-                            bool ok;
-                            if (pk == kPrimCsg)
-                                ok = csg_closest<(kLevel >= 3)>(sv, p.ref.index, o, d, shadow, bt, dep, prim);
-                            else
-                                ok = simple_closest<(kLevel >= 3)>(sv, pk, p.ref.index, o, d, shadow, dep);
-                            if (ok && better(dep, obj, prim, bt, bo, bp)) {
-                                bt = dep;
-                                bo = obj;
-                                bp = prim;
-                            }
+                            tb = (float)bt * 1.000001f;
                         }
                     }
                     tb = (float)bt * 1.000001f;
@@ -618,6 +618,275 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
         }
         if constexpr (kMulti) {
             if (clocks && (lane & 63u) == 0) atomicMax(&clocks[1 + scene], (unsigned long long)wall_clock64());
+        }
+    }
+}
+
+// Walk of scenes with any primitive kind (kLevel 2: all but lathes and sors;
+// 3: those too) through the binary tree.  What bounds it is the FP64 primitive
+// tests: a torus takes thousands of instructions, a node forty.  So each
+// lane walks nodes, and discards primitives by their own FP32 box, until it
+// holds one primitive to test (or its ray ends); then the lanes of the
+// wavefront test theirs together.  All kinds go through one copy of the
+// shape tests: one per use cost 256 registers and one wavefront per SIMD, and
+// 128 registers (four wavefronts, some spilling) beat both 168 and 256: 1.88,
+// 2.46 and 2.52 ms for the camera rays of the 10,000-leaf CSG field.  Together
+// with the leaves of CSG objects in the tree, the root finder in registers and
+// the filter programs, that launch went from 7.2 to 1.3 ms and the shaded
+// 5,000-leaf glass frame (641 x 359) from 767 to 70 ms.
+//
+// Rays per wavefront: with fewer rays than the resident grid has lanes, a
+// launch gives each wavefront only `wave_rays` of them (a power of two), so
+// that a ray waits for fewer others on its way.
+//
+// kMulti: as in trace_closest_body.
+template <int kLevel, bool kFlags, bool kCount, bool kMulti = false>
+__device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_stack) {
+    const uint32_t wl = threadIdx.x; // a block is one wavefront
+    const uint32_t gtid = blockIdx.x * kRefBlock + wl;
+    int32_t *my_spill = a.spill + (size_t)gtid * kStackSpill;
+    const bool occl = (a.kind & kRayOcclusion) != 0;
+    const uint32_t kind = a.kind & 0xFFu;
+    const bool shadow = (kind == PVX_RAY_SHADOW);
+    const uint32_t n = a.n;
+    if constexpr (kMulti) {
+        if (a.clocks && wl == 0) atomicMin(&a.clocks[0], (unsigned long long)wall_clock64());
+    }
+    const uint32_t per_wave = kMulti ? 64u : a.wave_rays;
+    if (!kMulti && wl >= per_wave) return;
+    const uint32_t step = gridDim.x * per_wave;
+    for (uint32_t i = blockIdx.x * per_wave + wl; i < n; i += step) {
+        uint32_t ri = i, scene = 0;
+        if constexpr (kMulti) {
+            const uint4 ch = a.chunks[__builtin_amdgcn_readfirstlane(i >> 6)];
+            scene = ch.x;
+            if ((i & 63u) >= ch.z) continue; // lane 0 always has a ray
+            ri = ch.y + (i & 63u);
+        }
+        const SceneView &sv = kMulti ? a.views[scene] : a.sv;
+        const uint32_t rk = (kFlags && a.kinds) ? (uint32_t)a.kinds[ri] : kind;
+        const pvx_ray r = a.rays[ri];
+        const D3 o = d3(r.o[0], r.o[1], r.o[2]), d = d3(r.d[0], r.d[1], r.d[2]);
+        double bt = kBoundHuge;
+        if (a.max_depth) {
+            const double md = a.max_depth[ri];
+            if (md >= kEpsilon) bt = md; // trace.cpp:157-158
+        }
+        const double occl_lim = bt - kShadowTolerance;
+        int32_t bo = -1, bp = 0;
+        RayF rf;
+        rf.ix = safe_inv(d.x);
+        rf.iy = safe_inv(d.y);
+        rf.iz = safe_inv(d.z);
+        rf.oix = (float)o.x * rf.ix;
+        rf.oiy = (float)o.y * rf.iy;
+        rf.oiz = (float)o.z * rf.iz;
+        float tb = (float)bt * 1.000001f;
+        uint32_t cnt_nodes = 0, cnt_prims = 0;
+        uint32_t inf_k = 0;             // objects outside the tree come first
+        uint32_t cur = 0, end = 0;      // primitives left of the leaf at hand
+        uint32_t slot_k = 0, slot_e = 0; // leaves left of the whole CSG object at hand
+        int32_t slot_obj = 0;
+        int32_t node = sv.root;
+        int sp = 0;
+        for (;;) {
+            // --- to the next primitive to test: its type, its index in that
+            // type's array, its object and the primitive id of a hit; a CSG
+            // leaf's slot (-1: no CSG filter)
+            uint32_t type = 0, shape = 0, rec = kNoRec, rflags = 0;
+            int32_t obj = 0, slot = -1;
+            const double *sph = nullptr;
+            bool have = false;
+            for (;;) {
+                if (slot_k < slot_e) {
+                    slot = (int32_t)sv.csg_leaves[slot_k++];
+                    const CsgSlot &c = sv.csg_slots[slot];
+                    type = c.type;
+                    shape = c.shape;
+                    rec = c.rec;
+                    rflags = c.rflags;
+                    obj = slot_obj;
+                    have = true;
+                    break;
+                }
+                uint32_t pk, index;
+                if (inf_k < sv.n_inf) {
+                    const InfRec inf = sv.inf[inf_k++];
+                    pk = inf.kind;
+                    index = inf.index;
+                    obj = inf.obj;
+                    if (kFlags && !precondition(sv.obj_flags[obj], rk)) continue;
+                    if (pk == kPrimPlane) {
+                        double dep;
+                        if (plane_hit(sv.planes[index], o, d, dep) && depth_ok(dep, shadow) &&
+                            better(dep, obj, 0, bt, bo, bp)) {
+                            bt = dep;
+                            bo = obj;
+                            bp = 0;
+                            tb = (float)bt * 1.000001f;
+                            if (occl && bt < occl_lim) { // blocked
+                                inf_k = sv.n_inf;
+                                node = kEmpty;
+                            }
+                        }
+                        continue;
+                    }
+                } else if (cur < end) {
+                    const PrimRec &p = sv.prims[cur++];
+                    const uint32_t ka = p.kind_axis;
+                    pk = ka & 15u;
+                    obj = p.obj;
+                    if (kFlags && !precondition(sv.obj_flags[obj], rk)) continue;
+                    if (pk == kPrimTriangle) {
+                        double dep;
+                        const int32_t prim = p.tri.prim;
+                        if (mesh_tri_hit_l<kLevel>(sv, p, ka, o, d, dep) && depth_ok(dep, shadow) &&
+                            better(dep, obj, prim, bt, bo, bp)) {
+                            bt = dep;
+                            bo = obj;
+                            bp = prim;
+                            tb = (float)bt * 1.000001f;
+                            if (occl && bt < occl_lim) {
+                                cur = end;
+                                node = kEmpty;
+                            }
+                        }
+                        continue;
+                    }
+                    if (pk == kPrimSphere) {
+                        sph = p.sph.c;
+                        type = PVX_SPHERE;
+                        have = true;
+                        break;
+                    }
+                    if (!ref_box_hit(p.ref, rf, tb)) continue;
+                    index = p.ref.index;
+                    if (pk != kPrimCsg) {
+                        if (pk == kPrimCsgLeaf) slot = (int32_t)index;
+                        type = p.ref.type;
+                        shape = p.ref.shape;
+                        rec = p.ref.rec;
+                        rflags = p.ref.rflags;
+                        have = true;
+                        break;
+                    }
+                } else if (node >= 0) {
+                    if (kCount) cnt_nodes++;
+                    const float4 *np = reinterpret_cast<const float4 *>(sv.nodes + node);
+                    const float4 na = np[0], nb = np[1], nc = np[2];
+                    const int4 nl = reinterpret_cast<const int4 *>(np)[3];
+                    float x0 = fmaf(na.x, rf.ix, -rf.oix), x1 = fmaf(na.y, rf.ix, -rf.oix);
+                    float y0 = fmaf(na.z, rf.iy, -rf.oiy), y1 = fmaf(na.w, rf.iy, -rf.oiy);
+                    float z0 = fmaf(nc.x, rf.iz, -rf.oiz), z1 = fmaf(nc.y, rf.iz, -rf.oiz);
+                    const float tn0 = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
+                    const float tf0 = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tb));
+                    x0 = fmaf(nb.x, rf.ix, -rf.oix);
+                    x1 = fmaf(nb.y, rf.ix, -rf.oix);
+                    y0 = fmaf(nb.z, rf.iy, -rf.oiy);
+                    y1 = fmaf(nb.w, rf.iy, -rf.oiy);
+                    z0 = fmaf(nc.z, rf.iz, -rf.oiz);
+                    z1 = fmaf(nc.w, rf.iz, -rf.oiz);
+                    const float tn1 = fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fmaxf(fminf(z0, z1), 0.0f));
+                    const float tf1 = fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fminf(fmaxf(z0, z1), tb));
+                    const bool h0 = tn0 <= tf0 * 1.000001f, h1 = tn1 <= tf1 * 1.000001f;
+                    if (h0 && h1) {
+                        const bool swap = tn1 < tn0;
+                        const int32_t farc = swap ? nl.x : nl.y;
+                        if (sp < kStackLds)
+                            s_stack[sp * kRefBlock + wl] = farc;
+                        else
+                            my_spill[sp - kStackLds] = farc;
+                        sp++;
+                        node = swap ? nl.y : nl.x;
+                        continue;
+                    }
+                    if (h0 || h1) {
+                        node = h0 ? nl.x : nl.y;
+                        continue;
+                    }
+                    if (sp == 0) {
+                        node = kEmpty;
+                    } else {
+                        sp--;
+                        node = sp < kStackLds ? s_stack[sp * kRefBlock + wl] : my_spill[sp - kStackLds];
+                    }
+                    continue;
+                } else if (node != kEmpty) {
+                    // leaf: ~node = first << 3 | (count - 1)
+                    const uint32_t leaf = (uint32_t)(~node);
+                    cur = leaf >> 3;
+                    end = cur + (leaf & 7u) + 1u;
+                    if (kCount) cnt_prims += end - cur;
+                    if (sp == 0) {
+                        node = kEmpty;
+                    } else {
+                        sp--;
+                        node = sp < kStackLds ? s_stack[sp * kRefBlock + wl] : my_spill[sp - kStackLds];
+                    }
+                    continue;
+                } else {
+                    break; // the ray's walk is over
+                }
+                if (pk == kPrimCsg) { // a whole CSG object: its leaves one by one
+                    slot_k = sv.csg_leaf_range[2 * index];
+                    slot_e = sv.csg_leaf_range[2 * index + 1];
+                    slot_obj = obj;
+                    continue;
+                }
+                type = PVX_QUADRIC; // the other kind outside the tree
+                shape = index;
+                have = true;
+                break;
+            }
+            if (!have) break;
+            // --- test it: its hits that the CSG filters keep
+            const int32_t prim = slot < 0 ? 0 : slot;
+            auto consider = [&](double dep) {
+                if (!depth_ok(dep, shadow) || !better(dep, obj, prim, bt, bo, bp)) return;
+                if (slot >= 0 && !csg_survives<(kLevel >= 3)>(sv, (uint32_t)slot, add3(o, mul3(d, dep))))
+                    return;
+                bt = dep;
+                bo = obj;
+                bp = prim;
+            };
+            bool done = false;
+            if constexpr (kLevel >= 3) {
+                if (type == PVX_LATHE || type == PVX_SOR) {
+                    rev_visit(sv, shape, o, d, slot >= 0, [&](double dep, int, double) { consider(dep); });
+                    done = true;
+                }
+            }
+            if (!done) {
+                double hs[kMaxLeafHits];
+                int nh;
+                if (rec != kNoRec) {
+                    const PlacedRec &r = sv.placed[rec];
+                    const bool xf = (rflags & kPlacedXf) != 0;
+                    const D3 P = xf ? pl_point(r.inv, o) : o, D = xf ? pl_dir(r.inv, d) : d;
+                    int side[2];
+                    nh = type == PVX_BOX ? box_hits_at(r.q, r.q + 3, P, D, hs, side)
+                                         : torus_hits_at(r.q[0], r.q[1], (rflags & kPlacedSturm) != 0, P, D, hs);
+                } else if (type == PVX_SPHERE) {
+                    const double *s = sph ? sph : sv.sph + 4 * (size_t)shape;
+                    nh = sphere_hits(d3(s[0], s[1], s[2]), s[3], o, d, hs);
+                } else {
+                    nh = other_hits(sv, type, shape, o, d, hs);
+                }
+                // nearest first: once one is kept, the others are farther
+                sort_hits(hs, nh);
+#pragma unroll 1
+                for (int j = 0; j < nh; j++) consider(pick_hit(hs, j));
+            }
+            tb = (float)bt * 1.000001f;
+            if (occl && bo >= 0 && bt < occl_lim) break; // blocked
+        }
+        a.hits[ri] = pvx_hit{bt, bo, bp};
+        if (kCount) {
+            a.node_visits[ri] = cnt_nodes;
+            a.prim_tests[ri] = cnt_prims;
+        }
+        if constexpr (kMulti) {
+            if (a.clocks && wl == 0) atomicMax(&a.clocks[1 + scene], (unsigned long long)wall_clock64());
         }
     }
 }

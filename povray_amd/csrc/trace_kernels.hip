@@ -21,7 +21,19 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kBlock];
     trace_closest_body<kLevel, kFlags, kCount, false>(a.sv, nullptr, nullptr, nullptr, a.rays, a.max_depth, a.kind,
                                                       a.kinds, a.n, a.hits, a.spill, a.node_visits, a.prim_tests,
-                                                      s_stack);
+                                                      s_stack, nullptr, nullptr, 1, nullptr, a.wave_rays);
+}
+
+// Scenes with any primitive kind (levels 2 and 3).
+template <int kLevel, bool kFlags, bool kCount>
+__global__ __launch_bounds__(kRefBlock, 4) void k_trace_ref(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kRefBlock];
+    trace_ref_body<kLevel, kFlags, kCount>(a, s_stack);
+}
+template <int kLevel, bool kFlags, bool kCount>
+__global__ __launch_bounds__(kRefBlock, 4) void k_trace_ref_multi(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kRefBlock];
+    trace_ref_body<kLevel, kFlags, kCount, true>(a, s_stack);
 }
 
 // Level-0 scenes (triangles, spheres, planes) through the binary tree.
@@ -426,6 +438,12 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest_kd(TraceArgs a) {
     }
 }
 
+#define PVX_FC_REF(K, ...)                                                                                     \
+    (k.flags ? (k.count ? run_ref(K<__VA_ARGS__ true, true>, a, nb, st, occ)                                   \
+                        : run_ref(K<__VA_ARGS__ true, false>, a, nb, st, occ))                                 \
+             : (k.count ? run_ref(K<__VA_ARGS__ false, true>, a, nb, st, occ)                                  \
+                        : run_ref(K<__VA_ARGS__ false, false>, a, nb, st, occ)))
+
 #if PVX_TRACE_PART == 12
 // All intersections of one object per ray, sorted ascending
 // (ObjectBase::All_Intersections, object.h:238).
@@ -529,7 +547,7 @@ __global__ void k_inside(SceneView sv, const double *pts, const uint32_t *objs, 
     if (i >= n) return;
     D3 p = d3(pts[3 * (size_t)i], pts[3 * (size_t)i + 1], pts[3 * (size_t)i + 2]);
     uint32_t ob = objs[i];
-    out[i] = shape_inside<kCsgMaxDepth, true>(sv, obj_type[ob], obj_index[ob], obj_flags[ob], p) ? 1 : 0;
+    out[i] = shape_inside<true>(sv, obj_type[ob], obj_index[ob], obj_flags[ob], p) ? 1 : 0;
 }
 #endif
 
@@ -538,6 +556,21 @@ template <class F>
 hipError_t run(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
     if (occ) return hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, reinterpret_cast<const void *>(kfn), kBlock, 0);
     hipLaunchKernelGGL(kfn, dim3(nb), dim3(kBlock), 0, st, a);
+    return hipGetLastError();
+}
+
+// A kernel of one-wavefront blocks: nb blocks of kBlock threads' worth.
+template <class F>
+hipError_t run_ref(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
+    constexpr int per = kBlock / kRefBlock;
+    if (occ) {
+        int w = 0;
+        const hipError_t e =
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&w, reinterpret_cast<const void *>(kfn), kRefBlock, 0);
+        *occ = w / per;
+        return e;
+    }
+    hipLaunchKernelGGL(kfn, dim3(nb * per), dim3(kRefBlock), 0, st, a);
     return hipGetLastError();
 }
 
@@ -575,7 +608,7 @@ hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint
 #elif PVX_TRACE_PART >= 2 && PVX_TRACE_PART <= 5 // single scene, every primitive kind
     constexpr bool kF = (PVX_TRACE_PART - 2) >= 2, kC = (PVX_TRACE_PART - 2) & 1;
     (void)k;
-    return run(k_trace_closest<2, kF, kC>, a, nb, st, occ);
+    return run_ref(k_trace_ref<2, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 6 // kd-tree
     return PVX_FC(k_trace_closest_kd, );
 #elif PVX_TRACE_PART == 7 // scene batches: 4-wide and binary walks
@@ -585,11 +618,11 @@ hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint
 #elif PVX_TRACE_PART >= 8 && PVX_TRACE_PART <= 11 // scene batches, every primitive kind
     constexpr bool kF = (PVX_TRACE_PART - 8) >= 2, kC = (PVX_TRACE_PART - 8) & 1;
     (void)k;
-    return run(k_trace_closest_multi<2, kF, kC>, a, nb, st, occ);
+    return run_ref(k_trace_ref_multi<2, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 13 // single scene with lathes or sors
-    return PVX_FC(k_trace_closest, 3, );
+    return PVX_FC_REF(k_trace_ref, 3, );
 #elif PVX_TRACE_PART == 14 // scene batches with lathes or sors
-    return PVX_FC(k_trace_closest_multi, 3, );
+    return PVX_FC_REF(k_trace_ref_multi, 3, );
 #elif PVX_TRACE_PART == 16 // single scene, level-0 primitives on the binary tree
     return k.walk == kWalkBinary0WW ? PVX_FC(k_trace_closest_bin0, true, ) : PVX_FC(k_trace_closest_bin0, false, );
 #elif PVX_TRACE_PART == 15 // light rays made in the kernel

@@ -16,6 +16,7 @@
 namespace pvx {
 
 constexpr int kBlock = 256;      // threads per block of every traversal kernel
+constexpr int kRefBlock = 64;    // ... of the walks of any primitive kind (one wavefront)
 constexpr int kStackLds = 24;    // traversal-stack entries per lane in LDS
 constexpr int kStackSpill = 40;  // further entries per lane in the spill area
 constexpr int kStackMax = kStackLds + kStackSpill;
@@ -65,6 +66,7 @@ struct TraceArgs {
     uint32_t kind;
     const uint8_t *kinds;
     uint32_t n;
+    uint32_t wave_rays; // walks of referenced primitives: rays per wavefront, a power of two <= 64
     pvx_hit *hits;
     int32_t *spill; // kSpillPerThread bytes for each thread of the grid
     uint32_t *node_visits;
