@@ -75,13 +75,12 @@ constexpr int kWgradItems = 12 + 4 + 4 + 2; // 32x32 gradient tiles of W1..W4
 // fused trainer: points per workgroup, LDS activation row pitch
 constexpr int kTrainPts = 64;
 constexpr int kTrainPitch = kTrainPts + 8;
-constexpr int kTrainThreads = 256;
+constexpr int kTrainThreads = 512;
+constexpr int kOwnParams = 2; // parameters a thread keeps in registers
 constexpr uint32_t kSpinLimit = 1u << 24; // grid-barrier wait bound (about a second)
 
-__device__ inline uint16_t f2bf(float f) { // round to nearest even (finite inputs)
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+__device__ inline uint16_t f2bf(float f) { // round to nearest even: v_cvt_pk_bf16_f32
+    return __builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
 __device__ inline f32x16 mfma(s16x8 a, s16x8 b, f32x16 c) {
@@ -220,24 +219,18 @@ __device__ inline void relu_back(const f32x16 &a0, const f32x16 &a1, const s16x4
     }
 }
 
-// Forward + backward of one 32-point tile (one wavefront).  Features come
-// from F (per point, in K-step order) or are computed from x; activations
-// go to rows of A (element (row, slot) at A[row * pitch + slot]).  Returns
-// the tile's squared error (lane 0).
-__device__ inline float tile_fwd_bwd(const uint16_t *sw, const float *sb, const uint16_t *Fp, const float *x,
-                                     bool valid, const float *target, float dscale, uint16_t *A, uint32_t pitch,
-                                     uint32_t slot) {
+// Forward + backward of one 32-point tile (one wavefront).  feature(s) is
+// the lane's B operand of K step s of layer 1; activations go to rows of A
+// (element (row, slot) at A[row * pitch + slot]).  Returns the tile's squared
+// error (lane 0).
+template <class Feature>
+__device__ inline float tile_fwd_bwd(const uint16_t *sw, const float *sb, Feature &&feature, bool valid,
+                                     const float *target, float dscale, uint16_t *A, uint32_t pitch, uint32_t slot) {
     const int lane = threadIdx.x & 63, p = lane & 31, h = lane >> 5;
     f32x16 a0 = zero16(), a1 = zero16();
+#pragma unroll
     for (int s = 0; s < kMlpIn / 16; s++) {
-        s16x8 b;
-        if (Fp) {
-            b = *reinterpret_cast<const s16x8 *>(Fp + 16 * s + 8 * h);
-            if (!valid)
-                for (int t = 0; t < 8; t++) b[t] = 0;
-        } else {
-            b = feat8(x, s, h);
-        }
+        const s16x8 b = feature(s);
         for (int t = 0; t < 8; t++) {
             const int f = 16 * s + 4 * h + (t & 3) + 8 * (t >> 2);
             A[(size_t)(kRowX0 + f) * pitch + slot] = (uint16_t)b[t];
@@ -370,7 +363,8 @@ __global__ __launch_bounds__(256) void k_mlp_fwd_bwd(TrainArgs a) {
     float x[6];
     for (int c = 0; c < 6; c++) x[c] = valid ? a.x[6 * (size_t)slot + c] : 0.0f;
     const float *tg = a.t + 3 * (size_t)(valid ? slot : 0);
-    const float l2 = tile_fwd_bwd(sw, sb, nullptr, x, valid, tg, a.dscale, a.acts, a.batch, slot);
+    const float l2 = tile_fwd_bwd(
+        sw, sb, [&](int s) { return feat8(x, s, lane >> 5); }, valid, tg, a.dscale, a.acts, a.batch, slot);
     if (lane == 0) a.loss_part[tile] = l2;
 }
 
@@ -415,16 +409,13 @@ __device__ inline void pack_param(uint8_t *pack, int i, float w) {
     }
 }
 
-// One Adam step on parameter i with gradient g (beta 0.9 / 0.99).
-__device__ inline float adam(int i, float g, float *w, float *m, float *v, float lr, float bc1, float bc2) {
+// One Adam step on a parameter with gradient g (beta 0.9 / 0.99).
+__device__ inline float adam(float g, float &w, float &m, float &v, float lr, float bc1, float bc2) {
     const float b1 = 0.9f, b2 = 0.99f, eps = 1e-8f;
-    float mi = b1 * m[i] + (1.0f - b1) * g;
-    float vi = b2 * v[i] + (1.0f - b2) * g * g;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-    w[i] = wi;
-    return wi;
+    m = b1 * m + (1.0f - b1) * g;
+    v = b2 * v + (1.0f - b2) * g * g;
+    w = w - lr * (m / bc1) / (sqrtf(v / bc2) + eps);
+    return w;
 }
 
 enum { kUpdPack = 0, kUpdGrad = 1 };
@@ -449,39 +440,39 @@ __global__ void k_fill_zero(uint32_t *p, size_t n) {
     if (i < n) p[i] = 0u;
 }
 
-// Grid barrier of the cooperative trainer: every thread releases its writes,
-// one thread per block arrives and waits for the generation to move on
-// (bounded: after kSpinLimit polls the error flag is raised and every block
-// leaves).  Returns false once the flag is up.
+// Grid barrier of the cooperative trainer: every wavefront waits until its
+// stores have arrived, then one thread per block releases them, arrives at a
+// counter that only grows (zero at launch) and waits until it has counted
+// `target` arrivals, modulo 2^32 (bounded: after kSpinLimit polls the error flag is raised
+// and every block leaves).  Returns false once the flag is up.  One thread
+// makes the release and the acquire for its block and polls relaxed: a
+// release writes the XCD's L2 back and an acquire drops it, and one of each
+// per wavefront and poll had the waiting blocks empty each other's L2 all
+// along.  Waiting on the arrivals themselves saves the hop through a last
+// arriver.
 struct GridBar {
-    unsigned count, gen, err, pad;
+    unsigned count, err, pad[2];
 };
-__device__ inline bool grid_sync(GridBar *b, unsigned nblocks) {
+__device__ inline bool grid_sync(GridBar *b, unsigned target) {
     __shared__ int s_ok;
-    __threadfence();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0); // vmcnt(0) expcnt(0) lgkmcnt(0)
     __syncthreads();
     if (threadIdx.x == 0) {
-        const unsigned g = __hip_atomic_load(&b->gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned arrived = __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        int ok = 1;
-        if (arrived == nblocks - 1) {
-            __hip_atomic_store(&b->count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&b->gen, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            uint32_t spins = 0;
-            while (__hip_atomic_load(&b->gen, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == g) {
-                __builtin_amdgcn_s_sleep(2);
-                if (++spins > kSpinLimit) {
-                    __hip_atomic_store(&b->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t spins = 0;
+        while ((int32_t)(__hip_atomic_load(&b->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
+            __builtin_amdgcn_s_sleep(1);
+            if (++spins > kSpinLimit) {
+                __hip_atomic_store(&b->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
             }
         }
-        if (__hip_atomic_load(&b->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) ok = 0;
-        s_ok = ok;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        s_ok = __hip_atomic_load(&b->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 0 : 1;
     }
     __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     return s_ok != 0;
 }
 
@@ -500,51 +491,105 @@ struct FusedArgs {
 };
 
 // `steps` Adam steps of batch = 64 x gridDim.x points in one cooperative
-// launch (waves 0 and 1 of a block take 32 points each; all four share the
-// gradient tiles, the reduction and the weight copies).
+// launch (waves 0 and 1 of a block take 32 points each; all eight share the
+// gradient tiles, the reduction and the weight copies).  Latency bounds a
+// step: two grid barriers and a memory round trip after each.  So what does
+// not depend on other blocks is not fetched behind a barrier: the next step's
+// features, targets and rates are loaded before the first one, and with
+// kOwnParams parameters or fewer a thread (a batch of 1,344 points or more)
+// the weights and moments stay in its registers for the whole run.  100 steps
+// of 2,048 points: 3.35 ms with fences and polls by every wavefront, 256
+// threads and the weights in memory; 2.0 ms so (load 1.1, forward + backward
+// 5.9, gradient tiles 2.1, barrier 3.8, reduction + Adam 3.1, barrier 3.8 us
+// a step).
+template <bool kOwn>
 __global__ __launch_bounds__(kTrainThreads) void k_mlp_train(FusedArgs a) {
     __shared__ __align__(16) uint16_t sw[kAllElems];
     __shared__ __align__(16) uint16_t acts[kActRows * kTrainPitch];
     __shared__ float sb[kBiasFloats];
-    const int lane = threadIdx.x & 63, p = lane & 31, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, p = lane & 31, h = lane >> 5, wv = threadIdx.x >> 6;
     const uint32_t G = gridDim.x, wg = blockIdx.x;
     const uint32_t per = (kMlpParams + G - 1) / G;
-    const uint32_t lo = wg * per, hi = min((uint32_t)kMlpParams, lo + per);
+    const uint32_t lo = min((uint32_t)kMlpParams, wg * per), hi = min((uint32_t)kMlpParams, lo + per);
+    float ow[kOwnParams], om[kOwnParams], ov[kOwnParams];
+    if constexpr (kOwn) {
+#pragma unroll
+        for (int q = 0; q < kOwnParams; q++) {
+            const uint32_t i = lo + q * kTrainThreads + threadIdx.x;
+            if (i < hi) {
+                ow[q] = a.w[i];
+                om[q] = a.m[i];
+                ov[q] = a.v[i];
+            }
+        }
+    }
+    s16x8 feat[kMlpIn / 16];
+    float target[3];
+    auto fetch = [&](uint32_t k) { // step k's sample of this lane (waves 0 and 1)
+        const uint32_t slot = (uint32_t)wv * 32 + p;
+        const uint32_t sseed = a.seed + 7919u * (a.step0 + k + 1);
+        const uint32_t src = mix32(sseed * 0x9E3779B9u + wg * kTrainPts + slot) % a.n;
+        const uint16_t *f = a.F + (size_t)src * kMlpIn + 8 * h;
+#pragma unroll
+        for (int s = 0; s < kMlpIn / 16; s++) feat[s] = *reinterpret_cast<const s16x8 *>(f + 16 * s);
+#pragma unroll
+        for (int c = 0; c < 3; c++) target[c] = a.t[3 * (size_t)src + c];
+    };
+    if (wv < 2 && a.steps > 0) fetch(0);
     for (uint32_t k = 0; k < a.steps; k++) {
         load_pack(a.pack, sw, kAllElems, sb);
         __syncthreads();
         // forward + backward of this block's 64 samples
         float l2 = 0.0f;
         if (wv < 2) {
-            const uint32_t slot = (uint32_t)wv * 32 + p;
-            const uint32_t sseed = a.seed + 7919u * (a.step0 + k + 1);
-            const uint32_t src = mix32(sseed * 0x9E3779B9u + wg * kTrainPts + slot) % a.n;
-            l2 = tile_fwd_bwd(sw, sb, a.F + (size_t)src * kMlpIn, nullptr, true, a.t + 3 * (size_t)src, a.dscale,
-                              acts, kTrainPitch, slot);
+            l2 = tile_fwd_bwd(sw, sb, [&](int s) { return feat[s]; }, true, target, a.dscale, acts, kTrainPitch,
+                              (uint32_t)wv * 32 + p);
+            if (k + 1 < a.steps) fetch(k + 1);
         }
         if (lane == 0 && wv < 2) a.loss_part[2 * wg + wv] = l2;
         __syncthreads();
         // this block's partial gradient
         for (uint32_t item = wv; item < (uint32_t)kWgradItems; item += kTrainThreads / 64)
             wgrad_tile(acts, kTrainPitch, 0, kTrainPts, item, a.partial + (size_t)wg * kMlpParams);
-        if (!grid_sync(a.bar, G)) return;
-        // reduce this block's slice of the parameters in block order, Adam
         const float lr = a.sched[3 * k], bc1 = a.sched[3 * k + 1], bc2 = a.sched[3 * k + 2];
-        for (uint32_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-            // block partials summed in block order, sixteen loads in flight
+        if (!grid_sync(a.bar, (2 * k + 1) * G)) return;
+        // reduce this block's slice of the parameters in block order, Adam:
+        // block partials summed in block order, thirty-two loads in flight
+        auto reduce = [&](uint32_t i) {
             float g = 0.0f;
-            for (uint32_t c0 = 0; c0 < G; c0 += 16) {
-                float pv[16];
+            for (uint32_t c0 = 0; c0 < G; c0 += 32) {
+                float pv[32];
 #pragma unroll
-                for (int u = 0; u < 16; u++)
+                for (int u = 0; u < 32; u++)
                     pv[u] = c0 + u < G ? a.partial[(size_t)(c0 + u) * kMlpParams + i] : 0.0f;
 #pragma unroll
-                for (int u = 0; u < 16; u++)
+                for (int u = 0; u < 32; u++)
                     if (c0 + u < G) g += pv[u];
             }
-            pack_param(a.pack, (int)i, adam((int)i, g, a.w, a.m, a.v, lr, bc1, bc2));
+            return g;
+        };
+        if constexpr (kOwn) {
+#pragma unroll
+            for (int q = 0; q < kOwnParams; q++) {
+                const uint32_t i = lo + q * kTrainThreads + threadIdx.x;
+                if (i < hi) pack_param(a.pack, (int)i, adam(reduce(i), ow[q], om[q], ov[q], lr, bc1, bc2));
+            }
+        } else {
+            for (uint32_t i = lo + threadIdx.x; i < hi; i += kTrainThreads)
+                pack_param(a.pack, (int)i, adam(reduce(i), a.w[i], a.m[i], a.v[i], lr, bc1, bc2));
         }
-        if (!grid_sync(a.bar, G)) return;
+        if (!grid_sync(a.bar, (2 * k + 2) * G)) return;
+    }
+    if constexpr (kOwn) {
+#pragma unroll
+        for (int q = 0; q < kOwnParams; q++) {
+            const uint32_t i = lo + q * kTrainThreads + threadIdx.x;
+            if (i < hi) {
+                a.w[i] = ow[q];
+                a.m[i] = om[q];
+                a.v[i] = ov[q];
+            }
+        }
     }
 }
 
@@ -673,12 +718,15 @@ int Surrogate::grad_batch(const float *x, const float *t, uint32_t n, float *los
 }
 
 int Surrogate::max_train_batch() {
-    int per_cu = 0, cus = 0, dev = 0;
+    int per_cu = 0, per_cu2 = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_mlp_train), kTrainThreads, 0) !=
-            hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(k_mlp_train<true>),
+                                                     kTrainThreads, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu2, reinterpret_cast<const void *>(k_mlp_train<false>),
+                                                     kTrainThreads, 0) != hipSuccess)
         return 0;
+    per_cu = std::min(per_cu, per_cu2);
     return per_cu * cus * kTrainPts;
 }
 
@@ -731,8 +779,10 @@ int Surrogate::train(const float *x, const float *t, uint32_t n, uint32_t steps,
         // each partly resident and spinning at its barrier, could hold the
         // CUs the other's missing blocks need
         std::lock_guard<std::mutex> lock(g_train_mu);
-        HIP_TRY(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k_mlp_train), dim3(G), dim3(kTrainThreads),
-                                           args, 0, st));
+        const bool own = (kMlpParams + G - 1) / G <= (uint32_t)(kOwnParams * kTrainThreads);
+        HIP_TRY(hipLaunchCooperativeKernel(
+            reinterpret_cast<const void *>(own ? k_mlp_train<true> : k_mlp_train<false>), dim3(G), dim3(kTrainThreads),
+            args, 0, st));
         step += steps;
         HIP_TRY(hipStreamSynchronize(st));
     }
@@ -741,7 +791,7 @@ int Surrogate::train(const float *x, const float *t, uint32_t n, uint32_t steps,
     HIP_TRY(hipMemcpyAsync(hb, bar.p, 16, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipMemcpyAsync(lp.data(), loss_part.p, lp.size() * 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    if (hb[2]) return fail(PVX_EDEVICE, "training grid barrier timed out");
+    if (hb[1]) return fail(PVX_EDEVICE, "training grid barrier timed out");
     if (final_loss) {
         double sum = 0;
         for (float f : lp) sum += f;
