@@ -295,7 +295,7 @@ enum {
 };
 
 typedef struct pvx_build_opts {
-    uint32_t max_leaf_size; /* triangles per BVH leaf (0 = default 4) */
+    uint32_t max_leaf_size; /* primitives per BVH leaf (0 = default: 1, GPU builder 4) */
     uint32_t sah_bins;      /* binned-SAH bins (0 = default 16)        */
     uint32_t accel;         /* PVX_ACCEL_BVH / PVX_ACCEL_BSP          */
     uint32_t bsp_max_depth; /* BSP tree depth limit (0 = 64, at most 64) */
@@ -366,7 +366,7 @@ int pvx_trace_closest_counted(pvx_scene *scene, const pvx_ray *rays,
  * traversal-stack spill area is a fixed 32 MiB device array of the library
  * (one per device, held until the process ends) instead of the per-stream
  * area pvx_trace_closest allocates on a stream's first launch, so the
- * persistent grid is capped at what it holds (819 blocks of 256 lanes).
+ * persistent grid is capped at what it holds (840 blocks of 256 lanes).
  * Every call on one device shares that array: calls that overlap in time on
  * one device (other streams, other threads) race and must not be issued.
  * The scene must live on the current device (PVX_EINVAL otherwise). */
@@ -386,11 +386,11 @@ enum {
      * only tested for occlusion, with the 4-wide tree walked ... */
     PVX_TRAVERSAL_PACKET = 4,    /* ... by each wavefront as one packet (one shared
                                     stack, ballots of the lanes' box tests)          */
-    PVX_TRAVERSAL_FUSED = 5,     /* ... while-while per lane (the default)          */
+    PVX_TRAVERSAL_FUSED = 5,     /* ... while-while per lane                        */
     PVX_TRAVERSAL_REFILL = 6,    /* ... while-while per lane, a wavefront refilling
                                     its free lanes with the next unstarted rays once
                                     16 or fewer of its lanes still hold rays         */
-    PVX_TRAVERSAL_LIGHT_BINARY = 7, /* ... through the binary tree, per lane      */
+    PVX_TRAVERSAL_LIGHT_BINARY = 7, /* ... through the binary tree (the default)  */
     PVX_TRAVERSAL_BINARY_WW = 8, /* binary tree, while-while (triangle/sphere scenes) */
     PVX_TRAVERSAL_REFILL_BINARY = 9 /* pvx_render's light rays as REFILL, through the
                                        binary tree                                  */

@@ -143,17 +143,131 @@ class Builder {
         return ~(int32_t)((start << 3) | (count - 1));
     }
 
-    // Choose a split for [b, e); returns the split position m (b < m < e).
-    uint32_t split(uint32_t b, uint32_t e, int depth, Box3 &lb, Box3 &rb) {
-        Box3 cb;
-        cb.empty();
-        for (uint32_t i = b; i < e; i++) {
-            const float *c = &cen_[3 * (size_t)idx_[i]];
-            for (int k = 0; k < 3; k++) {
-                cb.lo[k] = std::min(cb.lo[k], c[k]);
-                cb.hi[k] = std::max(cb.hi[k], c[k]);
+    // Boxes and counts of the primitives whose centroid falls in each bin of
+    // each axis.
+    struct Bins {
+        Box3 bb[3][kMaxBins];
+        uint32_t cnt[3][kMaxBins];
+        void clear(int bins) {
+            for (int a = 0; a < 3; a++)
+                for (int i = 0; i < bins; i++) {
+                    bb[a][i].empty();
+                    cnt[a][i] = 0;
+                }
+        }
+        void add(const Bins &o, int bins) {
+            for (int a = 0; a < 3; a++)
+                for (int i = 0; i < bins; i++) {
+                    bb[a][i].grow(o.bb[a][i]);
+                    cnt[a][i] += o.cnt[a][i];
+                }
+        }
+    };
+
+    int bin_of(uint32_t p, int a, float lo, float scale) const {
+        const int bi = (int)((cen_[3 * (size_t)p + a] - lo) * scale);
+        return std::min(bins_ - 1, std::max(0, bi));
+    }
+
+    // work(begin, end, result) over [b, e) and, where the range is above the
+    // grain of the subtree workers (the serial top of the tree), over parts of
+    // it on threads of their own, merged into `out`: minima, maxima and
+    // counts, so the result does not depend on the parts.  `out` is empty on
+    // entry.
+    template <class T, class Work, class Merge>
+    void in_parts(uint32_t b, uint32_t e, T &out, Work &&work, Merge &&merge) {
+        if (e - b <= 2 * kParallelGrain) {
+            work(b, e, out);
+            return;
+        }
+        const uint32_t parts =
+            std::min({16u, std::max(1u, std::thread::hardware_concurrency()), (e - b) / kParallelGrain});
+        std::vector<T> res(parts, out);
+        std::vector<std::thread> pool;
+        for (uint32_t k = 0; k < parts; k++)
+            pool.emplace_back([&, k]() {
+                work(b + (uint32_t)((uint64_t)(e - b) * k / parts), b + (uint32_t)((uint64_t)(e - b) * (k + 1) / parts),
+                     res[k]);
+            });
+        for (auto &t : pool) t.join();
+        for (const T &r : res) merge(out, r);
+    }
+
+    // A split of a few primitives: every position of every axis' centroid
+    // order.  Trees with one primitive a leaf make most of their splits here,
+    // where clearing and sweeping the bins costs several times the work.
+    // False when all centroids coincide.
+    static constexpr uint32_t kSweepMax = 8;
+    bool sweep_split(uint32_t b, uint32_t e, uint32_t &m, Box3 &lb, Box3 &rb) {
+        const uint32_t n = e - b;
+        Box3 box[kSweepMax];
+        for (uint32_t i = 0; i < n; i++) box[i] = prim_box(idx_[b + i]);
+        uint8_t best[kSweepMax] = {0};
+        float best_cost = INFINITY;
+        uint32_t best_k = 0;
+        for (int a = 0; a < 3; a++) {
+            uint8_t ord[kSweepMax];
+            float key[kSweepMax];
+            for (uint32_t i = 0; i < n; i++) { // insertion sort, stable
+                const float c = cen_[3 * (size_t)idx_[b + i] + a];
+                uint32_t j = i;
+                for (; j > 0 && key[j - 1] > c; j--) {
+                    key[j] = key[j - 1];
+                    ord[j] = ord[j - 1];
+                }
+                key[j] = c;
+                ord[j] = (uint8_t)i;
+            }
+            if (!(key[n - 1] > key[0])) continue;
+            float right[kSweepMax];
+            Box3 acc = box[ord[n - 1]];
+            for (uint32_t k = n - 1; k > 0; k--) {
+                right[k] = acc.half_area() * (float)(n - k);
+                acc.grow(box[ord[k - 1]]);
+            }
+            acc = box[ord[0]];
+            for (uint32_t k = 1; k < n; k++) {
+                const float cost = acc.half_area() * (float)k + right[k];
+                if (cost < best_cost) {
+                    best_cost = cost;
+                    best_k = k;
+                    std::memcpy(best, ord, n);
+                }
+                acc.grow(box[ord[k]]);
             }
         }
+        if (best_k == 0) return false;
+        uint32_t id[kSweepMax];
+        for (uint32_t i = 0; i < n; i++) id[i] = idx_[b + best[i]];
+        lb = box[best[0]];
+        for (uint32_t i = 1; i < best_k; i++) lb.grow(box[best[i]]);
+        rb = box[best[best_k]];
+        for (uint32_t i = best_k + 1; i < n; i++) rb.grow(box[best[i]]);
+        std::copy(id, id + n, idx_.begin() + b);
+        m = b + best_k;
+        return true;
+    }
+
+    // Choose a split for [b, e); returns the split position m (b < m < e).
+    uint32_t split(uint32_t b, uint32_t e, int depth, Box3 &lb, Box3 &rb) {
+        if (e - b == 2) {
+            lb = prim_box(idx_[b]);
+            rb = prim_box(idx_[b + 1]);
+            return b + 1;
+        }
+        uint32_t sm;
+        if (e - b <= kSweepMax && depth < kSahDepthLimit && sweep_split(b, e, sm, lb, rb)) return sm;
+        Box3 cb;
+        cb.empty();
+        in_parts<Box3>(b, e, cb, [&](uint32_t pb, uint32_t pe, Box3 &r) {
+            for (uint32_t i = pb; i < pe; i++) {
+                const float *c = &cen_[3 * (size_t)idx_[i]];
+                for (int k = 0; k < 3; k++) {
+                    r.lo[k] = std::min(r.lo[k], c[k]);
+                    r.hi[k] = std::max(r.hi[k], c[k]);
+                }
+            }
+        }, [](Box3 &x, const Box3 &y) { x.grow(y); });
         int axis = 0;
         float ext = cb.hi[0] - cb.lo[0];
         for (int k = 1; k < 3; k++)
@@ -162,25 +276,33 @@ class Builder {
                 axis = k;
             }
         uint32_t m = b + (e - b) / 2;
-        bool done = false;
         if (ext > 0.0f && depth < kSahDepthLimit) {
             // binned SAH over all three axes
             float best_cost = INFINITY;
             int best_axis = -1, best_bin = -1;
+            float scale[3];
             for (int a = 0; a < 3; a++) {
-                float extent = cb.hi[a] - cb.lo[a];
-                if (!(extent > 0.0f)) continue;
-                Box3 bb[kMaxBins];
-                uint32_t cnt[kMaxBins] = {0};
-                for (int i = 0; i < bins_; i++) bb[i].empty();
-                float scale = bins_ / extent;
-                for (uint32_t i = b; i < e; i++) {
-                    uint32_t p = idx_[i];
-                    int bi = (int)((cen_[3 * (size_t)p + a] - cb.lo[a]) * scale);
-                    bi = std::min(bins_ - 1, std::max(0, bi));
-                    cnt[bi]++;
-                    bb[bi].grow(prim_box(p));
+                const float extent = cb.hi[a] - cb.lo[a];
+                scale[a] = extent > 0.0f ? bins_ / extent : 0.0f;
+            }
+            Bins bn;
+            bn.clear(bins_);
+            in_parts<Bins>(b, e, bn, [&](uint32_t pb, uint32_t pe, Bins &r) {
+                for (uint32_t i = pb; i < pe; i++) {
+                    const uint32_t p = idx_[i];
+                    const Box3 bx = prim_box(p);
+                    for (int a = 0; a < 3; a++) {
+                        if (!(scale[a] > 0.0f)) continue;
+                        const int bi = bin_of(p, a, cb.lo[a], scale[a]);
+                        r.cnt[a][bi]++;
+                        r.bb[a][bi].grow(bx);
+                    }
                 }
+            }, [&](Bins &x, const Bins &y) { x.add(y, bins_); });
+            for (int a = 0; a < 3; a++) {
+                if (!(scale[a] > 0.0f)) continue;
+                const Box3 *bb = bn.bb[a];
+                const uint32_t *cnt = bn.cnt[a];
                 float right_area[kMaxBins];
                 uint32_t right_cnt[kMaxBins];
                 Box3 acc;
@@ -207,26 +329,24 @@ class Builder {
                 }
             }
             if (best_axis >= 0) {
-                float scale = bins_ / (cb.hi[best_axis] - cb.lo[best_axis]);
-                float lo_a = cb.lo[best_axis];
-                auto mid = std::partition(idx_.begin() + b, idx_.begin() + e, [&](uint32_t p) {
-                    int bi = (int)((cen_[3 * (size_t)p + best_axis] - lo_a) * scale);
-                    bi = std::min(bins_ - 1, std::max(0, bi));
-                    return bi <= best_bin;
-                });
+                const float lo_a = cb.lo[best_axis], sc = scale[best_axis];
+                auto mid = std::partition(idx_.begin() + b, idx_.begin() + e,
+                                          [&](uint32_t p) { return bin_of(p, best_axis, lo_a, sc) <= best_bin; });
                 m = (uint32_t)(mid - idx_.begin());
-                done = (m > b && m < e);
+                if (m > b && m < e) { // the children's boxes are their bins'
+                    lb.empty();
+                    rb.empty();
+                    for (int i = 0; i < bins_; i++) (i <= best_bin ? lb : rb).grow(bn.bb[best_axis][i]);
+                    return m;
+                }
             }
         }
-        if (!done) {
-            // object median along the widest centroid axis
-            m = b + (e - b) / 2;
-            std::nth_element(idx_.begin() + b, idx_.begin() + m, idx_.begin() + e,
-                             [&](uint32_t p, uint32_t q) {
-                                 float cp = cen_[3 * (size_t)p + axis], cq = cen_[3 * (size_t)q + axis];
-                                 return cp < cq || (cp == cq && p < q);
-                             });
-        }
+        // object median along the widest centroid axis
+        m = b + (e - b) / 2;
+        std::nth_element(idx_.begin() + b, idx_.begin() + m, idx_.begin() + e, [&](uint32_t p, uint32_t q) {
+            float cp = cen_[3 * (size_t)p + axis], cq = cen_[3 * (size_t)q + axis];
+            return cp < cq || (cp == cq && p < q);
+        });
         lb.empty();
         rb.empty();
         for (uint32_t i = b; i < m; i++) lb.grow(prim_box(idx_[i]));
@@ -323,12 +443,24 @@ void node_children(const Node &m, Cand &a, Cand &b) {
     b = Cand{m.c1, {m.lo1x, m.lo1y, m.lo1z}, {m.hi1x, m.hi1y, m.hi1z}};
 }
 
-int32_t collapse_rec(const std::vector<Node> &nodes, int32_t n, uint32_t d, std::vector<Node4> &out,
-                     uint32_t &depth) {
+// The primitives of each binary node's subtree, a contiguous range.
+struct Range {
+    uint32_t first, count;
+};
+
+int32_t collapse_rec(const std::vector<Node> &nodes, const std::vector<Range> &range, uint32_t leaf, int32_t n,
+                     uint32_t d, std::vector<Node4> &out, uint32_t &depth) {
     depth = std::max(depth, d);
+    // a child whose subtree holds no more than `leaf` primitives is a leaf
+    auto children = [&](int32_t node, Cand &a, Cand &b) {
+        node_children(nodes[node], a, b);
+        for (Cand *c : {&a, &b})
+            if (c->link >= 0 && range[c->link].count <= leaf)
+                c->link = ~(int32_t)((range[c->link].first << 3) | (range[c->link].count - 1));
+    };
     Cand c[4];
     int cnt = 2;
-    node_children(nodes[n], c[0], c[1]);
+    children(n, c[0], c[1]);
     while (cnt < 4) {
         int best = -1;
         float ba = -1.0f;
@@ -339,7 +471,7 @@ int32_t collapse_rec(const std::vector<Node> &nodes, int32_t n, uint32_t d, std:
             }
         if (best < 0) break;
         Cand a, b;
-        node_children(nodes[c[best].link], a, b);
+        children(c[best].link, a, b);
         c[best] = a;
         c[cnt++] = b;
     }
@@ -350,7 +482,7 @@ int32_t collapse_rec(const std::vector<Node> &nodes, int32_t n, uint32_t d, std:
         if (k >= cnt)
             links[k] = INT32_MIN;
         else
-            links[k] = c[k].link >= 0 ? collapse_rec(nodes, c[k].link, d + 1, out, depth) : c[k].link;
+            links[k] = c[k].link >= 0 ? collapse_rec(nodes, range, leaf, c[k].link, d + 1, out, depth) : c[k].link;
     }
     Node4 &w = out[(size_t)idx];
     for (int k = 0; k < 4; k++) {
@@ -369,16 +501,26 @@ int32_t collapse_rec(const std::vector<Node> &nodes, int32_t n, uint32_t d, std:
 
 } // namespace
 
-void collapse_bvh4(const std::vector<Node> &nodes, int32_t root, std::vector<Node4> &nodes4, int32_t &root4,
-                   uint32_t &depth4) {
+void collapse_bvh4(const std::vector<Node> &nodes, int32_t root, uint32_t leaf, std::vector<Node4> &nodes4,
+                   int32_t &root4, uint32_t &depth4) {
     nodes4.clear();
     depth4 = 0;
     if (root < 0) { // empty, or a single leaf
         root4 = root;
         return;
     }
+    std::vector<Range> range(nodes.size());
+    for (size_t i = nodes.size(); i-- > 0;) { // children come after their parent
+        auto of = [&](int32_t link) {
+            if (link >= 0) return range[link];
+            const uint32_t l = (uint32_t)~link;
+            return Range{l >> 3, (l & 7u) + 1u};
+        };
+        const Range a = of(nodes[i].c0), b = of(nodes[i].c1);
+        range[i] = Range{std::min(a.first, b.first), a.count + b.count};
+    }
     nodes4.reserve(nodes.size() / 2 + 1);
-    root4 = collapse_rec(nodes, root, 0, nodes4, depth4);
+    root4 = collapse_rec(nodes, range, leaf, root, 0, nodes4, depth4);
 }
 
 } // namespace pvx

@@ -155,7 +155,8 @@ struct pvx_batch {
     std::vector<pvx_scene *> scenes;
     uint32_t level = 0;     // largest has_complex of the scenes
     uint32_t any_flags = 0; // union of the scenes' object flags
-    uint32_t grid_ww = 0, grid = 0;
+    uint32_t grid = 0;      // resident blocks of the batch's walk
+    bool whole = false;     // its launches cover all rays (no scene can outgrow the LDS stack)
     pvx::DevBuf views, chunks, spill;
     pvx::HostBuf hchunks;
     hipEvent_t uploaded = nullptr; // last chunk-table upload (guards hchunks)

@@ -122,8 +122,7 @@ hipError_t pvx::trace_launch(const TraceKernel &k, const TraceArgs &a, uint32_t 
         }
     }
     switch (k.walk) {
-    case kWalkStep4:
-    case kWalkWW4:
+    case kWalkBinary0:
     case kWalkBinary: return trace_part7(k, a, nb, st, occ);
     case kWalkRevolution: return trace_part14(k, a, nb, st, occ);
     case kWalkComplex:
@@ -378,7 +377,7 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
         const TraceKernel k{level >= 3   ? kWalkRevolution
                             : level == 2 ? kWalkComplex
                             : level == 1 ? kWalkBinary
-                                         : kWalkWW4,
+                                         : kWalkBinary0,
                             h.any_flags != 0, false, false};
         TraceArgs none{};
         HIP_TRY(trace_launch(k, none, 0, nullptr, &per_cu));
@@ -431,6 +430,18 @@ extern "C" int pvx_scene_get_stats(const pvx_scene *s, pvx_scene_stats *out) {
     return PVX_OK;
 }
 
+// A walk whose stack cannot outgrow its LDS entries needs no spill area per
+// resident lane, so its launch covers all rays (kWholeGrid) instead of a
+// persistent grid: the hardware then hands out wavefronts as others end.  A
+// persistent grid with a fixed stride left less than half of its places
+// filled (camera rays of the 1.3M-triangle icosphere: 2.3 of 5 wavefronts per
+// SIMD on average).
+constexpr uint32_t kWholeGrid = 0x7FFFFFFFu;
+static bool stack_in_lds(const HostScene &h, bool wide) {
+    // a binary node pushes at most one link, a wide one three
+    return (wide ? 3 * (h.depth4 + 1) : h.depth + 1) <= (uint32_t)kStackLds;
+}
+
 // Rays per wavefront of a launch of n rays on a grid of `grid` blocks: 64,
 // halved while the grid still holds every wavefront at once.  A wavefront
 // runs every path that any of its rays takes, so below a full grid fewer rays
@@ -453,13 +464,10 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
     int r;
     if (!spill && (r = scene_spill(s, st, &spill))) return r;
     const uint32_t level = kernel_level(s->view);
-    // Walks of any primitive kind whose stack fits in LDS need no spill area
-    // per resident thread, so the launch covers all rays and the hardware
-    // hands out the wavefronts as others end: a ray's cost varies a hundredfold
-    // there (10,000-leaf CSG field, 921,600 rays: 1.89 ms on the persistent
-    // grid, 1.67 ms so).
-    if (!s->use_kd && level >= 2 && s->host.depth + 1 <= (uint32_t)kStackLds) grid = 0x7FFFFFFFu;
-    const uint32_t wave_rays = !s->use_kd && level >= 1 ? rays_per_wave(n, s->grid) : 64u;
+    const bool wide = level == 0 && (variant == PVX_TRAVERSAL_WIDE_WW || variant == PVX_TRAVERSAL_WIDE_STEP);
+    if (!s->use_kd && stack_in_lds(s->host, wide)) grid = kWholeGrid;
+    const bool few = !s->use_kd && !wide && variant != PVX_TRAVERSAL_BINARY_WW;
+    const uint32_t wave_rays = few ? rays_per_wave(n, s->grid) : 64u;
     uint32_t nblocks = (uint32_t)std::min<size_t>(grid, (n + 4 * wave_rays - 1) / (4 * wave_rays));
     const bool flags = s->view.any_flags != 0 && (ray_kind != PVX_RAY_PRIMARY || kinds);
     TraceKernel k{kWalkStep4, flags, kCount, false};
@@ -471,11 +479,14 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
         k.walk = kWalkComplex;
     else if (level == 0 && variant == PVX_TRAVERSAL_BINARY_WW)
         k.walk = kWalkBinary0WW;
-    else if (level == 1 || variant == PVX_TRAVERSAL_BINARY)
-        k.walk = level == 0 ? kWalkBinary0 : kWalkBinary;
-    else if (variant == PVX_TRAVERSAL_WIDE_WW ||
-             (variant == PVX_TRAVERSAL_DEFAULT && (ray_kind & 0xFFu) != PVX_RAY_SHADOW))
+    else if (level == 1)
+        k.walk = kWalkBinary;
+    else if (variant == PVX_TRAVERSAL_WIDE_WW)
         k.walk = kWalkWW4;
+    else if (variant == PVX_TRAVERSAL_WIDE_STEP)
+        k.walk = kWalkStep4;
+    else
+        k.walk = kWalkBinary0;
     TraceArgs ta{};
     ta.sv = s->view;
     ta.kd = s->kd;
@@ -622,12 +633,13 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     int r;
     int32_t *spill = nullptr;
     if ((r = scene_spill(s, st, &spill))) return r;
-    // by default the fixed-stride walk on twice the resident blocks (the
-    // light rays of one shaded point differ little in length, the tail of a
-    // launch more: 19.3 ms against 21.8 ms on the resident grid for the
-    // 1.3M-triangle frame); the refilling walk on the resident blocks, which
-    // have no tail to fill
-    const uint32_t grid = grid_blocks ? grid_blocks : next ? s->grid : 2 * s->grid;
+    // the fixed-stride walks on twice the resident blocks (the light rays of
+    // one shaded point differ little in length, the tail of a launch more:
+    // 19.3 ms against 21.8 ms on the resident grid for the 1.3M-triangle
+    // frame); the refilling walk on the resident blocks, which have no tail
+    // to fill; the binary walk over all rays when its stack fits in LDS
+    uint32_t grid = grid_blocks ? grid_blocks : next ? s->grid : 2 * s->grid;
+    if (!next && binary && stack_in_lds(s->host, false)) grid = kWholeGrid;
     const uint32_t nb = (uint32_t)std::min<size_t>(grid, ((size_t)n_rays + kBlock - 1) / kBlock);
     TraceArgs ta{};
     ta.wave_rays = 64;
@@ -701,6 +713,10 @@ extern "C" int pvx_trace_closest_noalloc(pvx_scene *s, const pvx_ray *rays, cons
 // ----------------------------------------------------------------------------
 // scene batches
 // ----------------------------------------------------------------------------
+static TraceWalk batch_walk(uint32_t level) {
+    return level >= 3 ? kWalkRevolution : level == 2 ? kWalkComplex : level == 1 ? kWalkBinary : kWalkBinary0;
+}
+
 extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx_batch **out) {
     if (!out) return fail(PVX_EINVAL, "null argument");
     *out = nullptr;
@@ -733,25 +749,21 @@ extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx
         pvx_batch_destroy(b);
         return fail(PVX_EDEVICE, std::string("batch set-up: ") + hipGetErrorString(e));
     }
-    // persistent grids of the two kernel families the batch can launch
-    int cus = 0, per_ww = 0, per = 0;
-    const TraceKernel kb{level >= 3   ? kWalkRevolution
-                         : level == 2 ? kWalkComplex
-                         : level == 1 ? kWalkBinary
-                                      : kWalkStep4,
-                         flags != 0, false, true};
-    const TraceKernel kw{kWalkWW4, flags != 0, false, true};
+    // the walk of the most demanding scene: over all rays when every scene's
+    // stack fits in LDS, else on a persistent grid
+    int cus = 0, per = 0;
+    const TraceKernel kb{batch_walk(level), flags != 0, false, true};
     TraceArgs none{};
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) e = trace_launch(kb, none, 0, nullptr, &per);
-    if (e == hipSuccess) e = trace_launch(kw, none, 0, nullptr, &per_ww);
     if (e != hipSuccess) {
         pvx_batch_destroy(b);
         return fail(PVX_EDEVICE, std::string("batch occupancy: ") + hipGetErrorString(e));
     }
     b->grid = (uint32_t)(cus * std::max(per, 1));
-    b->grid_ww = (uint32_t)(cus * std::max(per_ww, 1));
-    const size_t spill_bytes = (size_t)std::max(b->grid, b->grid_ww) * kBlock * kStackSpill * sizeof(int32_t);
+    b->whole = true;
+    for (const pvx_scene *s : b->scenes) b->whole = b->whole && stack_in_lds(s->host, false);
+    const size_t spill_bytes = (size_t)b->grid * kBlock * kStackSpill * sizeof(int32_t);
     if ((r = b->spill.reserve(spill_bytes)) != PVX_OK) {
         pvx_batch_destroy(b);
         return r;
@@ -823,17 +835,11 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     if (!rays || !hits) return fail(PVX_EINVAL, "null ray or hit buffer");
     const uint32_t n = b->n_chunks * 64u;
     const bool flags = b->any_flags != 0 && ray_kind != PVX_RAY_PRIMARY;
-    const bool ww = b->level == 0 && ray_kind != PVX_RAY_SHADOW;
-    const uint32_t nblocks = std::min<uint32_t>(ww ? b->grid_ww : b->grid, (n + kBlock - 1) / kBlock);
+    const uint32_t nblocks = std::min<uint32_t>(b->whole ? kWholeGrid : b->grid, (n + kBlock - 1) / kBlock);
     const SceneView *views = static_cast<const SceneView *>(b->views.p);
     const uint4 *chunks = static_cast<const uint4 *>(b->chunks.p);
     int32_t *spill = static_cast<int32_t *>(b->spill.p);
-    const TraceKernel k{b->level >= 3   ? kWalkRevolution
-                        : b->level == 2 ? kWalkComplex
-                        : b->level == 1 ? kWalkBinary
-                        : ww            ? kWalkWW4
-                                        : kWalkStep4,
-                        flags, kCount, true};
+    const TraceKernel k{batch_walk(b->level), flags, kCount, true};
     TraceArgs ta{};
     ta.wave_rays = 64;
     ta.views = views;

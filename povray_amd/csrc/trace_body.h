@@ -27,6 +27,26 @@ __device__ inline float safe_inv(double d) {
     return 1.0f / f;
 }
 
+// Node steps of the binary walk between two leaf passes.  A wavefront runs the
+// FP64 leaf code in every pass in which one of its lanes is at a leaf; with a
+// few node steps before it more lanes are.  Camera rays of the 1.3M-triangle
+// icosphere with 1, 2, 3, 4, 6, 8, 12 steps: 881, 833, 760, 735, 725, 735,
+// 779 us with four primitives a leaf, 591, 618, 654, 715 us from 4 on with
+// one; until every lane is at a leaf (while-while): 1071 us.
+constexpr int kNodeSteps = 4;
+
+// Blocks go to the eight XCDs in turn, each with an L2 of its own: the place
+// of this block's rays such that sixteen neighbouring wavefronts (of rays
+// that mostly walk the same nodes) share one (camera rays of the
+// 1.3M-triangle icosphere 568 -> 556 us, its reflections at 327,680 triangles
+// 253 -> 242 us; 4 or 64 neighbours: 571 and 560, 245 and 241 us).  Blocks past
+// the last whole group keep their place.
+__device__ __forceinline__ uint32_t xcd_block() {
+    constexpr uint32_t kXcds = 8, kRun = 16;
+    const uint32_t b = blockIdx.x, whole = gridDim.x / (kXcds * kRun) * (kXcds * kRun);
+    return b < whole ? (b / (kXcds * kRun) * kXcds + b % kXcds) * kRun + b / kXcds % kRun : b;
+}
+
 // Slab test of one referenced primitive's own box, as the nodes test theirs:
 // a leaf's primitives share a node box, and the FP64 tests behind this one
 // cost tens (a box) to thousands (a torus) of instructions.
@@ -218,7 +238,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                                                    uint32_t gen_S = 1, uint8_t *__restrict__ gen_vis = nullptr,
                                                    uint32_t wave_rays = 64) {
     const uint32_t lane = threadIdx.x;
-    const uint32_t gtid = blockIdx.x * kBlock + lane;
+    const uint32_t gtid = blockIdx.x * kWaveBlock + lane; // a block is one wavefront
     int32_t *my_spill = spill + (size_t)gtid * kStackSpill;
     // kRayOcclusion on a light-ray launch: stop at the first hit that the
     // caller counts as blocking (closer than max depth - SHADOW_TOLERANCE)
@@ -226,14 +246,14 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
     kind &= 0xFFu;
     const bool shadow = (kind == PVX_RAY_SHADOW);
     if constexpr (kMulti) {
-        if (clocks && (lane & 63u) == 0) atomicMin(&clocks[0], (unsigned long long)wall_clock64());
+        if (clocks && lane == 0) atomicMin(&clocks[0], (unsigned long long)wall_clock64());
     }
 
-    // level 1: wave_rays rays per wavefront (rays_per_wave in pvx.hip)
-    const bool part = kLevel == 1 && !kMulti;
-    if (part && (lane & 63u) >= wave_rays) return;
-    const uint32_t i0 = part ? (gtid >> 6) * wave_rays + (lane & 63u) : gtid;
-    const uint32_t istep = part ? gridDim.x * (kBlock / 64) * wave_rays : gridDim.x * kBlock;
+    // binary walks: wave_rays rays per wavefront (rays_per_wave in pvx.hip)
+    const bool part = (kLevel == 1 || kBin) && !kMulti && !kGen;
+    if (part && lane >= wave_rays) return;
+    const uint32_t i0 = xcd_block() * (part ? wave_rays : (uint32_t)kWaveBlock) + lane;
+    const uint32_t istep = gridDim.x * (part ? wave_rays : (uint32_t)kWaveBlock);
     for (uint32_t i = i0; i < n; i += istep) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
@@ -304,7 +324,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             node = kEmpty;                                                              \
         } else {                                                                        \
             sp--;                                                                       \
-            node = sp < kStackLds ? s_stack[sp * kBlock + lane] : my_spill[sp - kStackLds]; \
+            node = sp < kStackLds ? s_stack[sp * kWaveBlock + lane] : my_spill[sp - kStackLds]; \
         }                                                                               \
     } while (0)
         // one 4-wide inner-node step (triangle / sphere scenes): the hit
@@ -340,7 +360,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             };
             auto push = [&](int32_t x) {
                 if (sp < kStackLds)
-                    s_stack[sp * kBlock + lane] = x;
+                    s_stack[sp * kWaveBlock + lane] = x;
                 else
                     my_spill[sp - kStackLds] = x;
                 sp++;
@@ -441,7 +461,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                         farc = l.x;
                     }
                     if (sp < kStackLds)
-                        s_stack[sp * kBlock + lane] = farc;
+                        s_stack[sp * kWaveBlock + lane] = farc;
                     else
                         my_spill[sp - kStackLds] = farc;
                     sp++;
@@ -497,7 +517,8 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             }
         } else {
             while (node != kEmpty) {
-                if (node >= 0) {
+                for (int kk = 0; kk < kNodeSteps; kk++) {
+                    if (node < 0) break;
                     if (kCount) cnt_nodes++;
                     const float4 *np = reinterpret_cast<const float4 *>(sv.nodes + node);
                     const float4 a = np[0], b = np[1], c = np[2];
@@ -524,7 +545,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                             farc = l.x;
                         }
                         if (sp < kStackLds)
-                            s_stack[sp * kBlock + lane] = farc;
+                            s_stack[sp * kWaveBlock + lane] = farc;
                         else
                             my_spill[sp - kStackLds] = farc;
                         sp++;
@@ -539,7 +560,9 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                         node = l.y;
                         continue;
                     }
-                } else {
+                    PVX_POP();
+                }
+                if (node < 0 && node != kEmpty) {
                     // leaf: ~node = first << 3 | (count - 1)
                     const uint32_t leaf = (uint32_t)(~node);
                     const uint32_t first = leaf >> 3, count = (leaf & 7u) + 1u;
@@ -597,13 +620,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                         node = kEmpty;
                         continue;
                     }
-                }
-                // pop
-                if (sp == 0) {
-                    node = kEmpty;
-                } else {
-                    sp--;
-                    node = sp < kStackLds ? s_stack[sp * kBlock + lane] : my_spill[sp - kStackLds];
+                    PVX_POP();
                 }
             }
         }
@@ -617,7 +634,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             prim_tests[ri] = cnt_prims;
         }
         if constexpr (kMulti) {
-            if (clocks && (lane & 63u) == 0) atomicMax(&clocks[1 + scene], (unsigned long long)wall_clock64());
+            if (clocks && lane == 0) atomicMax(&clocks[1 + scene], (unsigned long long)wall_clock64());
         }
     }
 }
@@ -643,7 +660,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
 template <int kLevel, bool kFlags, bool kCount, bool kMulti = false>
 __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_stack) {
     const uint32_t wl = threadIdx.x; // a block is one wavefront
-    const uint32_t gtid = blockIdx.x * kRefBlock + wl;
+    const uint32_t gtid = blockIdx.x * kWaveBlock + wl;
     int32_t *my_spill = a.spill + (size_t)gtid * kStackSpill;
     const bool occl = (a.kind & kRayOcclusion) != 0;
     const uint32_t kind = a.kind & 0xFFu;
@@ -793,7 +810,7 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                         const bool swap = tn1 < tn0;
                         const int32_t farc = swap ? nl.x : nl.y;
                         if (sp < kStackLds)
-                            s_stack[sp * kRefBlock + wl] = farc;
+                            s_stack[sp * kWaveBlock + wl] = farc;
                         else
                             my_spill[sp - kStackLds] = farc;
                         sp++;
@@ -808,7 +825,7 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                         node = kEmpty;
                     } else {
                         sp--;
-                        node = sp < kStackLds ? s_stack[sp * kRefBlock + wl] : my_spill[sp - kStackLds];
+                        node = sp < kStackLds ? s_stack[sp * kWaveBlock + wl] : my_spill[sp - kStackLds];
                     }
                     continue;
                 } else if (node != kEmpty) {
@@ -821,7 +838,7 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                         node = kEmpty;
                     } else {
                         sp--;
-                        node = sp < kStackLds ? s_stack[sp * kRefBlock + wl] : my_spill[sp - kStackLds];
+                        node = sp < kStackLds ? s_stack[sp * kWaveBlock + wl] : my_spill[sp - kStackLds];
                     }
                     continue;
                 } else {

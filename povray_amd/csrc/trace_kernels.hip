@@ -17,8 +17,8 @@ namespace pvx {
 namespace {
 
 template <int kLevel, bool kFlags, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_trace_closest(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock) void k_trace_closest(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_closest_body<kLevel, kFlags, kCount, false>(a.sv, nullptr, nullptr, nullptr, a.rays, a.max_depth, a.kind,
                                                       a.kinds, a.n, a.hits, a.spill, a.node_visits, a.prim_tests,
                                                       s_stack, nullptr, nullptr, 1, nullptr, a.wave_rays);
@@ -26,13 +26,13 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest(TraceArgs a) {
 
 // Scenes with any primitive kind (levels 2 and 3).
 template <int kLevel, bool kFlags, bool kCount>
-__global__ __launch_bounds__(kRefBlock, 4) void k_trace_ref(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kRefBlock];
+__global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_ref_body<kLevel, kFlags, kCount>(a, s_stack);
 }
 template <int kLevel, bool kFlags, bool kCount>
-__global__ __launch_bounds__(kRefBlock, 4) void k_trace_ref_multi(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kRefBlock];
+__global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref_multi(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_ref_body<kLevel, kFlags, kCount, true>(a, s_stack);
 }
 
@@ -41,19 +41,20 @@ __global__ __launch_bounds__(kRefBlock, 4) void k_trace_ref_multi(TraceArgs a) {
 // leaves, needs 108 and spills; forcing 6 here spills and is slower).
 // kWW: while-while passes (inner nodes, then leaves, lane by lane).
 template <bool kWW, bool kFlags, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_trace_closest_bin0(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock) void k_trace_closest_bin0(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_closest_body<0, kFlags, kCount, kWW, false, false, true>(a.sv, nullptr, nullptr, nullptr, a.rays,
                                                                     a.max_depth, a.kind, a.kinds, a.n, a.hits,
-                                                                    a.spill, a.node_visits, a.prim_tests, s_stack);
+                                                                    a.spill, a.node_visits, a.prim_tests, s_stack,
+                                                                    nullptr, nullptr, 1, nullptr, a.wave_rays);
 }
 
 // Triangle scenes, camera and bounce rays: while-while traversal (78 VGPRs
 // and a 24 KB LDS stack per block: 6 wavefronts per SIMD; forcing 7 or 8
 // costs more in register pressure than it gains).
 template <bool kFlags, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_trace_closest_ww(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock) void k_trace_closest_ww(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_closest_body<0, kFlags, kCount, true>(a.sv, nullptr, nullptr, nullptr, a.rays, a.max_depth, a.kind,
                                                 a.kinds, a.n, a.hits, a.spill, a.node_visits, a.prim_tests, s_stack);
 }
@@ -63,8 +64,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest_ww(TraceArgs a) {
 // byte per ray.  5 wavefronts per SIMD: held to 80 VGPRs for 6 it was
 // slower (18.7 against 18.3 ms of light passes on the 1.3M-triangle frame).
 template <bool kFlags>
-__global__ __launch_bounds__(kBlock, 5) void k_light_ww(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock, 5) void k_light_ww(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
     trace_closest_body<0, kFlags, false, true, false, true>(a.sv, nullptr, nullptr, nullptr, nullptr, nullptr,
                                                             PVX_RAY_SHADOW | kRayOcclusion, nullptr, n, nullptr,
@@ -74,8 +75,8 @@ __global__ __launch_bounds__(kBlock, 5) void k_light_ww(TraceArgs a) {
 
 // The same light rays through the binary tree (level-0 leaf tests only).
 template <bool kFlags>
-__global__ __launch_bounds__(kBlock) void k_light_bin(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock) void k_light_bin(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
     trace_closest_body<0, kFlags, false, false, false, true, true>(
         a.sv, nullptr, nullptr, nullptr, nullptr, nullptr, PVX_RAY_SHADOW | kRayOcclusion, nullptr, n, nullptr, a.spill,
@@ -92,14 +93,14 @@ __global__ __launch_bounds__(kBlock) void k_light_bin(TraceArgs a) {
 // (92-96 VGPRs, no spills; held to 80 for 6 it spills and the camera-hit
 // light rays of the 1.3M-triangle frame take 12.2 instead of 11.3 ms).
 template <bool kFlags, bool kBin>
-__global__ __launch_bounds__(kBlock, 5) void k_light_dyn(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock, 5) void k_light_dyn(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     const SceneView &sv = a.sv;
     const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
     const uint32_t lane = threadIdx.x;
-    const uint32_t gtid = blockIdx.x * kBlock + lane;
+    const uint32_t gtid = blockIdx.x * kWaveBlock + lane;
     int32_t *my_spill = a.spill + (size_t)gtid * kStackSpill;
-    const uint32_t wl = lane & 63u;
+    const uint32_t wl = lane;
     bool have = false, done = false;
     uint32_t ri = 0;
     D3 o{0, 0, 0}, d{0, 0, 1};
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_light_dyn(TraceArgs a) {
     int sp = 0;
     auto push = [&](int32_t x) {
         if (sp < kStackLds)
-            s_stack[sp * kBlock + lane] = x;
+            s_stack[sp * kWaveBlock + lane] = x;
         else
             my_spill[sp - kStackLds] = x;
         sp++;
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_light_dyn(TraceArgs a) {
             node = kEmpty;
         } else {
             sp--;
-            node = sp < kStackLds ? s_stack[sp * kBlock + lane] : my_spill[sp - kStackLds];
+            node = sp < kStackLds ? s_stack[sp * kWaveBlock + lane] : my_spill[sp - kStackLds];
         }
     };
     while (true) {
@@ -297,19 +298,19 @@ __global__ __launch_bounds__(kBlock, 5) void k_light_dyn(TraceArgs a) {
 
 // The same kernels over a batch of scenes (chunk table and SceneView table).
 template <int kLevel, bool kFlags, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_trace_closest_multi(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
+__global__ __launch_bounds__(kWaveBlock) void k_trace_closest_multi(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_closest_body<kLevel, kFlags, kCount, false, true>(a.views[0], a.views, a.chunks, a.clocks, a.rays,
                                                             a.max_depth, a.kind, a.kinds, a.n, a.hits, a.spill,
                                                             a.node_visits, a.prim_tests, s_stack);
 }
 
 template <bool kFlags, bool kCount>
-__global__ __launch_bounds__(kBlock) void k_trace_closest_ww_multi(TraceArgs a) {
-    __shared__ int32_t s_stack[kStackLds * kBlock];
-    trace_closest_body<0, kFlags, kCount, true, true>(a.views[0], a.views, a.chunks, a.clocks, a.rays, a.max_depth,
-                                                      a.kind, a.kinds, a.n, a.hits, a.spill, a.node_visits,
-                                                      a.prim_tests, s_stack);
+__global__ __launch_bounds__(kWaveBlock) void k_trace_closest_bin0_multi(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
+    trace_closest_body<0, kFlags, kCount, false, true, false, true>(a.views[0], a.views, a.chunks, a.clocks, a.rays,
+                                                                     a.max_depth, a.kind, a.kinds, a.n, a.hits,
+                                                                     a.spill, a.node_visits, a.prim_tests, s_stack);
 }
 
 // Closest hit through the kd-tree (BSPTree::operator()(ray),
@@ -438,12 +439,6 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest_kd(TraceArgs a) {
     }
 }
 
-#define PVX_FC_REF(K, ...)                                                                                     \
-    (k.flags ? (k.count ? run_ref(K<__VA_ARGS__ true, true>, a, nb, st, occ)                                   \
-                        : run_ref(K<__VA_ARGS__ true, false>, a, nb, st, occ))                                 \
-             : (k.count ? run_ref(K<__VA_ARGS__ false, true>, a, nb, st, occ)                                  \
-                        : run_ref(K<__VA_ARGS__ false, false>, a, nb, st, occ)))
-
 #if PVX_TRACE_PART == 12
 // All intersections of one object per ray, sorted ascending
 // (ObjectBase::All_Intersections, object.h:238).
@@ -561,16 +556,16 @@ hipError_t run(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ
 
 // A kernel of one-wavefront blocks: nb blocks of kBlock threads' worth.
 template <class F>
-hipError_t run_ref(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
-    constexpr int per = kBlock / kRefBlock;
+hipError_t run_waves(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
+    constexpr int per = kBlock / kWaveBlock;
     if (occ) {
         int w = 0;
         const hipError_t e =
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&w, reinterpret_cast<const void *>(kfn), kRefBlock, 0);
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&w, reinterpret_cast<const void *>(kfn), kWaveBlock, 0);
         *occ = w / per;
         return e;
     }
-    hipLaunchKernelGGL(kfn, dim3(nb * per), dim3(kRefBlock), 0, st, a);
+    hipLaunchKernelGGL(kfn, dim3(nb * per), dim3(kWaveBlock), 0, st, a);
     return hipGetLastError();
 }
 
@@ -579,9 +574,9 @@ hipError_t run_ref(F *kfn, const TraceArgs &a, uint32_t nb, hipStream_t st, int 
 #define PVX_FN2(n) trace_part##n
 #define PVX_FN(n) PVX_FN2(n)
 // flags x count selection of one template
-#define PVX_FC(K, ...)                                                                                         \
-    (k.flags ? (k.count ? run(K<__VA_ARGS__ true, true>, a, nb, st, occ) : run(K<__VA_ARGS__ true, false>, a, nb, st, occ)) \
-             : (k.count ? run(K<__VA_ARGS__ false, true>, a, nb, st, occ) : run(K<__VA_ARGS__ false, false>, a, nb, st, occ)))
+#define PVX_FC(RUN, K, ...)                                                                                    \
+    (k.flags ? (k.count ? RUN(K<__VA_ARGS__ true, true>, a, nb, st, occ) : RUN(K<__VA_ARGS__ true, false>, a, nb, st, occ)) \
+             : (k.count ? RUN(K<__VA_ARGS__ false, true>, a, nb, st, occ) : RUN(K<__VA_ARGS__ false, false>, a, nb, st, occ)))
 
 #if PVX_TRACE_PART == 12
 hipError_t launch_all_intersections(const SceneView &sv, const pvx_ray *rays, const uint32_t *objs, uint32_t n,
@@ -602,37 +597,36 @@ hipError_t launch_inside(const SceneView &sv, const double *pts, const uint32_t 
 #else
 hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
 #if PVX_TRACE_PART == 0 // single scene, 4-wide walks
-    return k.walk == kWalkWW4 ? PVX_FC(k_trace_closest_ww, ) : PVX_FC(k_trace_closest, 0, );
+    return k.walk == kWalkWW4 ? PVX_FC(run_waves, k_trace_closest_ww, ) : PVX_FC(run_waves, k_trace_closest, 0, );
 #elif PVX_TRACE_PART == 1 // single scene, binary walk
-    return PVX_FC(k_trace_closest, 1, );
+    return PVX_FC(run_waves, k_trace_closest, 1, );
 #elif PVX_TRACE_PART >= 2 && PVX_TRACE_PART <= 5 // single scene, every primitive kind
     constexpr bool kF = (PVX_TRACE_PART - 2) >= 2, kC = (PVX_TRACE_PART - 2) & 1;
     (void)k;
-    return run_ref(k_trace_ref<2, kF, kC>, a, nb, st, occ);
+    return run_waves(k_trace_ref<2, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 6 // kd-tree
-    return PVX_FC(k_trace_closest_kd, );
+    return PVX_FC(run, k_trace_closest_kd, );
 #elif PVX_TRACE_PART == 7 // scene batches: 4-wide and binary walks
-    return k.walk == kWalkWW4    ? PVX_FC(k_trace_closest_ww_multi, )
-           : k.walk == kWalkStep4 ? PVX_FC(k_trace_closest_multi, 0, )
-                                  : PVX_FC(k_trace_closest_multi, 1, );
+    return k.walk == kWalkBinary0 ? PVX_FC(run_waves, k_trace_closest_bin0_multi, )
+                                  : PVX_FC(run_waves, k_trace_closest_multi, 1, );
 #elif PVX_TRACE_PART >= 8 && PVX_TRACE_PART <= 11 // scene batches, every primitive kind
     constexpr bool kF = (PVX_TRACE_PART - 8) >= 2, kC = (PVX_TRACE_PART - 8) & 1;
     (void)k;
-    return run_ref(k_trace_ref_multi<2, kF, kC>, a, nb, st, occ);
+    return run_waves(k_trace_ref_multi<2, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 13 // single scene with lathes or sors
-    return PVX_FC_REF(k_trace_ref, 3, );
+    return PVX_FC(run_waves, k_trace_ref, 3, );
 #elif PVX_TRACE_PART == 14 // scene batches with lathes or sors
-    return PVX_FC_REF(k_trace_ref_multi, 3, );
+    return PVX_FC(run_waves, k_trace_ref_multi, 3, );
 #elif PVX_TRACE_PART == 16 // single scene, level-0 primitives on the binary tree
-    return k.walk == kWalkBinary0WW ? PVX_FC(k_trace_closest_bin0, true, ) : PVX_FC(k_trace_closest_bin0, false, );
+    return k.walk == kWalkBinary0WW ? PVX_FC(run_waves, k_trace_closest_bin0, true, ) : PVX_FC(run_waves, k_trace_closest_bin0, false, );
 #elif PVX_TRACE_PART == 15 // light rays made in the kernel
     if (k.walk == kWalkLightDyn)
-        return k.flags ? run(k_light_dyn<true, false>, a, nb, st, occ) : run(k_light_dyn<false, false>, a, nb, st, occ);
+        return k.flags ? run_waves(k_light_dyn<true, false>, a, nb, st, occ) : run_waves(k_light_dyn<false, false>, a, nb, st, occ);
     if (k.walk == kWalkLightDynBin)
-        return k.flags ? run(k_light_dyn<true, true>, a, nb, st, occ) : run(k_light_dyn<false, true>, a, nb, st, occ);
+        return k.flags ? run_waves(k_light_dyn<true, true>, a, nb, st, occ) : run_waves(k_light_dyn<false, true>, a, nb, st, occ);
     if (k.walk == kWalkLightBin)
-        return k.flags ? run(k_light_bin<true>, a, nb, st, occ) : run(k_light_bin<false>, a, nb, st, occ);
-    return k.flags ? run(k_light_ww<true>, a, nb, st, occ) : run(k_light_ww<false>, a, nb, st, occ);
+        return k.flags ? run_waves(k_light_bin<true>, a, nb, st, occ) : run_waves(k_light_bin<false>, a, nb, st, occ);
+    return k.flags ? run_waves(k_light_ww<true>, a, nb, st, occ) : run_waves(k_light_ww<false>, a, nb, st, occ);
 #else
 #error "PVX_TRACE_PART out of range"
 #endif

@@ -15,11 +15,16 @@
 
 namespace pvx {
 
-constexpr int kBlock = 256;      // threads per block of every traversal kernel
-constexpr int kRefBlock = 64;    // ... of the walks of any primitive kind (one wavefront)
-constexpr int kStackLds = 24;    // traversal-stack entries per lane in LDS
-constexpr int kStackSpill = 40;  // further entries per lane in the spill area
+constexpr int kBlock = 256;      // lanes per unit of a traversal grid (threads per block of the kd walk)
+// Threads per block of the BVH walks: one wavefront, so that its place is
+// free for the next one as soon as it ends (a kBlock unit is four of them).
+constexpr int kWaveBlock = 64;
+constexpr int kStackLds = 25;    // traversal-stack entries per lane in LDS (see below)
+constexpr int kStackSpill = 39;  // further entries per lane in the spill area
 constexpr int kStackMax = kStackLds + kStackSpill;
+// 25 entries are 6,400 bytes a wavefront: 25 wavefronts fit a CU's 160 KB, and
+// the walks' registers allow 24.  (26 entries leave room for 21: camera rays
+// of the 1.3M-triangle icosphere 565 -> 659 us.)
 constexpr int32_t kEmpty = INT32_MIN;
 
 // Spill-area bytes per resident thread of a traversal grid.
