@@ -114,6 +114,8 @@ hipError_t pvx::trace_launch(const TraceKernel &k, const TraceArgs &a, uint32_t 
                                                                                                           occ);
         case kWalkKd: return trace_part6(k, a, nb, st, occ);
         case kWalkRevolution: return trace_part13(k, a, nb, st, occ);
+        case kWalkChain: return trace_part17(k, a, nb, st, occ);
+        case kWalkChainRev: return trace_part18(k, a, nb, st, occ);
         case kWalkLightWW:
         case kWalkLightDyn:
         case kWalkLightBin:
@@ -660,6 +662,37 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     ta.gen_refill_below = 16;
     HIP_TRY(trace_launch(TraceKernel{next ? (binary ? kWalkLightDynBin : kWalkLightDyn) : binary ? kWalkLightBin : kWalkLightWW,
                                      s->view.any_flags != 0, false, false},
+                         ta, nb, st));
+    return PVX_OK;
+}
+
+// Light rays followed through transparent objects (kWalkChain); false: the
+// scene's walk has no such form.
+bool pvx::has_light_chain(const pvx_scene *s) { return !s->use_kd && kernel_level(s->view) >= 2; }
+
+int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *depth, const uint32_t *owner, size_t n,
+                              uint32_t ray_kind, const MatRec *mats, float *col, uint32_t *more, hipStream_t st) {
+    if (n == 0) return PVX_OK;
+    int r;
+    int32_t *spill = nullptr;
+    if ((r = scene_spill(s, st, &spill))) return r;
+    TraceArgs ta{};
+    // the resident grid: a lane whose ray has ended takes another while the
+    // others follow theirs through further layers
+    ta.wave_rays = rays_per_wave(n, s->grid);
+    const uint32_t nb = (uint32_t)std::min<size_t>(s->grid, (n + 4 * ta.wave_rays - 1) / (4 * ta.wave_rays));
+    ta.sv = s->view;
+    ta.rays = rays;
+    ta.max_depth = depth;
+    ta.kind = ray_kind;
+    ta.n = (uint32_t)n;
+    ta.spill = spill;
+    ta.chain_mats = mats;
+    ta.chain_col = col;
+    ta.chain_owner = owner;
+    ta.chain_more = more;
+    HIP_TRY(trace_launch(TraceKernel{kernel_level(s->view) >= 3 ? kWalkChainRev : kWalkChain, s->view.any_flags != 0,
+                                     false, false},
                          ta, nb, st));
     return PVX_OK;
 }

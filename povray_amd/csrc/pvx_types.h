@@ -24,6 +24,7 @@ constexpr double kSmallTolerance = 1.0e-3;
 constexpr double kMaxDistance = 1.0e7;
 constexpr double kMinIsectDepth = 1.0e-4;
 constexpr double kShadowTolerance = 1.0e-3; // SHADOW_TOLERANCE (render/trace.cpp:81)
+constexpr int kMaxShadowSteps = 64; // transparent layers followed per light ray
 // Internal ray-kind bit: a light-ray launch whose caller only needs to know
 // whether something blocks the light (every material opaque).
 constexpr uint32_t kRayOcclusion = 0x100u;

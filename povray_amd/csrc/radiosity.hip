@@ -89,51 +89,74 @@ __global__ void k_lookup(const RadQuery *__restrict__ q, const uint32_t *__restr
         if (cx >= 0 && cy >= 0 && cz >= 0 && cx < c.dims[0] && cy < c.dims[1] && cz < c.dims[2]) {
             const float fb = (float)bound * 1.0001f;
             uint32_t cid = ((uint32_t)cz * c.dims[1] + (uint32_t)cy) * c.dims[0] + (uint32_t)cx;
-            for (uint32_t k = c.cell_start[cid]; k < c.cell_start[cid + 1]; k++) {
-                const RadRec *bp = c.recs + c.cell_items[k];
-                // FP32 pre-test of the quick-check sphere (conservative)
-                float fx = qx - bp->p[0], fy = qy - bp->p[1], fz = qz - bp->p[2];
-                float fq = bp->r * fb;
-                if (fx * fx + fy * fy + fz * fz > fq * fq + 1e-12f) continue;
-                const RadRec b = *bp;
-                double dx = qq.p[0] - b.p[0], dy = qq.p[1] - b.p[1], dz = qq.p[2] - b.p[2];
-                double sq = dx * dx + dy * dy + dz * dz;
-                double quick = (double)b.r * bound;
-                if (!(sq < quick * quick)) continue;
-                double dist = sqrt(sq);
-                double ri = b.r;
-                bool far = dist > kAvgNearEps;
-                double ux = 0, uy = 0, uz = 0;
-                if (far) {
-                    ux = dx / dist;
-                    uy = dy / dist;
-                    uz = dz / dist;
-                    double cs = b.tn[0] * ux + b.tn[1] * uy + b.tn[2] * uz;
-                    if (cs > 0.0) ri = cs * b.nearest + (1.0 - cs) * ri;
+            // FP32 pre-test of the quick-check sphere (conservative), kBatch
+            // records at a time: item, then record, is a chain of two loads
+            // whose latency bounds a lookup, so several are in flight; the
+            // ones that pass are taken in list order (a plain frame of the
+            // 5,000-box room at 1280x720: 8.8 -> 6.3 ms of lookups)
+            constexpr uint32_t kBatch = 8;
+            const uint32_t kend = c.cell_start[cid + 1];
+            for (uint32_t k0 = c.cell_start[cid]; k0 < kend; k0 += kBatch) {
+                uint32_t it[kBatch];
+                float bx[kBatch], by[kBatch], bz[kBatch], br[kBatch];
+#pragma unroll
+                for (uint32_t u = 0; u < kBatch; u++) it[u] = c.cell_items[min(k0 + u, kend - 1)];
+#pragma unroll
+                for (uint32_t u = 0; u < kBatch; u++) {
+                    const RadRec &rr = c.recs[it[u]];
+                    bx[u] = rr.p[0];
+                    by[u] = rr.p[1];
+                    bz[u] = rr.p[2];
+                    br[u] = rr.r;
                 }
-                if (!(dist < ri * bound)) continue;
-                double dd = (double)qq.n[0] * b.n[0] + (double)qq.n[1] * b.n[1] + (double)qq.n[2] * b.n[2];
-                double err = dist / ri + 2.0 * sqrt(fabs(1.0 - dd));
-                if (!(err < bound)) continue;
-                double in_front = 1.0;
-                if (far) {
-                    double hx = qq.n[0] + b.n[0], hy = qq.n[1] + b.n[1], hz = qq.n[2] + b.n[2];
-                    in_front = (ux * hx + uy * hy + uz * hz) / sqrt(hx * hx + hy * hy + hz * hz);
+                uint32_t pass = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < kBatch; u++) {
+                    const float fx = qx - bx[u], fy = qy - by[u], fz = qz - bz[u], fq = br[u] * fb;
+                    if (k0 + u < kend && !(fx * fx + fy * fy + fz * fz > fq * fq + 1e-12f)) pass |= 1u << u;
                 }
-                if (!(in_front > kInFrontLimit)) continue;
-                double w;
-                if (!sigmoid) {
-                    w = 1.0 - err / bound;
-                } else { // PSEUDO_SIGMOID_METHOD (final pass, bounce depth 0)
-                    w = err / bound;
-                    w = w < 0.5 ? 1.0 - (w * 2.0) * (w * 2.0) / 2.0 : ((1.0 - w) * 2.0) * ((1.0 - w) * 2.0) / 2.0;
-                }
-                if (in_front <= 0) w = w * (1 - in_front / kInFrontLimit);
-                if (w > kRadEps) {
-                    we[0] += b.E[0] * w;
-                    we[1] += b.E[1] * w;
-                    we[2] += b.E[2] * w;
-                    W += w;
+                for (; pass; pass &= pass - 1) {
+                    const uint32_t u = (uint32_t)__ffs((int)pass) - 1u;
+                    const RadRec b = c.recs[c.cell_items[k0 + u]];
+                    double dx = qq.p[0] - b.p[0], dy = qq.p[1] - b.p[1], dz = qq.p[2] - b.p[2];
+                    double sq = dx * dx + dy * dy + dz * dz;
+                    double quick = (double)b.r * bound;
+                    if (!(sq < quick * quick)) continue;
+                    double dist = sqrt(sq);
+                    double ri = b.r;
+                    bool far = dist > kAvgNearEps;
+                    double ux = 0, uy = 0, uz = 0;
+                    if (far) {
+                        ux = dx / dist;
+                        uy = dy / dist;
+                        uz = dz / dist;
+                        double cs = b.tn[0] * ux + b.tn[1] * uy + b.tn[2] * uz;
+                        if (cs > 0.0) ri = cs * b.nearest + (1.0 - cs) * ri;
+                    }
+                    if (!(dist < ri * bound)) continue;
+                    double dd = (double)qq.n[0] * b.n[0] + (double)qq.n[1] * b.n[1] + (double)qq.n[2] * b.n[2];
+                    double err = dist / ri + 2.0 * sqrt(fabs(1.0 - dd));
+                    if (!(err < bound)) continue;
+                    double in_front = 1.0;
+                    if (far) {
+                        double hx = qq.n[0] + b.n[0], hy = qq.n[1] + b.n[1], hz = qq.n[2] + b.n[2];
+                        in_front = (ux * hx + uy * hy + uz * hz) / sqrt(hx * hx + hy * hy + hz * hz);
+                    }
+                    if (!(in_front > kInFrontLimit)) continue;
+                    double w;
+                    if (!sigmoid) {
+                        w = 1.0 - err / bound;
+                    } else { // PSEUDO_SIGMOID_METHOD (final pass, bounce depth 0)
+                        w = err / bound;
+                        w = w < 0.5 ? 1.0 - (w * 2.0) * (w * 2.0) / 2.0 : ((1.0 - w) * 2.0) * ((1.0 - w) * 2.0) / 2.0;
+                    }
+                    if (in_front <= 0) w = w * (1 - in_front / kInFrontLimit);
+                    if (w > kRadEps) {
+                        we[0] += b.E[0] * w;
+                        we[1] += b.E[1] * w;
+                        we[2] += b.E[2] * w;
+                        W += w;
+                    }
                 }
             }
         }

@@ -32,7 +32,6 @@ namespace {
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr int kMaxInteriors = 10;           // objects a ray can be inside at once
-constexpr int kMaxShadowSteps = 64;         // transparent layers followed per light ray
 
 // Ray type bits, as Ray::SetFlags(type, parent) sets them (ray.cpp:155-166).
 enum : uint8_t { kFPrimary = 1, kFRefl = 2, kFRefr = 4, kFContinued = 8 };
@@ -1152,6 +1151,23 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
             } else {
                 tune[1] = pvx_tune_result{0, 0, 0.0, 0.0, 0, 0}; // no light rays: nothing to tune
             }
+        }
+        if (ns > 0 && has_light_chain(s)) { // every layer in one launch
+            HIP_TRY(hipEventRecord(t0, st));
+            k_zero_counters<<<1, 64, 0, st>>>(counters);
+            if ((rc = light_chain_internal(s, static_cast<const pvx_ray *>(b.srays[0].p),
+                                           static_cast<const double *>(b.sdepth[0].p),
+                                           static_cast<const uint32_t *>(b.sowner[0].p), ns, light_kind, sh.d_mats,
+                                           static_cast<float *>(b.scol.p), counters, st)))
+                return rc;
+            HIP_TRY(hipEventRecord(t1, st));
+            uint32_t more;
+            HIP_TRY(hipMemcpyAsync(&more, counters, 4, hipMemcpyDeviceToHost, st));
+            HIP_TRY(hipStreamSynchronize(st));
+            HIP_TRY(hipEventElapsedTime(&ms, t0, t1));
+            shadow_ms += ms;
+            n_shadow += (uint64_t)ns + more;
+            ns = 0;
         }
         for (int step = 0; ns > 0 && step < kMaxShadowSteps; step++) {
             HIP_TRY(hipEventRecord(t0, st));

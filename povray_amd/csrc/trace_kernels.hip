@@ -10,7 +10,7 @@
 #include "trace_launch.h"
 
 #ifndef PVX_TRACE_PART
-#error "build with -DPVX_TRACE_PART=<0..16>"
+#error "build with -DPVX_TRACE_PART=<0..18>"
 #endif
 
 namespace pvx {
@@ -29,6 +29,11 @@ template <int kLevel, bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     trace_ref_body<kLevel, kFlags, kCount>(a, s_stack);
+}
+template <int kLevel, bool kFlags>
+__global__ __launch_bounds__(kWaveBlock, 4) void k_light_chain(TraceArgs a) {
+    __shared__ int32_t s_stack[kStackLds * kWaveBlock];
+    trace_ref_body<kLevel, kFlags, false, false, true>(a, s_stack);
 }
 template <int kLevel, bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref_multi(TraceArgs a) {
@@ -627,6 +632,10 @@ hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint
     if (k.walk == kWalkLightBin)
         return k.flags ? run_waves(k_light_bin<true>, a, nb, st, occ) : run_waves(k_light_bin<false>, a, nb, st, occ);
     return k.flags ? run_waves(k_light_ww<true>, a, nb, st, occ) : run_waves(k_light_ww<false>, a, nb, st, occ);
+#elif PVX_TRACE_PART == 17 // light rays through transparent objects
+    return k.flags ? run_waves(k_light_chain<2, true>, a, nb, st, occ) : run_waves(k_light_chain<2, false>, a, nb, st, occ);
+#elif PVX_TRACE_PART == 18
+    return k.flags ? run_waves(k_light_chain<3, true>, a, nb, st, occ) : run_waves(k_light_chain<3, false>, a, nb, st, occ);
 #else
 #error "PVX_TRACE_PART out of range"
 #endif

@@ -3,7 +3,7 @@
 // The traversal kernels are templates over the walk, the object-flag
 // precondition, the counting mode and single/multi-scene batches.  They are
 // instantiated in trace_kernels.hip, which the Makefile compiles once per
-// part (PVX_TRACE_PART = 0..16), each part holding a few instantiations, so
+// part (PVX_TRACE_PART = 0..18), each part holding a few instantiations, so
 // that they build in parallel; trace_launch() picks the part.
 #ifndef PVX_TRACE_LAUNCH_H
 #define PVX_TRACE_LAUNCH_H
@@ -47,7 +47,9 @@ enum TraceWalk : uint32_t {
     kWalkBinary0 = 8,  // level-0 scene (triangles, spheres) through the binary tree
     kWalkLightBin = 9,  // light rays made in the kernel, binary tree (occlusion)
     kWalkBinary0WW = 10, // kWalkBinary0 in while-while passes
-    kWalkLightDynBin = 11 // kWalkLightDyn through the binary tree
+    kWalkLightDynBin = 11, // kWalkLightDyn through the binary tree
+    kWalkChain = 12,       // light rays through transparent objects, every kind but lathes and sors
+    kWalkChainRev = 13     // ... with lathes and sors
 };
 
 struct TraceKernel {
@@ -86,6 +88,12 @@ struct TraceArgs {
     uint8_t *gen_vis;
     uint32_t *gen_next; // kWalkLightDyn: next ray to hand out (zero at launch)
     const uint32_t *gen_count; // when set: n = gen_count[0] * gen_S, read on the device
+    // kWalkChain: ray k's colour is chain_col[3 * chain_owner[k]]; the number
+    // of continued rays is added to chain_more
+    const MatRec *chain_mats;
+    float *chain_col;
+    const uint32_t *chain_owner;
+    uint32_t *chain_more;
     uint32_t gen_refill_below; // kWalkLightDyn: refill once no more than this many lanes hold rays
 };
 
@@ -123,6 +131,8 @@ PVX_TRACE_PART_DECL(13);
 PVX_TRACE_PART_DECL(14);
 PVX_TRACE_PART_DECL(15);
 PVX_TRACE_PART_DECL(16);
+PVX_TRACE_PART_DECL(17);
+PVX_TRACE_PART_DECL(18);
 
 } // namespace pvx
 
