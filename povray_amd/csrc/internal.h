@@ -181,7 +181,7 @@ int trace_closest_internal(pvx_scene *s, const pvx_ray *rays, const double *max_
 // the number of groups there and n_rays only bounds the grid.  `binary`:
 // through the binary tree (one node or leaf per pass per lane).
 bool has_light_chain(const pvx_scene *s);
-int light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *depth, const uint32_t *owner, size_t n,
+int light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *depth, size_t n,
                          uint32_t ray_kind, const MatRec *mats, float *col, uint32_t *more, hipStream_t st);
 int light_rays_internal(pvx_scene *s, const LightGroup *groups, const LightRec *lights, uint32_t S,
                         uint32_t n_rays, uint8_t *vis, uint32_t *next, uint32_t grid, const uint32_t *count,

@@ -670,7 +670,7 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
 // scene's walk has no such form.
 bool pvx::has_light_chain(const pvx_scene *s) { return !s->use_kd && kernel_level(s->view) >= 2; }
 
-int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *depth, const uint32_t *owner, size_t n,
+int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *depth, size_t n,
                               uint32_t ray_kind, const MatRec *mats, float *col, uint32_t *more, hipStream_t st) {
     if (n == 0) return PVX_OK;
     int r;
@@ -689,7 +689,6 @@ int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *d
     ta.spill = spill;
     ta.chain_mats = mats;
     ta.chain_col = col;
-    ta.chain_owner = owner;
     ta.chain_more = more;
     HIP_TRY(trace_launch(TraceKernel{kernel_level(s->view) >= 3 ? kWalkChainRev : kWalkChain, s->view.any_flags != 0,
                                      false, false},

@@ -914,7 +914,7 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
             on = false;
             if (bo >= 0 && bt < depth - kShadowTolerance && bt > kShadowTolerance) {
                 const MatRec &m = a.chain_mats[bo];
-                float *c = a.chain_col + 3 * (size_t)a.chain_owner[ri];
+                float *c = a.chain_col + 3 * (size_t)ri;
                 if (m.opaque) {
                     c[0] = c[1] = c[2] = 0.0f;
                 } else {

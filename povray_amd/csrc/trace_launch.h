@@ -88,11 +88,10 @@ struct TraceArgs {
     uint8_t *gen_vis;
     uint32_t *gen_next; // kWalkLightDyn: next ray to hand out (zero at launch)
     const uint32_t *gen_count; // when set: n = gen_count[0] * gen_S, read on the device
-    // kWalkChain: ray k's colour is chain_col[3 * chain_owner[k]]; the number
-    // of continued rays is added to chain_more
+    // kWalkChain: ray k's colour is chain_col[3 * k]; the number of continued
+    // rays is added to chain_more
     const MatRec *chain_mats;
     float *chain_col;
-    const uint32_t *chain_owner;
     uint32_t *chain_more;
     uint32_t gen_refill_below; // kWalkLightDyn: refill once no more than this many lanes hold rays
 };

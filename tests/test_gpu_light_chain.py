@@ -1,0 +1,69 @@
+"""Light rays followed through glass in the walk, the bounces of a frame
+together: frames against the oracle's TraceRay, with area lights (several
+light rays a hit), supersampling (more hits wait), and many layers in a row;
+the light-ray count is the layer-by-layer one."""
+import numpy as np
+import pytest
+
+from oracle.oracle import OracleScene
+from povray_amd import _abi as A
+from povray_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _q(a):
+    return np.round(np.clip(a, 0.0, 1.0) * 255.0).astype(np.int32)
+
+
+def _close(img, ref):
+    # the parity bar of the shaded frames: 1/255 on 99.9 % of the pixels
+    assert np.mean(np.abs(_q(img) - _q(ref)).max(-1) <= 1) >= 0.999
+
+
+def _layers(n, lights):
+    """n glass boxes in a row between the light and a floor, a torus among
+    them (the walk of any primitive kind)."""
+    c1 = np.array([[-2.0, 0.5 + 0.1 * k, -2.0] for k in range(n)])
+    objects = [[A.PVX_BOX, k, 0, 0] for k in range(n)] + [[A.PVX_TORUS, 0, 0, 0], [A.PVX_PLANE, 0, 0, 0]]
+    m = len(objects)
+    glass = np.arange(m) < n
+    return scenes.Scene(
+        name=f"layers{n}", objects=np.array(objects, np.uint32), box_corner1=c1, box_corner2=c1 + [[4.0, 0.05, 4.0]],
+        box_transform=np.full(n, -1, np.int32), torus_major=np.array([1.0]), torus_minor=np.array([0.2]),
+        torus_transform=np.array([0], np.int32), torus_sturm=np.array([1], np.uint8),
+        transforms=np.array([scenes._xf_row(scenes.translation_transform([0.0, 0.25, 0.0]))]),
+        plane_normal=np.array([[0.0, 1.0, 0.0]]), plane_distance=np.array([0.0]),
+        camera=scenes.look_at_camera((0.0, 0.35, -6.0), (0.0, 0.2, 0.0), 96, 54), lights=lights,
+        materials=dict(pigment=np.full((m, 3), 0.9), diffuse=np.full(m, 0.6), ambient=np.full(m, 0.05),
+                       phong=np.zeros(m), phong_size=np.full(m, 40.0), reflection=np.zeros(m), ior=np.ones(m),
+                       transmit=np.where(glass, 0.8, 0.0), filter=np.where(glass, 0.15, 0.0)),
+        settings=dict(max_trace_level=6, adc_bailout=1.0 / 255.0))
+
+
+POINT = [dict(kind="point", position=np.array([0.5, 20.0, -0.3]), colour=np.ones(3))]
+AREA = [dict(kind="area", position=np.array([0.0, 12.0, 0.0]), axis1=np.array([2.0, 0.0, 0.0]),
+             axis2=np.array([0.0, 0.0, 2.0]), size=(3, 4), colour=np.ones(3))]
+
+
+@pytest.mark.parametrize("n,lights", [(1, POINT), (20, POINT), (40, POINT), (6, AREA), (3, POINT + AREA)])
+def test_layers(gpu, n, lights):
+    s = _layers(n, lights)
+    g = gpu.GpuScene(s)
+    g.set_shading()
+    img, st = g.render()
+    ref, rst = OracleScene(s).render(s)
+    _close(img, ref)
+    assert st["shadow_rays"] >= st["closest_rays"] // 4  # the layers' rays are counted
+    again, st2 = g.render()
+    assert np.array_equal(img, again) and st2["shadow_rays"] == st["shadow_rays"]
+
+
+def test_supersampled_glass_field(gpu):
+    s = scenes.csg_scene(n_objects=400, width=64, height=36)
+    offs = gpu.m1_offsets()
+    g = gpu.GpuScene(s)
+    g.set_shading()
+    img, _ = g.render_samples(offs)
+    ref, _ = OracleScene(s).render(s, offsets=offs)
+    _close(img, ref)
