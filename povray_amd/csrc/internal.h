@@ -110,6 +110,7 @@ struct RenderBuffers {
     // light stream and its events
     DevBuf contrib_b, shade_b, lslot_b, lterm_b, groups_b, refill;
     DevBuf gcount; // light groups of the bounces of each parity (two words)
+    HostBuf hcnt;  // a bounce's counts (pinned, written by its last scan)
     StreamHolder light_stream;
     EventPool events;
 };

@@ -76,8 +76,9 @@ __global__ void k_fill(float *p, size_t n, float v) {
 // counters: [0] light rays, [1] light-ray slots, [2] next queue size,
 // [3] lit (hit, light) groups whose light rays the traversal kernel makes
 constexpr uint32_t kGroupCounter = 3;
-__global__ void k_zero_counters(uint32_t *c) {
+__global__ void k_zero_counters(uint32_t *c, uint32_t *word) {
     if (threadIdx.x < 64) c[threadIdx.x] = 0;
+    if (word && threadIdx.x == 0) *word = 0;
 }
 
 __global__ void k_zero_word(uint32_t *c) {
@@ -664,8 +665,12 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_block(const uint32_t *__res
     if (t == kScanBlock - 1) sums[blockIdx.x] = s[t];
 }
 // ... scan of the block sums (one block, up to 1024 x 8 sums) ...
+// The bounce's counts go to `out`, host memory that the host reads once the
+// stream has come here (a copy of its own took as long as this kernel).
 __global__ __launch_bounds__(kScanBlock) void k_scan_sums(uint32_t *__restrict__ sums, uint32_t nb,
-                                                          uint32_t *__restrict__ total) {
+                                                          const uint32_t *__restrict__ counters,
+                                                          const uint32_t *__restrict__ gcount,
+                                                          uint32_t *__restrict__ out) {
     __shared__ uint32_t s[kScanBlock];
     const uint32_t t = threadIdx.x;
     constexpr int kPer = 8;
@@ -688,7 +693,12 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_sums(uint32_t *__restrict__
         uint32_t idx = t * kPer + k;
         if (idx < nb) sums[idx] = before + loc[k];
     }
-    if (t == kScanBlock - 1) *total = s[t];
+    if (t == kScanBlock - 1) {
+        out[0] = counters[0];
+        out[1] = counters[1];
+        out[2] = s[t];
+        out[kGroupCounter] = *gcount;
+    }
 }
 // ... then every child is copied to its place in the next queue.
 __global__ void k_emit(const uint32_t *__restrict__ nchild, const uint32_t *__restrict__ offs,
@@ -886,8 +896,9 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     // for the light pass of bounce j - 2 before reusing its buffers.
     const bool overlap = packet;
     if ((r = ensure_queue(nray)) || (r = b.offsets.reserve(16 * S)) || (r = b.counters.reserve(256)) ||
-        (r = b.refill.reserve(256)) || (r = b.gcount.reserve(256)))
+        (r = b.refill.reserve(256)) || (r = b.gcount.reserve(256)) || (r = b.hcnt.reserve(64)))
         return r;
+    uint32_t *hcnt = static_cast<uint32_t *>(b.hcnt.p);
     // Frames whose light rays are followed through transparent objects keep
     // the hits and light rays of several bounces and follow them in one launch
     // at the end (or when the buffers are full): a launch lasts as long as its
@@ -1129,8 +1140,7 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         }
         const size_t l0 = chain ? n_lights : 0;
         uint32_t *gcount = static_cast<uint32_t *>(b.gcount.p) + par;
-        k_zero_counters<<<1, 64, 0, st>>>(counters);
-        k_zero_word<<<1, 64, 0, st>>>(gcount);
+        k_zero_counters<<<1, 64, 0, st>>>(counters, gcount);
         const bool rev = s->view.has_complex >= 3; // lathes / sors in the scene
         (packet ? (rev ? k_shade<true, true> : k_shade<true, false>)
                 : (rev ? k_shade<false, true> : k_shade<false, false>))<<<(n + 127) / 128, 128, 0, st>>>(
@@ -1166,12 +1176,11 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         if (nb > (uint32_t)kScanBlock * 8) return fail(PVX_EUNSUPPORTED, "ray queue above 8M rays");
         k_scan_block<<<nb, kScanBlock, 0, st>>>(static_cast<const uint32_t *>(b.nchild.p), n,
                                                 static_cast<uint32_t *>(b.offs.p), static_cast<uint32_t *>(b.sums.p));
-        k_scan_sums<<<1, kScanBlock, 0, st>>>(static_cast<uint32_t *>(b.sums.p), nb, counters + 2);
+        k_scan_sums<<<1, kScanBlock, 0, st>>>(static_cast<uint32_t *>(b.sums.p), nb, counters, gcount, hcnt);
         HIP_TRY(hipGetLastError());
-        uint32_t cnt[kGroupCounter + 1];
-        HIP_TRY(hipMemcpyAsync(cnt, counters, sizeof cnt, hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipMemcpyAsync(&cnt[kGroupCounter], gcount, 4, hipMemcpyDeviceToHost, st)); // light groups
         HIP_TRY(hipStreamSynchronize(st));
+        uint32_t cnt[kGroupCounter + 1];
+        for (uint32_t k = 0; k <= kGroupCounter; k++) cnt[k] = static_cast<volatile uint32_t *>(hcnt)[k];
         float ms = 0.0f;
         HIP_TRY(hipEventElapsedTime(&ms, t0, t1));
         trace_ms += ms;
@@ -1251,7 +1260,7 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
             if (rc) return rc;
             HIP_TRY(hipEventRecord(t1, st));
             n_shadow += ns;
-            k_zero_counters<<<1, 64, 0, st>>>(counters);
+            k_zero_counters<<<1, 64, 0, st>>>(counters, nullptr);
             k_shadow_step<<<(ns + 255) / 256, 256, 0, st>>>(
                 p, static_cast<const pvx_ray *>(b.srays[sq].p), static_cast<const double *>(b.sdepth[sq].p),
                 static_cast<const uint32_t *>(b.sowner[sq].p), static_cast<const pvx_hit *>(b.shits.p), ns,
