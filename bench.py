@@ -570,7 +570,8 @@ def main():
     stream.synchronize()
     node_visits = nv.download(np.uint32, n).astype(np.float64)
     prim_tests = pt.download(np.uint32, n).astype(np.float64)
-    bytes_node = 64.0 if tune["variant"] == A.PVX_TRAVERSAL_BINARY else float(st["node_bytes"])
+    wide = (A.PVX_TRAVERSAL_WIDE_WW, A.PVX_TRAVERSAL_WIDE_STEP)  # 128-byte nodes; the others walk the binary tree
+    bytes_node = 128.0 if tune["variant"] in wide else float(st["node_bytes"])
     bytes_prim = float(st["tri_bytes"])
     bytes_ray = 48.0 + 16.0 + bytes_node * node_visits.mean() + bytes_prim * prim_tests.mean()
     log(f"per ray: {node_visits.mean():.1f} node visits ({bytes_node:.0f} B), {prim_tests.mean():.1f} prim tests "

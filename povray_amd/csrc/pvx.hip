@@ -419,13 +419,13 @@ extern "C" int pvx_scene_destroy(pvx_scene *s) {
 
 extern "C" int pvx_scene_get_stats(const pvx_scene *s, pvx_scene_stats *out) {
     if (!s || !out) return fail(PVX_EINVAL, "null argument");
-    const bool wide = s->view.wide != 0; // the tree the closest-hit kernels walk
-    out->n_nodes = s->use_kd ? s->host.kd_nodes.size() : wide ? s->n_nodes4 : s->n_nodes2;
+    // the tree the default walks take
+    out->n_nodes = s->use_kd ? s->host.kd_nodes.size() : s->n_nodes2;
     out->n_prims = s->use_kd ? s->host.kd_list.size() : s->n_prims;
-    out->node_bytes = s->use_kd ? sizeof(KdNode) : wide ? sizeof(Node4) : sizeof(Node);
+    out->node_bytes = s->use_kd ? sizeof(KdNode) : sizeof(Node);
     out->tri_bytes = sizeof(PrimRec);
     out->device_bytes = s->device_bytes;
-    out->bvh_depth = s->use_kd ? s->host.kd_depth : wide ? s->host.depth4 : s->host.depth;
+    out->bvh_depth = s->use_kd ? s->host.kd_depth : s->host.depth;
     out->n_infinite = (uint32_t)s->host.inf.size();
     out->build_ms = s->host.build_ms;
     out->bvh_build_ms = s->host.bvh_ms;
@@ -867,7 +867,10 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     if (!rays || !hits) return fail(PVX_EINVAL, "null ray or hit buffer");
     const uint32_t n = b->n_chunks * 64u;
     const bool flags = b->any_flags != 0 && ray_kind != PVX_RAY_PRIMARY;
-    const uint32_t nblocks = std::min<uint32_t>(b->whole ? kWholeGrid : b->grid, (n + kBlock - 1) / kBlock);
+    // with per-scene clocks the persistent grid: every wavefront's start is an
+    // atomic on one word (64 scenes, 45 M rays, one wavefront per chunk: 9.4 ms
+    // instead of 7.1 ms in 64 launches)
+    const uint32_t nblocks = std::min<uint32_t>(b->whole && !clk ? kWholeGrid : b->grid, (n + kBlock - 1) / kBlock);
     const SceneView *views = static_cast<const SceneView *>(b->views.p);
     const uint4 *chunks = static_cast<const uint4 *>(b->chunks.p);
     int32_t *spill = static_cast<int32_t *>(b->spill.p);
