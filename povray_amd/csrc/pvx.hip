@@ -432,27 +432,10 @@ extern "C" int pvx_scene_get_stats(const pvx_scene *s, pvx_scene_stats *out) {
     return PVX_OK;
 }
 
-// A walk whose stack cannot outgrow its LDS entries needs no spill area per
-// resident lane, so its launch covers all rays (kWholeGrid) instead of a
-// persistent grid: the hardware then hands out wavefronts as others end.  A
-// persistent grid with a fixed stride left less than half of its places
-// filled (camera rays of the 1.3M-triangle icosphere: 2.3 of 5 wavefronts per
-// SIMD on average).
-constexpr uint32_t kWholeGrid = 0x7FFFFFFFu;
+// Whether the walk may launch over all rays (kWholeGrid).
 static bool stack_in_lds(const HostScene &h, bool wide) {
     // a binary node pushes at most one link, a wide one three
     return (wide ? 3 * (h.depth4 + 1) : h.depth + 1) <= (uint32_t)kStackLds;
-}
-
-// Rays per wavefront of a launch of n rays on a grid of `grid` blocks: 64,
-// halved while the grid still holds every wavefront at once.  A wavefront
-// runs every path that any of its rays takes, so below a full grid fewer rays
-// each end sooner (plain radiosity of the 5,000-box room, whose rounds gather
-// some ten thousand rays: 53 ms with 64 rays per wavefront, 45 ms so).
-static uint32_t rays_per_wave(size_t n, uint32_t grid) {
-    uint32_t r = 64;
-    while (r > 1 && n <= (size_t)grid * (kBlock / 64) * (r / 2)) r /= 2;
-    return r;
 }
 
 // One closest-hit launch with an explicit traversal variant and grid.
@@ -470,7 +453,7 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
     if (!s->use_kd && stack_in_lds(s->host, wide)) grid = kWholeGrid;
     const bool few = !s->use_kd && !wide && variant != PVX_TRAVERSAL_BINARY_WW;
     const uint32_t wave_rays = few ? rays_per_wave(n, s->grid) : 64u;
-    uint32_t nblocks = (uint32_t)std::min<size_t>(grid, (n + 4 * wave_rays - 1) / (4 * wave_rays));
+    const uint32_t nblocks = launch_units(n, wave_rays, grid);
     const bool flags = s->view.any_flags != 0 && (ray_kind != PVX_RAY_PRIMARY || kinds);
     TraceKernel k{kWalkStep4, flags, kCount, false};
     if (s->use_kd)
@@ -642,7 +625,7 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     // to fill; the binary walk over all rays when its stack fits in LDS
     uint32_t grid = grid_blocks ? grid_blocks : next ? s->grid : 2 * s->grid;
     if (!next && binary && stack_in_lds(s->host, false)) grid = kWholeGrid;
-    const uint32_t nb = (uint32_t)std::min<size_t>(grid, ((size_t)n_rays + kBlock - 1) / kBlock);
+    const uint32_t nb = launch_units(n_rays, 64, grid);
     TraceArgs ta{};
     ta.wave_rays = 64;
     ta.sv = s->view;
@@ -680,7 +663,7 @@ int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *d
     // the resident grid: a lane whose ray has ended takes another while the
     // others follow theirs through further layers
     ta.wave_rays = rays_per_wave(n, s->grid);
-    const uint32_t nb = (uint32_t)std::min<size_t>(s->grid, (n + 4 * ta.wave_rays - 1) / (4 * ta.wave_rays));
+    const uint32_t nb = launch_units(n, ta.wave_rays, s->grid);
     ta.sv = s->view;
     ta.rays = rays;
     ta.max_depth = depth;
@@ -870,7 +853,7 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     // with per-scene clocks the persistent grid: every wavefront's start is an
     // atomic on one word (64 scenes, 45 M rays, one wavefront per chunk: 9.4 ms
     // instead of 7.1 ms in 64 launches)
-    const uint32_t nblocks = std::min<uint32_t>(b->whole && !clk ? kWholeGrid : b->grid, (n + kBlock - 1) / kBlock);
+    const uint32_t nblocks = launch_units(n, 64, b->whole && !clk ? kWholeGrid : b->grid);
     const SceneView *views = static_cast<const SceneView *>(b->views.p);
     const uint4 *chunks = static_cast<const uint4 *>(b->chunks.p);
     int32_t *spill = static_cast<int32_t *>(b->spill.p);

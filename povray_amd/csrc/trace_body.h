@@ -35,17 +35,7 @@ __device__ inline float safe_inv(double d) {
 // one; until every lane is at a leaf (while-while): 1071 us.
 constexpr int kNodeSteps = 4;
 
-// Blocks go to the eight XCDs in turn, each with an L2 of its own: the place
-// of this block's rays such that sixteen neighbouring wavefronts (of rays
-// that mostly walk the same nodes) share one (camera rays of the
-// 1.3M-triangle icosphere 568 -> 556 us, its reflections at 327,680 triangles
-// 253 -> 242 us; 4 or 64 neighbours: 571 and 560, 245 and 241 us).  Blocks past
-// the last whole group keep their place.
-__device__ __forceinline__ uint32_t xcd_block() {
-    constexpr uint32_t kXcds = 8, kRun = 16;
-    const uint32_t b = blockIdx.x, whole = gridDim.x / (kXcds * kRun) * (kXcds * kRun);
-    return b < whole ? (b / (kXcds * kRun) * kXcds + b % kXcds) * kRun + b / kXcds % kRun : b;
-}
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_place(blockIdx.x, gridDim.x); }
 
 // Slab test of one referenced primitive's own box, as the nodes test theirs:
 // a leaf's primitives share a node box, and the FP64 tests behind this one
@@ -254,7 +244,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
     if (part && lane >= wave_rays) return;
     const uint32_t i0 = xcd_block() * (part ? wave_rays : (uint32_t)kWaveBlock) + lane;
     const uint32_t istep = gridDim.x * (part ? wave_rays : (uint32_t)kWaveBlock);
-    for (uint32_t i = i0; i < n; i += istep) {
+    for (uint32_t i = i0; i < n; i = next_ray(i, istep, n)) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
             const uint4 ch = chunks[__builtin_amdgcn_readfirstlane(i >> 6)];
@@ -684,7 +674,8 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
     uint32_t layers = 0;     // kChain: blockers passed so far
     bool on = false;         // kChain: the ray goes on behind a blocker
     uint32_t more = 0;       // kChain: continued rays
-    for (uint32_t i = kChain && wl >= per_wave ? n : (kMulti ? blockIdx.x : xcd_block()) * per_wave + wl; i < n; i += kChain && on ? 0u : step) {
+    for (uint32_t i = kChain && wl >= per_wave ? n : (kMulti ? blockIdx.x : xcd_block()) * per_wave + wl; i < n;
+         i = kChain && on ? i : next_ray(i, step, n)) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
             const uint4 ch = a.chunks[__builtin_amdgcn_readfirstlane(i >> 6)];
@@ -939,7 +930,8 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
         if constexpr (kMulti) {
             if (a.clocks && wl == 0) atomicMax(&a.clocks[1 + scene], (unsigned long long)wall_clock64());
         }
-    }    if constexpr (kChain) {
+    }
+    if constexpr (kChain) {
         for (int off = 32; off > 0; off >>= 1) more += __shfl_xor(more, off, 64);
         if (wl == 0 && more) atomicAdd(a.chain_more, more);
     }

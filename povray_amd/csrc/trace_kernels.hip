@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest_kd(TraceArgs a) {
     };
     kind &= 0xFFu; // closest hits only (the occlusion bit is a hint)
     const bool shadow = (kind == PVX_RAY_SHADOW);
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i = next_ray(i, gridDim.x * kBlock, n)) {
         const pvx_ray r = rays[i];
         const uint32_t rk = (kFlags && kinds) ? (uint32_t)kinds[i] : kind;
         const D3 o = d3(r.o[0], r.o[1], r.o[2]), d = d3(r.d[0], r.d[1], r.d[2]);

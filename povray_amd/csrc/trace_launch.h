@@ -12,13 +12,10 @@
 
 #include "../../include/pvx.h"
 #include "pvx_types.h"
+#include "ray_grid.h"
 
 namespace pvx {
 
-constexpr int kBlock = 256;      // lanes per unit of a traversal grid (threads per block of the kd walk)
-// Threads per block of the BVH walks: one wavefront, so that its place is
-// free for the next one as soon as it ends (a kBlock unit is four of them).
-constexpr int kWaveBlock = 64;
 constexpr int kStackLds = 25;    // traversal-stack entries per lane in LDS (see below)
 constexpr int kStackSpill = 39;  // further entries per lane in the spill area
 constexpr int kStackMax = kStackLds + kStackSpill;
