@@ -449,7 +449,11 @@ __global__ void k_fill_zero(uint32_t *p, size_t n) {
 // release writes the XCD's L2 back and an acquire drops it, and one of each
 // per wavefront and poll had the waiting blocks empty each other's L2 all
 // along.  Waiting on the arrivals themselves saves the hop through a last
-// arriver.
+// arriver.  The wait behind the release is written out: the write-back counts
+// as a memory operation in flight, but the compiler, which sees none since the
+// wait before the barrier, leaves out the fence's own wait, and the arrival
+// then overtakes the data (with other streams at work, weights that differed
+// from run to run).
 struct GridBar {
     unsigned count, err, pad[2];
 };
@@ -460,6 +464,7 @@ __device__ inline bool grid_sync(GridBar *b, unsigned target) {
     __syncthreads();
     if (threadIdx.x == 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __builtin_amdgcn_s_waitcnt(0);
         __hip_atomic_fetch_add(&b->count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         uint32_t spins = 0;
         while ((int32_t)(__hip_atomic_load(&b->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {

@@ -48,6 +48,20 @@ def test_batch_frames_equal_per_scene_frames(gpu, mode):
         assert bst["fallbacks"] <= bst["final_misses"]
 
 
+@pytest.mark.parametrize("n_streams", [2, 3])
+def test_learned_batches_repeat(gpu, n_streams):
+    # one network trains while other streams work: the same weights, hence the
+    # same images, every time
+    gs = [_gpu(gpu, s) for s in _scenes()]
+    batch = gpu.GpuBatch(gs)
+    first, sst, _, _ = batch.radiosity_render(mode=A.PVX_RADIOSITY_LEARNED, n_streams=n_streams)
+    for _ in range(12):
+        imgs, st, _, _ = batch.radiosity_render(mode=A.PVX_RADIOSITY_LEARNED, n_streams=n_streams)
+        assert [x["train_loss"] for x in st] == [x["train_loss"] for x in sst]
+        for a, b in zip(imgs, first):
+            assert np.array_equal(a, b)
+
+
 def test_batch_scene_plain_frame_vs_oracle(gpu):
     s = _scenes()[0]
     over = dict(count=50)
