@@ -328,6 +328,7 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
     UP(h.csg_children, csg_children);
     UP(h.csg_slots, csg_slots);
     UP(h.csg_tests, csg_tests);
+    UP(h.csg_start, csg_start);
     UP(h.placed, placed);
     UP(h.csg_leaves, csg_leaves);
     UP(h.csg_leaf_range, csg_leaf_range);

@@ -283,8 +283,9 @@ struct CsgTest {
 // A CSG operand: the filter program of its node (`start`; the operand's own
 // tests [skip, skip_to) are left out), the operand that stands for that node
 // in the next enclosing intersection or merge (`up`, -1 at the root), and the
-// operand's own shape.  Programs are per node, so their total size is linear
-// in the tree.
+// operand's own shape.  Every node has a program of its own, also a union (it
+// filters nothing, but Inside runs it), so an operand's test stands in the
+// program of each node above it: at most eight, the nesting limit.
 struct CsgSlot {
     uint32_t start, skip, skip_to;
     int32_t up;
@@ -365,6 +366,7 @@ struct SceneView {
     const CsgChild *csg_children;
     const CsgSlot *csg_slots;        // per csg_children slot
     const CsgTest *csg_tests;        // the filter programs
+    const uint32_t *csg_start;       // per CSG node: where its program starts
     const PlacedRec *placed;         // boxes and tori with their placement
     const uint32_t *csg_leaves;      // leaf slots of each CSG root, contiguous
     const uint32_t *csg_leaf_range;  // 2 per CSG node: [begin, end) into csg_leaves

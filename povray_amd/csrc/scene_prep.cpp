@@ -954,6 +954,7 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
     out.csg.resize(d.n_csg);
     out.csg_children.resize(d.n_csg_children);
     std::vector<int32_t> owner_slot(d.n_csg, -1);
+    std::vector<uint8_t> shared(d.n_csg_children, 0); // 2: in the child ranges of several nodes (leaves only)
     for (uint32_t i = 0; i < d.n_csg; i++) {
         const pvx_csg_node &n = d.csg[i];
         if (n.op < PVX_CSG_UNION || n.op > PVX_CSG_MERGE) {
@@ -975,6 +976,7 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
                 return PVX_EUNSUPPORTED;
             }
             out.csg_children[slot] = CsgChild{c.type, c.index, c.flags, i};
+            shared[slot] = (uint8_t)std::min(2, shared[slot] + 1);
             if (c.type == PVX_CSG) {
                 if (owner_slot[c.index] >= 0) {
                     err = "CSG node shared by two parents";
@@ -997,8 +999,11 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         }
         return m;
     };
+    // nodes in a cycle have no root above them: nothing may follow them
+    std::vector<bool> reached(d.n_csg, false);
     std::function<void(uint32_t)> collect = [&](uint32_t node) {
         const CsgNode &n = out.csg[node];
+        reached[node] = true;
         for (uint32_t k = 0; k < n.count; k++) {
             const CsgChild &c = out.csg_children[n.first + k];
             if (c.type == PVX_CSG)
@@ -1051,33 +1056,36 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
     // --- CSG filter programs (CsgTest) ----------------------------------------
     // A node's program is written back to front: `emit` puts the tests of one
     // operand before those already there and returns where they start, given
-    // where to go when p is inside it and when it is not.
+    // where to go when p is inside it and when it is not.  Programs follow the
+    // operands downward only, so they are right also where two nodes' child
+    // ranges share a leaf.
     out.csg_slots.resize(d.n_csg_children);
-    std::vector<uint32_t> node_start(d.n_csg, kCsgUp);
+    out.csg_start.assign(d.n_csg, kCsgUp);
+    std::vector<CsgTest> rev;  // reversed; entry k of m is at base + m - 1 - k
+    std::vector<uint32_t> seg; // where each operand's tests start
+    auto emit = [&](auto &&self, uint32_t slot, uint32_t in, uint32_t no) -> uint32_t {
+        const CsgChild &c = out.csg_children[slot];
+        if (c.type == PVX_CSG) {
+            const CsgNode &m = out.csg[c.index];
+            const bool all = m.op == PVX_CSG_INTERSECTION; // intersection: every operand; union, merge: any
+            uint32_t at = all ? in : no;                   // after the last operand
+            for (uint32_t k = m.count; k-- > 0;)
+                at = all ? self(self, m.first + k, at, no) : self(self, m.first + k, in, at);
+            return at;
+        }
+        const auto pr = placed(c.type, c.index);
+        rev.push_back(CsgTest{c.type | ((c.flags & PVX_FLAG_INVERTED) ? 1u << 8 : 0u) | pr.second << 16,
+                              pr.first != kNoRec ? pr.first : c.index, in, no});
+        return (uint32_t)rev.size() - 1;
+    };
     for (uint32_t i = 0; i < d.n_csg; i++) {
         const CsgNode &n = out.csg[i];
-        if (n.op == PVX_CSG_UNION) continue;
-        std::vector<CsgTest> rev; // reversed; entry k of m is at base + m - 1 - k
-        // labels below kCsgDrop count entries of `rev` from its end of program
-        std::function<uint32_t(uint32_t, uint32_t, uint32_t)> emit = [&](uint32_t slot, uint32_t in,
-                                                                          uint32_t no) -> uint32_t {
-            const CsgChild &c = out.csg_children[slot];
-            if (c.type == PVX_CSG) {
-                const CsgNode &m = out.csg[c.index];
-                const bool all = m.op == PVX_CSG_INTERSECTION; // intersection: every operand; union, merge: any
-                uint32_t at = all ? in : no;                   // after the last operand
-                for (uint32_t k = m.count; k-- > 0;) at = all ? emit(m.first + k, at, no) : emit(m.first + k, in, at);
-                return at;
-            }
-            const auto pr = placed(c.type, c.index);
-            rev.push_back(CsgTest{c.type | ((c.flags & PVX_FLAG_INVERTED) ? 1u << 8 : 0u) | pr.second << 16,
-                                  pr.first != kNoRec ? pr.first : c.index, in, no});
-            return (uint32_t)rev.size() - 1;
-        };
+        if (!reached[i]) continue;
+        rev.clear(); // labels below kCsgDrop count its entries from the end of the program
+        seg.assign(n.count + 1, kCsgUp);
         uint32_t at = kCsgUp;
-        std::vector<uint32_t> seg(n.count + 1, kCsgUp); // where each operand's tests start
         for (uint32_t k = n.count; k-- > 0;) {
-            at = n.op == PVX_CSG_MERGE ? emit(n.first + k, kCsgDrop, at) : emit(n.first + k, at, kCsgDrop);
+            at = n.op == PVX_CSG_INTERSECTION ? emit(emit, n.first + k, at, kCsgDrop) : emit(emit, n.first + k, kCsgDrop, at);
             seg[k] = at;
         }
         const uint32_t base = (uint32_t)out.csg_tests.size(), m = (uint32_t)rev.size();
@@ -1088,28 +1096,23 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
             t.next_out = label(t.next_out);
             out.csg_tests.push_back(t);
         }
-        node_start[i] = label(at);
-        for (uint32_t k = 0; k < n.count; k++) {
-            out.csg_slots[n.first + k].skip = label(seg[k]);
-            out.csg_slots[n.first + k].skip_to = label(seg[k + 1]);
-        }
-    }
-    for (uint32_t i = 0; i < d.n_csg; i++) {
-        const CsgNode &n = out.csg[i];
+        out.csg_start[i] = label(at);
+        const bool filters = n.op != PVX_CSG_UNION;
         int32_t up = n.parent_slot; // past the unions, which filter nothing
         while (up >= 0 && out.csg[out.csg_children[up].node].op == PVX_CSG_UNION)
             up = out.csg[out.csg_children[up].node].parent_slot;
         for (uint32_t k = 0; k < n.count; k++) {
             CsgSlot &s = out.csg_slots[n.first + k];
             const CsgChild &c = out.csg_children[n.first + k];
-            s.start = node_start[i];
-            if (n.op == PVX_CSG_UNION) s.skip = s.skip_to = kCsgUp;
-            s.up = up;
-            s.type = c.type;
-            s.shape = c.index;
             const auto pr = placed(c.type, c.index);
-            s.rec = pr.first;
-            s.rflags = pr.second;
+            s = CsgSlot{filters ? out.csg_start[i] : kCsgUp,
+                        filters ? label(seg[k]) : kCsgUp,
+                        filters ? label(seg[k + 1]) : kCsgUp,
+                        up,
+                        c.type,
+                        c.index,
+                        pr.first,
+                        pr.second};
         }
     }
 
@@ -1207,7 +1210,8 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
     // only the leaves whose box it crosses, nearest first, instead of every
     // leaf of every object it passes.  Objects with other leaves stay whole
     // (a disc's box does not bound its half-space, planes and quadrics are
-    // unbounded, lathes and sors depend on being CSG operands).  The boxes
+    // unbounded, lathes and sors depend on being CSG operands), and so do
+    // those whose child ranges overlap another's.  The boxes
     // are widened by 1e-4 of their size: a leaf's computed hit may lie off
     // its surface by the root finder's error (below 1e-6 of the size).
     struct CsgPart {
@@ -1219,6 +1223,7 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         const CsgNode &n = out.csg[node];
         for (uint32_t k = 0; k < n.count; k++) {
             const CsgChild &c = out.csg_children[n.first + k];
+            if (shared[n.first + k] > 1) return false; // its filters are not this node's alone
             DBox b = clip;
             if (n.op == PVX_CSG_INTERSECTION)
                 for (uint32_t j = 0; j < n.count; j++) {

@@ -43,6 +43,7 @@ struct HostScene {
     std::vector<CsgChild> csg_children;
     std::vector<CsgSlot> csg_slots;
     std::vector<CsgTest> csg_tests;
+    std::vector<uint32_t> csg_start;
     std::vector<PlacedRec> placed;
     std::vector<uint32_t> csg_leaves;
     std::vector<uint32_t> csg_leaf_range;

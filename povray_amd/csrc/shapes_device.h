@@ -11,7 +11,6 @@
 
 namespace pvx {
 
-constexpr int kCsgMaxDepth = 8;     // nesting limit of CSG trees on the device
 constexpr int kMaxLeafHits = 4;     // hits one leaf shape can push (torus: 4)
 
 struct D3 {
@@ -854,53 +853,32 @@ __device__ inline bool leaf_inside(const SceneView &sv, uint32_t type, uint32_t 
     }
 }
 
-// Is p inside the operand in csg_children slot `slot` (CSGIntersection::Inside
-// and CSGUnion::Inside, csg.cpp:405-454)?  The operand's subtree is walked
-// through the nodes' parent links with one operand test in the loop body: a
-// recursion over the nesting levels gave every level its own inlined copy of
-// all shape tests (240 registers, and lanes at different levels ran them one
-// after the other).
-template <bool kRev = false>
-__device__ inline bool csg_slot_inside(const SceneView &sv, uint32_t slot, D3 p) {
-    uint32_t cur = slot;
-    for (;;) {
-        const CsgChild c = sv.csg_children[cur];
-        bool in;
-        if (c.type == PVX_CSG) {
-            const CsgNode &n = sv.csg[c.index];
-            if (n.count > 0) {
-                cur = n.first;
-                continue;
-            }
-            in = n.op == 2; // no operands: an intersection holds everything
-        } else {
-            in = leaf_inside<kRev>(sv, c.type, c.index, c.flags, p);
-        }
-        // the result of `cur`: on to its next sibling, or up
-        for (;;) {
-            if (cur == slot) return in;
-            const uint32_t node = sv.csg_children[cur].node;
-            const CsgNode &n = sv.csg[node];
-            const bool last = cur + 1 == n.first + n.count;
-            // an intersection ends at the first operand outside, a union or
-            // merge at the first inside
-            if ((n.op == 2) == in && !last) {
-                cur++;
-                break;
-            }
-            cur = (uint32_t)n.parent_slot; // its result is `in`
-        }
+// One test of a CSG filter program (CsgTest): is p inside its operand?
+template <bool kRev>
+__device__ inline bool csg_test(const SceneView &sv, const CsgTest &t, D3 p) {
+    const uint32_t type = t.what & 0xFFu;
+    const bool inv = (t.what >> 8) & 1u;
+    if (type == PVX_BOX || type == PVX_TORUS) {
+        const PlacedRec &r = sv.placed[t.index];
+        const D3 q = ((t.what >> 16) & kPlacedXf) ? pl_point(r.inv, p) : p;
+        return type == PVX_BOX ? box_inside_at(r.q, r.q + 3, q, inv) : torus_inside_at(r.q[0], r.q[1], q, inv);
     }
+    return leaf_inside<kRev>(sv, type, t.index, inv ? (uint32_t)PVX_FLAG_INVERTED : 0u, p);
 }
 
-// Inside test of a whole object (CSG node `index` or a single shape).
+// Inside test of a whole object (CSG node `index` or a single shape;
+// CSGIntersection::Inside and CSGUnion::Inside, csg.cpp:405-454).  A node's
+// program ends at kCsgUp when p is inside every operand of an intersection,
+// or inside none of a union's or merge's.
 template <bool kRev = false>
 __device__ inline bool shape_inside(const SceneView &sv, uint32_t type, uint32_t index, uint32_t flags, D3 p) {
     if (type != PVX_CSG) return leaf_inside<kRev>(sv, type, index, flags, p);
-    const CsgNode &n = sv.csg[index];
-    for (uint32_t k = 0; k < n.count; k++)
-        if (csg_slot_inside<kRev>(sv, n.first + k, p) != (n.op == 2)) return n.op != 2;
-    return n.op == 2;
+    uint32_t pc = sv.csg_start[index];
+    while (pc < kCsgDrop) {
+        const CsgTest t = sv.csg_tests[pc];
+        pc = csg_test<kRev>(sv, t, p) ? t.next_in : t.next_out;
+    }
+    return (pc == kCsgUp) == (sv.csg[index].op == PVX_CSG_INTERSECTION);
 }
 
 // Hits of one leaf shape other than a sphere, box or torus in
@@ -1006,17 +984,7 @@ __device__ inline bool csg_survives(const SceneView &sv, uint32_t slot, D3 ip) {
             if (pc == kCsgUp) break;
             if (pc == kCsgDrop) return false;
             const CsgTest t = sv.csg_tests[pc];
-            const uint32_t type = t.what & 0xFFu;
-            const bool inv = (t.what >> 8) & 1u;
-            bool in;
-            if (type == PVX_BOX || type == PVX_TORUS) {
-                const PlacedRec &r = sv.placed[t.index];
-                const D3 q = ((t.what >> 16) & kPlacedXf) ? pl_point(r.inv, ip) : ip;
-                in = type == PVX_BOX ? box_inside_at(r.q, r.q + 3, q, inv) : torus_inside_at(r.q[0], r.q[1], q, inv);
-            } else {
-                in = leaf_inside<kRev>(sv, type, t.index, inv ? (uint32_t)PVX_FLAG_INVERTED : 0u, ip);
-            }
-            pc = in ? t.next_in : t.next_out;
+            pc = csg_test<kRev>(sv, t, ip) ? t.next_in : t.next_out;
         }
     } while (cur >= 0);
     return true;

@@ -129,3 +129,29 @@ def test_few_rays_equal_many(gpu, make):
     full = g.find_intersection(rays)
     for n in (1, 2, 63, 64, 65, 1023, 4097, 32769, 131073):
         _same(g.find_intersection(rays[:n]), full[:n])
+
+
+def test_child_ranges_that_overlap(gpu):
+    # nodes whose child ranges share leaves: Inside goes by each node's own operands
+    r = np.random.default_rng(9)
+    n = 14
+    centre, kids = r.uniform(-1.0, 1.0, (n, 3)), []
+    for k in range(n):
+        kids.append([A.PVX_SPHERE if k % 3 else A.PVX_BOX, k, A.PVX_FLAG_INVERTED if k % 5 == 4 else 0, 0])
+    ops = [A.PVX_CSG_UNION, A.PVX_CSG_INTERSECTION, A.PVX_CSG_MERGE]
+    nodes = [[ops[i % 3], int(a), int(c), 0]
+             for i, (a, c) in enumerate(zip(r.integers(0, n - 4, 12), r.integers(2, 5, 12)))]
+    for i, op in enumerate(ops):  # two nodes below each
+        kids += [[A.PVX_CSG, 2 * i, 0, 0], [A.PVX_CSG, 2 * i + 1, 0, 0]]
+        nodes.append([op, len(kids) - 2, 2, 0])
+    roots = [i for i in range(len(nodes)) if i >= 6]
+    s = scenes.Scene(
+        name="overlap", objects=np.array([[A.PVX_CSG, i, 0, 0] for i in roots], np.uint32),
+        sphere_center=centre, sphere_radius=r.uniform(0.5, 1.2, n), box_corner1=centre - 0.6,
+        box_corner2=centre + 0.6, box_transform=np.full(n, -1, np.int32), csg=np.array(nodes, np.uint32),
+        csg_children=np.array(kids, np.uint32), camera=scenes.look_at_camera((0.0, 0.5, -6.0), (0.0, 0.0, 0.0), 97, 71))
+    g, orc = gpu.GpuScene(s), OracleScene(s)
+    pts = r.uniform(-2.0, 2.0, (20000, 3))
+    for ob in range(len(roots)):
+        which = np.full(pts.shape[0], ob, np.uint32)
+        assert np.array_equal(g.inside(pts, which), orc.inside(pts, which)), nodes[roots[ob]]
