@@ -905,7 +905,9 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     // slowest rays, whatever their number.  The finished hits are accumulated
     // bounce by bounce as before, so the image is the same.  The 5,000-leaf
     // glass frame (641 x 359, 19 bounces): 51 ms with a launch per bounce, 22 ms
-    // with one for every four frames' worth of rays, 21.7 ms for sixteen.
+    // with one for every four frames' worth of rays, 21.7 ms for sixteen, so
+    // four wait, and no more than kWaitBytes beyond the first (every light
+    // adds to what a hit keeps).
     const bool chain = !packet && has_light_chain(s);
     size_t hit_cap = 0, light_cap = 0; // hits and light rays that may wait
     auto ensure_chain = [&](size_t hits, size_t lights) -> int {
@@ -921,8 +923,21 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         return PVX_OK;
     };
     if (chain) {
-        const size_t hits = std::max(nray, std::min<size_t>(16 * nray, (size_t)4 << 20));
-        if ((r = ensure_chain(hits, std::max(nray * spp, std::min(hits * spp, (size_t)16 << 20))))) return r;
+        constexpr size_t kWaitBytes = (size_t)256 << 20;
+        const size_t per_hit = 12 + sizeof(ShadeOut) + 4 + 20 * nl + spp * (sizeof(pvx_ray) + 8 + 4 + 12);
+        const size_t hits = nray + std::min(3 * nray, kWaitBytes / per_hit);
+        if ((r = ensure_chain(hits, hits * spp))) {
+            // no room: give back what was reserved, one frame's worth then
+            // takes less than light rays followed a layer a launch
+            (void)hipGetLastError();
+            for (DevBuf *d : {&b.contrib, &b.shade, &b.lslot, &b.lterm, &b.pix[0], &b.srays[0], &b.sdepth[0],
+                              &b.sowner[0], &b.scol}) {
+                DevBuf gone;
+                std::swap(gone.p, d->p);
+                std::swap(gone.cap, d->cap);
+            }
+            if ((r = ensure_queue(nray)) || (r = ensure_chain(nray, nray * spp))) return r;
+        }
     } else if ((r = packet ? ensure_packet(nray) : ensure_shadow(nray * spp))) {
         return r;
     }

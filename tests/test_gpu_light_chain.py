@@ -2,12 +2,14 @@
 together: frames against the oracle's TraceRay, with area lights (several
 light rays a hit), supersampling (more hits wait), and many layers in a row;
 the light-ray count is the layer-by-layer one."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle.oracle import OracleScene
 from povray_amd import _abi as A
-from povray_amd import scenes
+from povray_amd import hip, scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +69,22 @@ def test_supersampled_glass_field(gpu):
     img, _ = g.render_samples(offs)
     ref, _ = OracleScene(s).render(s, offsets=offs)
     _close(img, ref)
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    hip.check(hip._lib().hipMemGetInfo(C.byref(free), C.byref(total)), "hipMemGetInfo")
+    return free.value
+
+
+def test_waiting_light_rays_are_bounded(gpu):
+    # 64 lights: a hit keeps 1.3 KB and its light rays 4.6 KB.  One frame's
+    # worth is 85 MB, and the hits that wait beyond it at most 256 MB.
+    lights = [dict(kind="point", position=np.array([0.5 * k, 20.0, -0.3]), colour=np.full(3, 1.0 / 64)) for k in range(64)]
+    s = _layers(3, lights)
+    g = gpu.GpuScene(s)
+    g.set_shading()
+    g.render(32, 18)  # the scene's fixed buffers
+    free = _free_bytes()
+    g.render(160, 90)
+    assert free - _free_bytes() < (256 + 85 + 100) << 20
