@@ -905,9 +905,10 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     // slowest rays, whatever their number.  The finished hits are accumulated
     // bounce by bounce as before, so the image is the same.  The 5,000-leaf
     // glass frame (641 x 359, 19 bounces): 51 ms with a launch per bounce, 22 ms
-    // with one for every four frames' worth of rays, 21.7 ms for sixteen, so
-    // four wait, and no more than kWaitBytes beyond the first (every light
-    // adds to what a hit keeps).
+    // with one for every four frames' worth of rays, 21.7 ms for sixteen; the
+    // 10,000-leaf one at 320 x 180, of 4.8 frames' worth, 17.7 and 15.0 ms.  So
+    // up to sixteen wait, but no more than kWaitBytes beyond the first (every
+    // light adds to what a hit keeps).
     const bool chain = !packet && has_light_chain(s);
     size_t hit_cap = 0, light_cap = 0; // hits and light rays that may wait
     auto ensure_chain = [&](size_t hits, size_t lights) -> int {
@@ -925,7 +926,7 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     if (chain) {
         constexpr size_t kWaitBytes = (size_t)256 << 20;
         const size_t per_hit = 12 + sizeof(ShadeOut) + 4 + 20 * nl + spp * (sizeof(pvx_ray) + 8 + 4 + 12);
-        const size_t hits = nray + std::min(3 * nray, kWaitBytes / per_hit);
+        const size_t hits = nray + std::min(15 * nray, kWaitBytes / per_hit);
         if ((r = ensure_chain(hits, hits * spp))) {
             // no room: give back what was reserved, one frame's worth then
             // takes less than light rays followed a layer a launch
