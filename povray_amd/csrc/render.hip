@@ -978,11 +978,15 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     p.bailout = sh.bailout;
     for (int k = 0; k < 3; k++) p.bg[k] = sh.background[k];
 
-    hipEvent_t e0, e1, t0, t1;
+    // t0, t1: a bounce's own launches; w0, w1: the waiting light rays', which
+    // may be followed between a bounce's records and their read-back
+    hipEvent_t e0, e1, t0, t1, w0, w1;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventCreate(&t0));
     HIP_TRY(hipEventCreate(&t1));
+    HIP_TRY(hipEventCreate(&w0));
+    HIP_TRY(hipEventCreate(&w1));
     double trace_ms = 0.0, shadow_ms = 0.0;
     uint64_t n_closest = 0, n_shadow = 0;
     uint32_t bounces = 0;
@@ -1087,13 +1091,13 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         uint32_t more = 0;
         if (n_lights > 0) {
             uint32_t *d_more = static_cast<uint32_t *>(b.gcount.p) + 8;
-            HIP_TRY(hipEventRecord(t0, st));
+            HIP_TRY(hipEventRecord(w0, st));
             k_zero_word<<<1, 64, 0, st>>>(d_more);
             if ((rr = light_chain_internal(s, static_cast<const pvx_ray *>(b.srays[0].p),
                                            static_cast<const double *>(b.sdepth[0].p), n_lights, light_kind, sh.d_mats,
                                            static_cast<float *>(b.scol.p), d_more, st)))
                 return rr;
-            HIP_TRY(hipEventRecord(t1, st));
+            HIP_TRY(hipEventRecord(w1, st));
             HIP_TRY(hipMemcpyAsync(&more, d_more, 4, hipMemcpyDeviceToHost, st));
         }
         for (const Waiting &w : waiting) {
@@ -1111,7 +1115,7 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         HIP_TRY(hipStreamSynchronize(st));
         if (n_lights > 0) {
             float ms = 0.0f;
-            HIP_TRY(hipEventElapsedTime(&ms, t0, t1));
+            HIP_TRY(hipEventElapsedTime(&ms, w0, w1));
             shadow_ms += ms;
             n_shadow += n_lights + more;
         }
@@ -1138,7 +1142,8 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
         } else if (chain) {
             if (n_hits + n > hit_cap || n_lights + (size_t)n * spp > light_cap) {
                 if ((r = follow_waiting())) return r;
-                if ((n > hit_cap || (size_t)n * spp > light_cap) && (r = ensure_chain(std::max(hit_cap, (size_t)n), std::max(light_cap, (size_t)n * spp))))
+                if ((n > hit_cap || (size_t)n * spp > light_cap) &&
+                    (r = ensure_chain(std::max(hit_cap, (size_t)n), std::max(light_cap, (size_t)n * spp))))
                     return r;
             }
         } else if ((r = ensure_shadow((size_t)n * spp))) {
@@ -1370,6 +1375,8 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     (void)hipEventDestroy(e1);
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
+    (void)hipEventDestroy(w0);
+    (void)hipEventDestroy(w1);
     if (stats) {
         stats->closest_rays = n_closest;
         stats->shadow_rays = n_shadow;

@@ -88,3 +88,32 @@ def test_waiting_light_rays_are_bounded(gpu):
     free = _free_bytes()
     g.render(160, 90)
     assert free - _free_bytes() < (256 + 85 + 100) << 20
+
+
+def _many_lights(n, w, h):
+    """A glass frame whose hits keep so much (`n` lights) that only a few
+    frames' worth wait: light rays are followed in the middle of the frame."""
+    s = scenes.csg_scene(n_objects=1000, width=w, height=h)
+    r = np.random.default_rng(4)
+    s.lights = [dict(kind="point", position=p, colour=np.full(3, 1.0 / n)) for p in r.uniform(-30.0, 30.0, (n, 3))]
+    return s
+
+
+def test_light_rays_followed_mid_frame(gpu):
+    # 256 lights: a hit keeps 24 KB, 256 MB hold 2.2 more frames' worth of 96 x
+    # 54 rays.  Against light rays followed a layer a launch, which waits for
+    # none (the kd-tree's frames): image and light-ray count.  The light rays
+    # are followed between a bounce's closest hits and the read-back of their
+    # time, which must not take the light rays' for its own (all is on one
+    # stream, so the two sums are parts of the frame).
+    s = _many_lights(256, 96, 54)
+    g, steps = gpu.GpuScene(s), gpu.GpuScene(s, accel=A.PVX_ACCEL_BSP)
+    g.set_shading()
+    steps.set_shading()
+    ref, rst = steps.render()
+    for _ in range(2):
+        img, st = g.render()
+        assert st["closest_rays"] > 3.2 * 96 * 54
+        assert np.array_equal(img, ref)
+        assert st["shadow_rays"] == rst["shadow_rays"] and st["closest_rays"] == rst["closest_rays"]
+        assert st["trace_ms"] + st["shadow_ms"] <= 1.01 * st["total_ms"]
