@@ -1186,22 +1186,29 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         }
         return a;
     };
-    std::function<Bnd(uint32_t, uint32_t, uint32_t)> shape_bnd = [&](uint32_t type, uint32_t index,
-                                                                       uint32_t flags) -> Bnd {
-        if (type != PVX_CSG) {
-            DBox b = leaf_box(type, index);
-            return Bnd{b, (flags & PVX_FLAG_INVERTED) ? DBox::unbounded() : b};
-        }
-        const CsgNode &n = out.csg[index];
+    // of every operand below a root, once
+    std::vector<Bnd> slot_bnd(d.n_csg_children);
+    auto bound_csg = [&](auto &&self, uint32_t node) -> Bnd {
+        const CsgNode &n = out.csg[node];
         DBox S = DBox::empty(), V = (n.op == PVX_CSG_INTERSECTION) ? DBox::unbounded() : DBox::empty();
         for (uint32_t k = 0; k < n.count; k++) {
             const CsgChild &c = out.csg_children[n.first + k];
-            Bnd cb = shape_bnd(c.type, c.index, c.flags);
+            Bnd &cb = slot_bnd[n.first + k];
+            if (c.type == PVX_CSG) {
+                cb = self(self, c.index);
+            } else {
+                const DBox box = leaf_box(c.type, c.index);
+                cb = Bnd{box, (c.flags & PVX_FLAG_INVERTED) ? DBox::unbounded() : box};
+            }
             S = join(S, cb.S);
             V = (n.op == PVX_CSG_INTERSECTION) ? meet(V, cb.V) : join(V, cb.V);
         }
         if (n.op == PVX_CSG_INTERSECTION) S = meet(S, V);
         return Bnd{S, V};
+    };
+    // the surface bound of an object's shape
+    auto surface_box = [&](uint32_t type, uint32_t index) -> DBox {
+        return type == PVX_CSG ? bound_csg(bound_csg, index).S : leaf_box(type, index);
     };
 
     // A bounded CSG object of spheres, boxes, tori and cones enters the tree as
@@ -1218,24 +1225,38 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         uint32_t slot;
         DBox box;
     };
-    std::function<bool(uint32_t, const DBox &, std::vector<CsgPart> &)> split_csg =
-        [&](uint32_t node, const DBox &clip, std::vector<CsgPart> &parts) -> bool {
+    auto can_split = [&](auto &&self, uint32_t node) -> bool {
         const CsgNode &n = out.csg[node];
         for (uint32_t k = 0; k < n.count; k++) {
             const CsgChild &c = out.csg_children[n.first + k];
-            if (shared[n.first + k] > 1) return false; // its filters are not this node's alone
-            DBox b = clip;
-            if (n.op == PVX_CSG_INTERSECTION)
-                for (uint32_t j = 0; j < n.count; j++) {
-                    const CsgChild &sib = out.csg_children[n.first + j];
-                    if (j != k) b = meet(b, shape_bnd(sib.type, sib.index, sib.flags).V);
-                }
+            if (c.type == PVX_CSG ? !self(self, c.index)
+                                  : shared[n.first + k] > 1 || (c.type != PVX_SPHERE && c.type != PVX_BOX &&
+                                                                c.type != PVX_TORUS && c.type != PVX_CONE))
+                return false;
+        }
+        return true;
+    };
+    auto split_csg = [&](auto &&self, uint32_t node, const DBox &clip, std::vector<CsgPart> &parts) -> void {
+        const CsgNode &n = out.csg[node];
+        // of an intersection's operand: the regions of the ones after it, and
+        // (as the loop goes on) of the ones before it
+        const bool meets = n.op == PVX_CSG_INTERSECTION;
+        std::vector<DBox> after;
+        DBox before = clip;
+        if (meets) {
+            after.assign(n.count + 1, DBox::unbounded());
+            for (uint32_t k = n.count; k-- > 0;) after[k] = meet(after[k + 1], slot_bnd[n.first + k].V);
+        }
+        for (uint32_t k = 0; k < n.count; k++) {
+            const CsgChild &c = out.csg_children[n.first + k];
+            const Bnd &cb = slot_bnd[n.first + k];
+            DBox b = meets ? meet(before, after[k + 1]) : clip;
+            if (meets) before = meet(before, cb.V);
             if (c.type == PVX_CSG) {
-                if (!split_csg(c.index, b, parts)) return false;
+                self(self, c.index, b, parts);
                 continue;
             }
-            if (c.type != PVX_SPHERE && c.type != PVX_BOX && c.type != PVX_TORUS && c.type != PVX_CONE) return false;
-            b = meet(b, leaf_box(c.type, c.index));
+            b = meet(b, cb.S);
             bool empty = false;
             for (int a = 0; a < 3; a++) {
                 const double pad = 1.0e-4 * std::fabs(b.hi[a] - b.lo[a]) +
@@ -1246,7 +1267,6 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
             }
             if (!empty) parts.push_back(CsgPart{n.first + k, b});
         }
-        return true;
     };
     const bool bvh_accel = !opts || opts->accel == PVX_ACCEL_BVH;
 
@@ -1299,7 +1319,7 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
             pr.kind_axis = kPrimSphere;
             for (int k = 0; k < 3; k++) pr.sph.c[k] = out.sph[4 * ob.index + k];
             pr.sph.r = out.sph[4 * ob.index + 3];
-            to_fbox(shape_bnd(ob.type, ob.index, 0).S, lo, hi);
+            to_fbox(surface_box(ob.type, ob.index), lo, hi);
             add_prim(pr, lo, hi);
             break;
         }
@@ -1312,13 +1332,13 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
                            : ob.type == PVX_CONE  ? kPrimCone
                                                   : kPrimDisc;
             pr.ref.index = ob.index;
-            to_fbox(shape_bnd(ob.type, ob.index, 0).S, lo, hi);
+            to_fbox(surface_box(ob.type, ob.index), lo, hi);
             add_prim(pr, lo, hi);
             out.has_complex = std::max<uint32_t>(out.has_complex, ob.type == PVX_BOX ? 1u : 2u);
             break;
         }
         case PVX_CSG: {
-            DBox b = shape_bnd(ob.type, ob.index, 0).S;
+            DBox b = surface_box(ob.type, ob.index);
             if (!b.bounded || !(b.lo[0] <= b.hi[0] && b.lo[1] <= b.hi[1] && b.lo[2] <= b.hi[2])) {
                 if (!b.bounded) {
                     out.inf.push_back(InfRec{kPrimCsg, ob.index, (int32_t)o, 0});
@@ -1329,7 +1349,8 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
             }
             out.has_complex = 2;
             std::vector<CsgPart> parts;
-            if (bvh_accel && split_csg(ob.index, DBox::unbounded(), parts)) {
+            if (bvh_accel && can_split(can_split, ob.index)) {
+                split_csg(split_csg, ob.index, DBox::unbounded(), parts);
                 for (const CsgPart &part : parts) {
                     pr.kind_axis = kPrimCsgLeaf;
                     pr.ref.index = part.slot;
@@ -1355,7 +1376,7 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         case PVX_SOR:
             pr.kind_axis = kPrimRevolution;
             pr.ref.index = ob.index;
-            to_fbox(shape_bnd(ob.type, ob.index, 0).S, lo, hi);
+            to_fbox(surface_box(ob.type, ob.index), lo, hi);
             add_prim(pr, lo, hi);
             break;
         case PVX_POLYGON: {

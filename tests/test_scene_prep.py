@@ -65,3 +65,29 @@ def test_cycle_of_csg_nodes(prep, op):
     _in_child(lambda: prep(_spheres(nodes, kids, [3]))[0], 0)  # no object refers to the cycles
     for root in (0, 2):
         _in_child(lambda: prep(_spheres(nodes, kids, [root]))[:2], (1, "a nested CSG node is listed as a top-level object"))
+
+
+def _holes(n):
+    """A box minus n spheres: one CSG object, an intersection of n + 1 operands."""
+    r = np.random.default_rng(1)
+    kids = [[A.PVX_BOX, 0, 0, 0]] + [[A.PVX_SPHERE, k, A.PVX_FLAG_INVERTED, 0] for k in range(n)]
+    return scenes.Scene(
+        name="holes", objects=np.array([[A.PVX_CSG, 0, 0, 0]], np.uint32), sphere_center=r.uniform(-4.0, 4.0, (n, 3)),
+        sphere_radius=np.full(n, 0.2), box_corner1=np.array([[-4.0, -4.0, -4.0]]),
+        box_corner2=np.array([[4.0, 4.0, 4.0]]), box_transform=np.array([-1], np.int32),
+        csg=np.array([[A.PVX_CSG_INTERSECTION, 0, n + 1, 0]], np.uint32), csg_children=np.array(kids, np.uint32),
+        camera=scenes.look_at_camera((0.0, 0.0, -12.0), (0.0, 0.0, 0.0), 16, 12))
+
+
+def test_wide_difference_is_linear(prep):
+    # eight times the operands: eight times the work and a little more for the
+    # deeper tree, not sixty-four times
+    ms = []
+    for n in (1000, 8000):
+        s, best = _holes(n), 1e9
+        for _ in range(5):
+            rc, msg, t, sizes = prep(s)
+            assert rc == 0 and sizes[0] == n + 1, msg
+            best = min(best, t)
+        ms.append(best)
+    assert ms[1] < 24.0 * ms[0]
