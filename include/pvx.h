@@ -365,7 +365,8 @@ int pvx_trace_closest_counted(pvx_scene *scene, const pvx_ray *rays,
  * hipMalloc).  Same arguments, results and checks as pvx_trace_closest; the
  * traversal-stack spill area is a fixed 32 MiB device array of the library
  * (one per device, held until the process ends) instead of the per-stream
- * area pvx_trace_closest allocates on a stream's first launch, so the
+ * area pvx_trace_closest allocates on a stream's first launch for a tree
+ * that may need one (deeper than 24 levels in the binary tree), so the
  * persistent grid is capped at what it holds (840 blocks of 256 lanes).
  * Every call on one device shares that array: calls that overlap in time on
  * one device (other streams, other threads) race and must not be issued.
@@ -398,7 +399,8 @@ enum {
 
 typedef struct pvx_tune_result {
     uint32_t variant;      /* chosen PVX_TRAVERSAL_*                        */
-    uint32_t grid_blocks;  /* chosen persistent grid (blocks of 256 lanes)  */
+    uint32_t grid_blocks;  /* chosen persistent grid (blocks of 256 lanes);
+                              see pvx_scene_set_traversal for where it counts */
     double best_ms;        /* its time per launch on the sample              */
     double default_ms;     /* the untuned choice's time on the same sample   */
     uint32_t tile_w;       /* pvx_render_autotune's camera rays: the chosen  */
@@ -406,9 +408,9 @@ typedef struct pvx_tune_result {
                               tile_w 0 with tile_h 1: row-major)             */
 } pvx_tune_result;
 
-/* Autotuner: times the traversal variants this scene admits on persistent
- * grids of one and two times the resident blocks, over the caller's sample
- * rays (device), and keeps the fastest for later closest-hit calls on rays
+/* Autotuner: times the traversal variants this scene admits (on persistent
+ * grids of one and two times the resident blocks where the variant takes one)
+ * over the caller's sample rays (device), and keeps the fastest for later closest-hit calls on rays
  * of the same class (PVX_RAY_SHADOW, or every other kind).  No reference
  * counterpart (the reference has one traversal).  Results of later calls are
  * unchanged; only their speed is. */
@@ -419,7 +421,10 @@ int pvx_scene_autotune(pvx_scene *scene, const pvx_ray *rays, size_t n, uint32_t
  * choice saved from an earlier pvx_scene_autotune); variant
  * PVX_TRAVERSAL_DEFAULT with grid_blocks 0 restores the untuned behaviour.
  * PVX_EINVAL for a variant the scene does not admit or grid_blocks above
- * twice the resident blocks.  Not to be called while launches on the scene
+ * twice the resident blocks.  A walk whose stack always fits in LDS (binary
+ * trees of depth up to 24, 4-wide ones up to 7; depths as in
+ * pvx_scene_get_stats for the binary tree) launches over all rays at once,
+ * and grid_blocks then changes nothing.  Not to be called while launches on the scene
  * are being issued from another thread. */
 int pvx_scene_set_traversal(pvx_scene *scene, uint32_t ray_kind, uint32_t variant, uint32_t grid_blocks);
 

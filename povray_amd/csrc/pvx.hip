@@ -392,8 +392,8 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
     return PVX_OK;
 }
 
-// The scene's spill area for launches on `st` (allocated on the stream's
-// first launch; freed with the scene).
+// The scene's spill area for launches on `st` (allocated on the first launch
+// on the stream whose walk may need one; freed with the scene).
 static int scene_spill(pvx_scene *s, hipStream_t st, int32_t **out) {
     std::lock_guard<std::mutex> lock(s->spill_mu);
     for (const auto &e : s->spills)
@@ -433,10 +433,19 @@ extern "C" int pvx_scene_get_stats(const pvx_scene *s, pvx_scene_stats *out) {
     return PVX_OK;
 }
 
-// Whether the walk may launch over all rays (kWholeGrid).
+// Whether the walk's stack cannot outgrow its LDS entries: it needs no spill
+// area, and may launch over all rays (kWholeGrid).
 static bool stack_in_lds(const HostScene &h, bool wide) {
     // a binary node pushes at most one link, a wide one three
     return (wide ? 3 * (h.depth4 + 1) : h.depth + 1) <= (uint32_t)kStackLds;
+}
+
+// Whether a closest-hit launch with `variant` covers all rays whatever grid
+// was picked for it.
+static bool whole_grid(const pvx_scene *s, uint32_t variant) {
+    const bool wide = kernel_level(s->view) == 0 &&
+                      (variant == PVX_TRAVERSAL_WIDE_WW || variant == PVX_TRAVERSAL_WIDE_STEP);
+    return !s->use_kd && stack_in_lds(s->host, wide);
 }
 
 // One closest-hit launch with an explicit traversal variant and grid.
@@ -447,11 +456,13 @@ template <bool kCount>
 static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_depth, uint32_t ray_kind,
                           const uint8_t *kinds, size_t n, pvx_hit *hits, uint32_t *nv, uint32_t *pt,
                           hipStream_t st, uint32_t variant, uint32_t grid, int32_t *spill = nullptr) {
-    int r;
-    if (!spill && (r = scene_spill(s, st, &spill))) return r;
     const uint32_t level = kernel_level(s->view);
     const bool wide = level == 0 && (variant == PVX_TRAVERSAL_WIDE_WW || variant == PVX_TRAVERSAL_WIDE_STEP);
-    if (!s->use_kd && stack_in_lds(s->host, wide)) grid = kWholeGrid;
+    int r;
+    if (whole_grid(s, variant))
+        grid = kWholeGrid;
+    else if (!spill && !s->use_kd && (r = scene_spill(s, st, &spill))) // the kd walk keeps its stack itself
+        return r;
     const bool few = !s->use_kd && !wide && variant != PVX_TRAVERSAL_BINARY_WW;
     const uint32_t wave_rays = few ? rays_per_wave(n, s->grid) : 64u;
     const uint32_t nblocks = launch_units(n, wave_rays, grid);
@@ -581,7 +592,7 @@ int pvx::autotune_internal(pvx_scene *s, const pvx_ray *rays, const double *max_
         r = time_one(PVX_TRAVERSAL_DEFAULT, s->grid, dflt);
         for (uint32_t v : variants)
             for (uint32_t g : {s->grid, 2 * s->grid}) {
-                if (r) break;
+                if (r || (g != s->grid && whole_grid(s, v))) break; // one launch shape
                 double ms = 0;
                 r = time_one(v, g, ms);
                 if (!r && ms < best) {
@@ -618,7 +629,7 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     if (n_rays == 0) return PVX_OK;
     int r;
     int32_t *spill = nullptr;
-    if ((r = scene_spill(s, st, &spill))) return r;
+    if (!stack_in_lds(s->host, !binary) && (r = scene_spill(s, st, &spill))) return r;
     // the fixed-stride walks on twice the resident blocks (the light rays of
     // one shaded point differ little in length, the tail of a launch more:
     // 19.3 ms against 21.8 ms on the resident grid for the 1.3M-triangle
@@ -659,7 +670,7 @@ int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *d
     if (n == 0) return PVX_OK;
     int r;
     int32_t *spill = nullptr;
-    if ((r = scene_spill(s, st, &spill))) return r;
+    if (!stack_in_lds(s->host, false) && (r = scene_spill(s, st, &spill))) return r;
     TraceArgs ta{};
     // the resident grid: a lane whose ray has ended takes another while the
     // others follow theirs through further layers
@@ -780,7 +791,7 @@ extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx
     b->whole = true;
     for (const pvx_scene *s : b->scenes) b->whole = b->whole && stack_in_lds(s->host, false);
     const size_t spill_bytes = (size_t)b->grid * kBlock * kStackSpill * sizeof(int32_t);
-    if ((r = b->spill.reserve(spill_bytes)) != PVX_OK) {
+    if (!b->whole && (r = b->spill.reserve(spill_bytes)) != PVX_OK) {
         pvx_batch_destroy(b);
         return r;
     }
