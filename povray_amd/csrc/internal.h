@@ -155,6 +155,7 @@ struct pvx_batch {
     int device = 0;
     std::vector<pvx_scene *> scenes;
     uint32_t level = 0;     // largest has_complex of the scenes
+    uint32_t kinds = 0;     // union of the scenes' kinds
     uint32_t any_flags = 0; // union of the scenes' object flags
     uint32_t grid = 0;      // resident blocks of the batch's walk
     bool whole = false;     // its launches cover all rays (no scene can outgrow the LDS stack)

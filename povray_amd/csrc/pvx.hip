@@ -106,14 +106,17 @@ hipError_t pvx::trace_launch(const TraceKernel &k, const TraceArgs &a, uint32_t 
         switch (k.walk) {
         case kWalkStep4:
         case kWalkWW4: return trace_part0(k, a, nb, st, occ);
+        case kWalkSimple:
         case kWalkBinary: return trace_part1(k, a, nb, st, occ);
         case kWalkBinary0:
         case kWalkBinary0WW: return trace_part16(k, a, nb, st, occ);
+        case kWalkCsg:
         case kWalkComplex:
             return (k.flags ? (k.count ? trace_part5 : trace_part4) : (k.count ? trace_part3 : trace_part2))(k, a, nb, st,
                                                                                                           occ);
         case kWalkKd: return trace_part6(k, a, nb, st, occ);
         case kWalkRevolution: return trace_part13(k, a, nb, st, occ);
+        case kWalkChainCsg:
         case kWalkChain: return trace_part17(k, a, nb, st, occ);
         case kWalkChainRev: return trace_part18(k, a, nb, st, occ);
         case kWalkLightWW:
@@ -125,8 +128,10 @@ hipError_t pvx::trace_launch(const TraceKernel &k, const TraceArgs &a, uint32_t 
     }
     switch (k.walk) {
     case kWalkBinary0:
+    case kWalkSimple:
     case kWalkBinary: return trace_part7(k, a, nb, st, occ);
     case kWalkRevolution: return trace_part14(k, a, nb, st, occ);
+    case kWalkCsg:
     case kWalkComplex:
         return (k.flags ? (k.count ? trace_part11 : trace_part10) : (k.count ? trace_part9 : trace_part8))(k, a, nb, st,
                                                                                                         occ);
@@ -224,6 +229,14 @@ static void scene_free(pvx_scene *s) {
 // tree), 1 (+ boxes) or 2 (+ tori, CSG).  A triangle scene whose 4-wide tree
 // is too deep for the traversal stack takes the binary tree (family 1).
 static uint32_t kernel_level(const SceneView &v) { return v.has_complex == 0 && !v.wide ? 1u : v.has_complex; }
+
+// The default walk through the binary tree of scenes up to `level` whose
+// objects include `kinds`.
+static TraceWalk binary_walk(uint32_t level, uint32_t kinds) {
+    if (level >= 3) return kWalkRevolution;
+    if (level == 2) return kinds & kKindTorus ? kWalkComplex : kinds & kKindCsg ? kWalkCsg : kWalkSimple;
+    return level == 1 ? kWalkBinary : kWalkBinary0;
+}
 
 // The no-allocation closest-hit entry point keeps its traversal-stack spill
 // area in this fixed device array (one copy per device).
@@ -368,7 +381,10 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
     // the 4-wide walk pushes up to three links per level
     v.wide = (h.has_complex == 0 && 3 * h.depth4 + 1 < (uint32_t)kStackMax) ? 1u : 0u;
     v.n_inf = (uint32_t)h.inf.size();
+    v.n_inf_planes = h.n_inf_planes;
+    v.n_inf_plain = h.n_inf_plain;
     v.any_flags = h.any_flags;
+    v.kinds = h.kinds;
     v.has_complex = h.has_complex;
 
     // persistent grid: enough resident blocks to fill every CU
@@ -376,12 +392,7 @@ extern "C" int pvx_scene_create(const pvx_scene_desc *desc, const pvx_build_opts
     HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device));
     int per_cu = 0;
     {
-        const uint32_t level = kernel_level(v);
-        const TraceKernel k{level >= 3   ? kWalkRevolution
-                            : level == 2 ? kWalkComplex
-                            : level == 1 ? kWalkBinary
-                                         : kWalkBinary0,
-                            h.any_flags != 0, false, false};
+        const TraceKernel k{binary_walk(kernel_level(v), v.kinds), h.any_flags != 0, false, false};
         TraceArgs none{};
         HIP_TRY(trace_launch(k, none, 0, nullptr, &per_cu));
     }
@@ -470,20 +481,12 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
     TraceKernel k{kWalkStep4, flags, kCount, false};
     if (s->use_kd)
         k.walk = kWalkKd;
-    else if (level >= 3)
-        k.walk = kWalkRevolution;
-    else if (level == 2)
-        k.walk = kWalkComplex;
     else if (level == 0 && variant == PVX_TRAVERSAL_BINARY_WW)
         k.walk = kWalkBinary0WW;
-    else if (level == 1)
-        k.walk = kWalkBinary;
-    else if (variant == PVX_TRAVERSAL_WIDE_WW)
-        k.walk = kWalkWW4;
-    else if (variant == PVX_TRAVERSAL_WIDE_STEP)
-        k.walk = kWalkStep4;
+    else if (wide)
+        k.walk = variant == PVX_TRAVERSAL_WIDE_WW ? kWalkWW4 : kWalkStep4;
     else
-        k.walk = kWalkBinary0;
+        k.walk = binary_walk(level, s->view.kinds);
     TraceArgs ta{};
     ta.sv = s->view;
     ta.kd = s->kd;
@@ -685,9 +688,10 @@ int pvx::light_chain_internal(pvx_scene *s, const pvx_ray *rays, const double *d
     ta.chain_mats = mats;
     ta.chain_col = col;
     ta.chain_more = more;
-    HIP_TRY(trace_launch(TraceKernel{kernel_level(s->view) >= 3 ? kWalkChainRev : kWalkChain, s->view.any_flags != 0,
-                                     false, false},
-                         ta, nb, st));
+    const TraceWalk walk = kernel_level(s->view) >= 3         ? kWalkChainRev
+                           : s->view.kinds & kKindTorus ? kWalkChain
+                                                        : kWalkChainCsg;
+    HIP_TRY(trace_launch(TraceKernel{walk, s->view.any_flags != 0, false, false}, ta, nb, st));
     return PVX_OK;
 }
 
@@ -740,10 +744,6 @@ extern "C" int pvx_trace_closest_noalloc(pvx_scene *s, const pvx_ray *rays, cons
 // ----------------------------------------------------------------------------
 // scene batches
 // ----------------------------------------------------------------------------
-static TraceWalk batch_walk(uint32_t level) {
-    return level >= 3 ? kWalkRevolution : level == 2 ? kWalkComplex : level == 1 ? kWalkBinary : kWalkBinary0;
-}
-
 extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx_batch **out) {
     if (!out) return fail(PVX_EINVAL, "null argument");
     *out = nullptr;
@@ -751,19 +751,21 @@ extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx
     int dev = 0;
     HIP_TRY(hipGetDevice(&dev));
     std::vector<SceneView> views(n_scenes);
-    uint32_t level = 0, flags = 0;
+    uint32_t level = 0, flags = 0, kinds = 0;
     for (uint32_t k = 0; k < n_scenes; k++) {
         const pvx_scene *s = scenes[k];
         if (!s) return fail(PVX_EINVAL, "null scene in the batch");
         if (s->device != dev) return fail(PVX_EINVAL, "scene " + std::to_string(k) + " lives on another device");
         views[k] = s->view;
         level = std::max(level, kernel_level(s->view));
+        kinds |= s->view.kinds;
         flags |= s->view.any_flags;
     }
     pvx_batch *b = new pvx_batch();
     b->device = dev;
     b->scenes.assign(scenes, scenes + n_scenes);
     b->level = level;
+    b->kinds = kinds;
     b->any_flags = flags;
     int r;
     if ((r = b->views.reserve(views.size() * sizeof(SceneView))) != PVX_OK) {
@@ -779,7 +781,7 @@ extern "C" int pvx_batch_create(pvx_scene *const *scenes, uint32_t n_scenes, pvx
     // the walk of the most demanding scene: over all rays when every scene's
     // stack fits in LDS, else on a persistent grid
     int cus = 0, per = 0;
-    const TraceKernel kb{batch_walk(level), flags != 0, false, true};
+    const TraceKernel kb{binary_walk(level, kinds), flags != 0, false, true};
     TraceArgs none{};
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess) e = trace_launch(kb, none, 0, nullptr, &per);
@@ -869,7 +871,7 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     const SceneView *views = static_cast<const SceneView *>(b->views.p);
     const uint4 *chunks = static_cast<const uint4 *>(b->chunks.p);
     int32_t *spill = static_cast<int32_t *>(b->spill.p);
-    const TraceKernel k{batch_walk(b->level), flags, kCount, true};
+    const TraceKernel k{binary_walk(b->level, b->kinds), flags, kCount, true};
     TraceArgs ta{};
     ta.wave_rays = 64;
     ta.views = views;

@@ -346,6 +346,8 @@ struct InfRec {
     uint32_t pad;
 };
 
+constexpr uint32_t kKindTorus = 1u, kKindCsg = 2u; // SceneView::kinds
+
 // Everything a kernel needs, passed by value.
 struct SceneView {
     const Node *nodes;
@@ -385,8 +387,10 @@ struct SceneView {
     uint32_t wide;     // 1: triangle/sphere scene traversed through nodes4
     int32_t root;      // root link (node index or leaf link); INT32_MIN = empty
     uint32_t n_inf;
+    uint32_t n_inf_planes, n_inf_plain; // the planes, the planes and quadrics, which come first in inf
     uint32_t any_flags;
-    uint32_t has_complex; // 0: mesh triangles/spheres only, 1: + boxes, stand-alone triangles, 2: + tori or CSG,
+    uint32_t kinds;       // kKind* bits: what a level-2 walk must be able to test
+    uint32_t has_complex; // 0: mesh triangles/spheres only, 1: + boxes, stand-alone triangles, 2: + any other but
                           // 3: + lathes or sors
 };
 

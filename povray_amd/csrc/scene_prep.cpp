@@ -1526,7 +1526,13 @@ int prepare_scene(const pvx_scene_desc &d, const pvx_build_opts *opts, HostScene
         }
     }
 
+    auto first = [&](auto &&is) { return (uint32_t)(std::stable_partition(out.inf.begin(), out.inf.end(), is) - out.inf.begin()); };
+    out.n_inf_plain = first([](const InfRec &r) { return r.kind != kPrimCsg; });
+    out.n_inf_planes = first([](const InfRec &r) { return r.kind == kPrimPlane; });
     if (uses_rev) out.has_complex = 3; // lathes / sors: the level-3 walks
+    if (!out.tori.empty()) out.kinds |= kKindTorus;
+    for (uint32_t o = 0; o < d.n_objects; o++)
+        if (d.objects[o].type == PVX_CSG) out.kinds |= kKindCsg;
     // --- BVH ---------------------------------------------------------------------
     // One primitive a leaf in the binary tree the default walks take (camera
     // rays of the 1.3M-triangle icosphere with 1, 2 and 4: 591, 622, 733 us;

@@ -22,7 +22,8 @@ struct HostScene {
     std::vector<Node4> nodes4; // 4-wide tree (triangle / sphere scenes)
     int32_t root4 = INT32_MIN;
     uint32_t depth4 = 0;
-    std::vector<InfRec> inf;
+    std::vector<InfRec> inf; // objects outside the tree: planes, quadrics, CSG
+    uint32_t n_inf_planes = 0, n_inf_plain = 0;
     std::vector<uint32_t> obj_flags;
     std::vector<uint32_t> obj_type;
     std::vector<PlaneRec> planes;
@@ -52,7 +53,8 @@ struct HostScene {
     std::vector<int32_t> obj_mesh_xf; // per object: a mesh's placement (xforms index) or -1
     std::vector<float> mesh_vtx, mesh_nrm;
     uint32_t any_flags = 0;
-    uint32_t has_complex = 0; // 0: triangles/spheres, 1: + boxes, 2: + tori or CSG, 3: + lathes or sors
+    uint32_t has_complex = 0; // 0: triangles/spheres, 1: + boxes, 2: + any other kind but lathes and sors, 3: + those
+    uint32_t kinds = 0;       // kKind* bits
     uint64_t n_triangles = 0;
     double build_ms = 0.0;
     double bvh_ms = 0.0;         // the tree build alone

@@ -152,9 +152,9 @@ __device__ inline bool quadric_closest(const QuadricRec &q, D3 o, D3 d, bool sha
     return found;
 }
 
-// Closest valid hit of a box / torus / stand-alone triangle object
-// (Find_Intersection over its IStack); with kRev also lathes and sors.
-template <bool kRev = false>
+// Closest valid hit of an object of any kind but CSG (Find_Intersection over
+// its IStack); with kRev also lathes and sors, without kTorus no tori.
+template <bool kRev = false, bool kTorus = true>
 __device__ inline bool simple_closest(const SceneView &sv, uint32_t kind, uint32_t index, D3 o,
                                       D3 d, bool shadow, double &dep_out) {
     if constexpr (kRev) {
@@ -183,12 +183,13 @@ __device__ inline bool simple_closest(const SceneView &sv, uint32_t kind, uint32
     double hs[kMaxLeafHits];
     int side[4];
     int nh = kind == kPrimBox    ? box_hits(sv.boxes[index], sv.xforms, o, d, hs, side)
-             : kind == kPrimCone ? cone_hits(sv.cones[index], sv.xforms, o, d, hs, side)
-                                 : torus_hits(sv.tori[index], sv.xforms, o, d, hs);
+             : !kTorus || kind == kPrimCone ? cone_hits(sv.cones[index], sv.xforms, o, d, hs, side)
+                                            : torus_hits(sv.tori[index], sv.xforms, o, d, hs);
     bool found = false;
     double best = 0.0;
-    for (int j = 0; j < nh; j++) {
-        if (depth_ok(hs[j], shadow) && (!found || hs[j] < best)) {
+#pragma unroll
+    for (int j = 0; j < kMaxLeafHits; j++) {
+        if (j < nh && depth_ok(hs[j], shadow) && (!found || hs[j] < best)) {
             best = hs[j];
             found = true;
         }
@@ -197,8 +198,9 @@ __device__ inline bool simple_closest(const SceneView &sv, uint32_t kind, uint32
     return found;
 }
 
-// kLevel 0: triangles and spheres; 1: also boxes and stand-alone triangles
-// (the levels above: trace_ref_body).
+// kLevel 0: triangles and spheres; 1: also boxes and stand-alone triangles; 2:
+// also cones, discs, polygons and quadrics (the walk of scenes with tori or
+// CSG: trace_ref_body).
 // kWW: while-while traversal (triangle scenes, camera and bounce rays).
 // kMulti: rays of many scenes in one launch.  `n` is then 64 x the number of
 // chunks; chunk c = {scene, first ray, ray count <= 64} covers the wavefront
@@ -240,7 +242,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
     }
 
     // binary walks: wave_rays rays per wavefront (rays_per_wave in pvx.hip)
-    const bool part = (kLevel == 1 || kBin) && !kMulti && !kGen;
+    const bool part = (kLevel >= 1 || kBin) && !kMulti && !kGen;
     if (part && lane >= wave_rays) return;
     const uint32_t i0 = xcd_block() * (part ? wave_rays : (uint32_t)kWaveBlock) + lane;
     const uint32_t istep = gridDim.x * (part ? wave_rays : (uint32_t)kWaveBlock);
@@ -283,7 +285,9 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
             const InfRec inf = sv.inf[k];
             if (kFlags && !precondition(sv.obj_flags[inf.obj], rk)) continue;
             double dep;
-            const bool ok = inf.kind == kPrimPlane && plane_hit(sv.planes[inf.index], o, d, dep) && depth_ok(dep, shadow);
+            const bool ok = kLevel >= 2 && inf.kind == kPrimQuadric
+                                ? quadric_closest(sv.quadrics[inf.index], o, d, shadow, dep)
+                                : inf.kind == kPrimPlane && plane_hit(sv.planes[inf.index], o, d, dep) && depth_ok(dep, shadow);
             if (ok && better(dep, inf.obj, 0, bt, bo, bp)) {
                 bt = dep;
                 bo = inf.obj;
@@ -603,6 +607,16 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
                                     }
                             }
                             tb = (float)bt * 1.000001f;
+                        } else if (kLevel >= 2) { // boxes, stand-alone triangles, cones, discs and polygons
+                            if (!ref_box_hit(p.ref, rf, tb)) continue;
+                            double dep;
+                            if (simple_closest<false, false>(sv, pk, p.ref.index, o, d, shadow, dep) &&
+                                better(dep, obj, 0, bt, bo, bp)) {
+                                bt = dep;
+                                bo = obj;
+                                bp = 0;
+                            }
+                            tb = (float)bt * 1.000001f;
                         }
                     }
                     tb = (float)bt * 1.000001f;
@@ -629,8 +643,8 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
     }
 }
 
-// Walk of scenes with any primitive kind (kLevel 2: all but lathes and sors;
-// 3: those too) through the binary tree.  What bounds it is the FP64 primitive
+// Walk of scenes with CSG or tori (kLevel 2: every kind but lathes and sors,
+// without kTorus no tori; 3: those too) through the binary tree.  What bounds it is the FP64 primitive
 // tests: a torus takes thousands of instructions, a node forty.  So each
 // lane walks nodes, and discards primitives by their own FP32 box, until it
 // holds one primitive to test (or its ray ends); then the lanes of the
@@ -641,6 +655,14 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
 // with the leaves of CSG objects in the tree, the root finder in registers and
 // the filter programs, that launch went from 7.2 to 1.3 ms and the shaded
 // 5,000-leaf glass frame (641 x 359) from 767 to 70 ms.
+//
+// Cheap tests do not repay the waiting, and the quartic costs registers (944
+// bytes of scratch a lane) also where nothing needs it.  So scenes without
+// tori take an instantiation without it (20 bytes), and scenes without CSG
+// too the walk above.  Camera rays of the mixed field (459 cones and
+// cylinders, discs, polygons, CSG; 519 x 302) 269 -> 222 us without the
+// quartic; 300 cones at 640 x 480 200 -> 162 so, 86 us with the tests at the
+// leaf; 300 discs 160 -> 127 and 54 us.
 //
 // Rays per wavefront: with fewer rays than the resident grid has lanes, a
 // launch gives each wavefront only `wave_rays` of them (a power of two), so
@@ -654,7 +676,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
 // written.  One launch instead of one per layer, each of which lasted as long
 // as its slowest ray: the 5,000-leaf glass frame (641 x 359) made 249 such
 // launches of 0.2 ms.
-template <int kLevel, bool kFlags, bool kCount, bool kMulti = false, bool kChain = false>
+template <int kLevel, bool kTorus, bool kFlags, bool kCount, bool kMulti = false, bool kChain = false>
 __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_stack) {
     const uint32_t wl = threadIdx.x; // a block is one wavefront
     const uint32_t gtid = blockIdx.x * kWaveBlock + wl;
@@ -702,13 +724,32 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
         rf.oix = (float)o.x * rf.ix;
         rf.oiy = (float)o.y * rf.iy;
         rf.oiz = (float)o.z * rf.iz;
-        float tb = (float)bt * 1.000001f;
         uint32_t cnt_nodes = 0, cnt_prims = 0;
-        uint32_t inf_k = 0;             // objects outside the tree come first
+        // Objects outside the tree come first: the planes and, without tori, the
+        // quadrics, which the lanes go through together (loads of one address;
+        // 150 quadrics, 640 x 480 camera rays: 565 us one by one, 175 us so),
+        // then the others (a second copy of the quadric's test costs the walk
+        // with the quartic 2 %)
+        const uint32_t n_here = kTorus ? sv.n_inf_planes : sv.n_inf_plain;
+        for (uint32_t k = 0; k < n_here; k++) {
+            const InfRec inf = sv.inf[k];
+            if (kFlags && !precondition(sv.obj_flags[inf.obj], rk)) continue;
+            double dep;
+            if ((kTorus || inf.kind == kPrimPlane ? plane_hit(sv.planes[inf.index], o, d, dep) && depth_ok(dep, shadow)
+                                        : quadric_closest(sv.quadrics[inf.index], o, d, shadow, dep)) &&
+                better(dep, inf.obj, 0, bt, bo, bp)) {
+                bt = dep;
+                bo = inf.obj;
+                bp = 0;
+            }
+        }
+        const bool blocked = occl && bo >= 0 && bt < occl_lim;
+        float tb = (float)bt * 1.000001f;
+        uint32_t inf_k = blocked ? sv.n_inf : n_here;
         uint32_t cur = 0, end = 0;      // primitives left of the leaf at hand
         uint32_t slot_k = 0, slot_e = 0; // leaves left of the whole CSG object at hand
         int32_t slot_obj = 0;
-        int32_t node = sv.root;
+        int32_t node = blocked ? kEmpty : sv.root;
         int sp = 0;
         for (;;) {
             // --- to the next primitive to test: its type, its index in that
@@ -730,32 +771,22 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                     have = true;
                     break;
                 }
-                uint32_t pk, index;
+                uint32_t index;
                 if (inf_k < sv.n_inf) {
                     const InfRec inf = sv.inf[inf_k++];
-                    pk = inf.kind;
                     index = inf.index;
                     obj = inf.obj;
                     if (kFlags && !precondition(sv.obj_flags[obj], rk)) continue;
-                    if (pk == kPrimPlane) {
-                        double dep;
-                        if (plane_hit(sv.planes[index], o, d, dep) && depth_ok(dep, shadow) &&
-                            better(dep, obj, 0, bt, bo, bp)) {
-                            bt = dep;
-                            bo = obj;
-                            bp = 0;
-                            tb = (float)bt * 1.000001f;
-                            if (occl && bt < occl_lim) { // blocked
-                                inf_k = sv.n_inf;
-                                node = kEmpty;
-                            }
-                        }
-                        continue;
+                    if (kTorus && inf.kind != kPrimCsg) {
+                        type = PVX_QUADRIC;
+                        shape = index;
+                        have = true;
+                        break;
                     }
                 } else if (cur < end) {
                     const PrimRec &p = sv.prims[cur++];
                     const uint32_t ka = p.kind_axis;
-                    pk = ka & 15u;
+                    const uint32_t pk = ka & 15u;
                     obj = p.obj;
                     if (kFlags && !precondition(sv.obj_flags[obj], rk)) continue;
                     if (pk == kPrimTriangle) {
@@ -848,16 +879,10 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                 } else {
                     break; // the ray's walk is over
                 }
-                if (pk == kPrimCsg) { // a whole CSG object: its leaves one by one
-                    slot_k = sv.csg_leaf_range[2 * index];
-                    slot_e = sv.csg_leaf_range[2 * index + 1];
-                    slot_obj = obj;
-                    continue;
-                }
-                type = PVX_QUADRIC; // the other kind outside the tree
-                shape = index;
-                have = true;
-                break;
+                // a whole CSG object: its leaves one by one
+                slot_k = sv.csg_leaf_range[2 * index];
+                slot_e = sv.csg_leaf_range[2 * index + 1];
+                slot_obj = obj;
             }
             if (!have) break;
             // --- test it: its hits that the CSG filters keep
@@ -885,13 +910,14 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
                     const bool xf = (rflags & kPlacedXf) != 0;
                     const D3 P = xf ? pl_point(r.inv, o) : o, D = xf ? pl_dir(r.inv, d) : d;
                     int side[2];
-                    nh = type == PVX_BOX ? box_hits_at(r.q, r.q + 3, P, D, hs, side)
-                                         : torus_hits_at(r.q[0], r.q[1], (rflags & kPlacedSturm) != 0, P, D, hs);
+                    nh = !kTorus || type == PVX_BOX
+                             ? box_hits_at(r.q, r.q + 3, P, D, hs, side)
+                             : torus_hits_at(r.q[0], r.q[1], (rflags & kPlacedSturm) != 0, P, D, hs);
                 } else if (type == PVX_SPHERE) {
                     const double *s = sph ? sph : sv.sph + 4 * (size_t)shape;
                     nh = sphere_hits(d3(s[0], s[1], s[2]), s[3], o, d, hs);
                 } else {
-                    nh = other_hits(sv, type, shape, o, d, hs);
+                    nh = other_hits<(kLevel < 3 && !kTorus)>(sv, type, shape, o, d, hs);
                 }
                 // nearest first: once one is kept, the others are farther
                 sort_hits(hs, nh);

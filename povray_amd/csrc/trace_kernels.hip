@@ -24,21 +24,21 @@ __global__ __launch_bounds__(kWaveBlock) void k_trace_closest(TraceArgs a) {
                                                       s_stack, nullptr, nullptr, 1, nullptr, a.wave_rays);
 }
 
-// Scenes with any primitive kind (levels 2 and 3).
-template <int kLevel, bool kFlags, bool kCount>
+// Scenes with CSG or tori (levels 2 and 3).
+template <int kLevel, bool kTorus, bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
-    trace_ref_body<kLevel, kFlags, kCount>(a, s_stack);
+    trace_ref_body<kLevel, kTorus, kFlags, kCount>(a, s_stack);
 }
-template <int kLevel, bool kFlags>
+template <int kLevel, bool kTorus, bool kFlags>
 __global__ __launch_bounds__(kWaveBlock, 4) void k_light_chain(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
-    trace_ref_body<kLevel, kFlags, false, false, true>(a, s_stack);
+    trace_ref_body<kLevel, kTorus, kFlags, false, false, true>(a, s_stack);
 }
-template <int kLevel, bool kFlags, bool kCount>
+template <int kLevel, bool kTorus, bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref_multi(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
-    trace_ref_body<kLevel, kFlags, kCount, true>(a, s_stack);
+    trace_ref_body<kLevel, kTorus, kFlags, kCount, true>(a, s_stack);
 }
 
 // Level-0 scenes (triangles, spheres, planes) through the binary tree.
@@ -603,25 +603,26 @@ hipError_t launch_inside(const SceneView &sv, const double *pts, const uint32_t 
 hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint32_t nb, hipStream_t st, int *occ) {
 #if PVX_TRACE_PART == 0 // single scene, 4-wide walks
     return k.walk == kWalkWW4 ? PVX_FC(run_waves, k_trace_closest_ww, ) : PVX_FC(run_waves, k_trace_closest, 0, );
-#elif PVX_TRACE_PART == 1 // single scene, binary walk
-    return PVX_FC(run_waves, k_trace_closest, 1, );
-#elif PVX_TRACE_PART >= 2 && PVX_TRACE_PART <= 5 // single scene, every primitive kind
+#elif PVX_TRACE_PART == 1 // single scene, binary walks with the tests at the leaf
+    return k.walk == kWalkSimple ? PVX_FC(run_waves, k_trace_closest, 2, ) : PVX_FC(run_waves, k_trace_closest, 1, );
+#elif PVX_TRACE_PART >= 2 && PVX_TRACE_PART <= 5 // single scene with CSG or tori
     constexpr bool kF = (PVX_TRACE_PART - 2) >= 2, kC = (PVX_TRACE_PART - 2) & 1;
-    (void)k;
-    return run_waves(k_trace_ref<2, kF, kC>, a, nb, st, occ);
+    return k.walk == kWalkCsg ? run_waves(k_trace_ref<2, false, kF, kC>, a, nb, st, occ)
+                              : run_waves(k_trace_ref<2, true, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 6 // kd-tree
     return PVX_FC(run, k_trace_closest_kd, );
-#elif PVX_TRACE_PART == 7 // scene batches: 4-wide and binary walks
-    return k.walk == kWalkBinary0 ? PVX_FC(run_waves, k_trace_closest_bin0_multi, )
-                                  : PVX_FC(run_waves, k_trace_closest_multi, 1, );
-#elif PVX_TRACE_PART >= 8 && PVX_TRACE_PART <= 11 // scene batches, every primitive kind
+#elif PVX_TRACE_PART == 7 // scene batches: binary walks with the tests at the leaf
+    return k.walk == kWalkBinary0  ? PVX_FC(run_waves, k_trace_closest_bin0_multi, )
+           : k.walk == kWalkSimple ? PVX_FC(run_waves, k_trace_closest_multi, 2, )
+                                   : PVX_FC(run_waves, k_trace_closest_multi, 1, );
+#elif PVX_TRACE_PART >= 8 && PVX_TRACE_PART <= 11 // scene batches with CSG or tori
     constexpr bool kF = (PVX_TRACE_PART - 8) >= 2, kC = (PVX_TRACE_PART - 8) & 1;
-    (void)k;
-    return run_waves(k_trace_ref_multi<2, kF, kC>, a, nb, st, occ);
+    return k.walk == kWalkCsg ? run_waves(k_trace_ref_multi<2, false, kF, kC>, a, nb, st, occ)
+                              : run_waves(k_trace_ref_multi<2, true, kF, kC>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 13 // single scene with lathes or sors
-    return PVX_FC(run_waves, k_trace_ref, 3, );
+    return PVX_FC(run_waves, k_trace_ref, 3, true, );
 #elif PVX_TRACE_PART == 14 // scene batches with lathes or sors
-    return PVX_FC(run_waves, k_trace_ref_multi, 3, );
+    return PVX_FC(run_waves, k_trace_ref_multi, 3, true, );
 #elif PVX_TRACE_PART == 16 // single scene, level-0 primitives on the binary tree
     return k.walk == kWalkBinary0WW ? PVX_FC(run_waves, k_trace_closest_bin0, true, ) : PVX_FC(run_waves, k_trace_closest_bin0, false, );
 #elif PVX_TRACE_PART == 15 // light rays made in the kernel
@@ -633,9 +634,14 @@ hipError_t PVX_FN(PVX_TRACE_PART)(const TraceKernel &k, const TraceArgs &a, uint
         return k.flags ? run_waves(k_light_bin<true>, a, nb, st, occ) : run_waves(k_light_bin<false>, a, nb, st, occ);
     return k.flags ? run_waves(k_light_ww<true>, a, nb, st, occ) : run_waves(k_light_ww<false>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 17 // light rays through transparent objects
-    return k.flags ? run_waves(k_light_chain<2, true>, a, nb, st, occ) : run_waves(k_light_chain<2, false>, a, nb, st, occ);
+    if (k.walk == kWalkChainCsg)
+        return k.flags ? run_waves(k_light_chain<2, false, true>, a, nb, st, occ)
+                       : run_waves(k_light_chain<2, false, false>, a, nb, st, occ);
+    return k.flags ? run_waves(k_light_chain<2, true, true>, a, nb, st, occ)
+                   : run_waves(k_light_chain<2, true, false>, a, nb, st, occ);
 #elif PVX_TRACE_PART == 18
-    return k.flags ? run_waves(k_light_chain<3, true>, a, nb, st, occ) : run_waves(k_light_chain<3, false>, a, nb, st, occ);
+    return k.flags ? run_waves(k_light_chain<3, true, true>, a, nb, st, occ)
+                   : run_waves(k_light_chain<3, true, false>, a, nb, st, occ);
 #else
 #error "PVX_TRACE_PART out of range"
 #endif

@@ -30,8 +30,8 @@ constexpr size_t kSpillPerThread = (size_t)kStackSpill * sizeof(int32_t);
 // Traversal walks: the 4-wide tree one node or leaf per pass (triangle and
 // sphere scenes, light rays), the 4-wide tree while-while (camera and bounce
 // rays), the binary tree (+ boxes and stand-alone triangles), the binary tree
-// with every primitive kind (+ tori, CSG, cones, ...), the kd-tree, the
-// binary tree with lathes and sors as well.
+// with every primitive kind but lathes and sors, the kd-tree, the binary tree
+// with lathes and sors as well.
 enum TraceWalk : uint32_t {
     kWalkStep4 = 0,
     kWalkWW4 = 1,
@@ -46,7 +46,10 @@ enum TraceWalk : uint32_t {
     kWalkBinary0WW = 10, // kWalkBinary0 in while-while passes
     kWalkLightDynBin = 11, // kWalkLightDyn through the binary tree
     kWalkChain = 12,       // light rays through transparent objects, every kind but lathes and sors
-    kWalkChainRev = 13     // ... with lathes and sors
+    kWalkChainRev = 13,    // ... with lathes and sors
+    kWalkSimple = 14,      // kWalkBinary with cones, discs, polygons and quadrics
+    kWalkCsg = 15,         // kWalkComplex without tori
+    kWalkChainCsg = 16     // kWalkChain without tori
 };
 
 struct TraceKernel {

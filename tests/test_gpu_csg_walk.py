@@ -155,3 +155,49 @@ def test_child_ranges_that_overlap(gpu):
     for ob in range(len(roots)):
         which = np.full(pts.shape[0], ob, np.uint32)
         assert np.array_equal(g.inside(pts, which), orc.inside(pts, which)), nodes[roots[ob]]
+
+
+def _no_csg(s):
+    s.objects = s.objects[s.objects[:, 0] != A.PVX_CSG]
+    return s
+
+
+# what a scene holds picks its walk: cones, discs, polygons and quadrics alone,
+# with CSG, with tori
+BY_CONTENT = [("simple", lambda: _no_csg(scenes.cone_scene(n=60, width=97, height=71))),
+              ("quadrics", lambda: _no_csg(scenes.cone_scene(n=1, n_discs=3, n_quadrics=40, n_polygons=0, width=97, height=71))),
+              ("csg", lambda: scenes.cone_scene(n=60, width=97, height=71)),
+              ("torus", lambda: scenes.torus_scene(n=20, width=97, height=71)),
+              ("placed", lambda: scenes.placed_mesh_scene(level=2, width=97, height=71))]
+
+
+@pytest.mark.parametrize("name,make", BY_CONTENT)
+def test_walks_by_content(gpu, name, make):
+    s = make()
+    rays = scenes.camera_rays_np(s.camera)
+    r = np.random.default_rng(3)
+    md = r.uniform(4.0, 20.0, rays.shape[0])
+    g, kd, orc = gpu.GpuScene(s), gpu.GpuScene(s, accel=A.PVX_ACCEL_BSP), OracleScene(s)
+    boxes = scenes.radiosity_scene(n_boxes=50, width=64, height=48)  # a batch takes the walk of both
+    both = gpu.GpuBatch([g, gpu.GpuScene(boxes)])
+    box_rays = scenes.camera_rays_np(boxes.camera)
+    for kind, dist in ((A.PVX_RAY_IMAGE, None), (A.PVX_RAY_REFLECTION, None), (A.PVX_RAY_SHADOW, md)):
+        h = g.find_intersection(rays, dist, kind)
+        _same(h, kd.find_intersection(rays, dist, kind))
+        c = orc.find_intersection(rays, dist, kind, method=0)
+        assert np.array_equal(h["obj"], c["obj"]) and np.array_equal(h["prim"], c["prim"])
+        hit = c["obj"] >= 0
+        assert np.abs(h["t"][hit] / c["t"][hit] - 1.0).max(initial=0.0) <= 1e-5
+        mds = None if dist is None else [dist, np.full(box_rays.shape[0], 5.0)]
+        _same(h, both.find_intersection([rays, box_rays], kind, mds)[0])
+        for n in (1, 63, 1025):  # few rays per wavefront
+            _same(h[:n], g.find_intersection(rays[:n], None if dist is None else dist[:n], kind))
+
+
+def test_batch_of_every_walk(gpu):
+    made = [make() for _, make in BY_CONTENT]
+    rays = [scenes.camera_rays_np(s.camera) for s in made]
+    gs = [gpu.GpuScene(s) for s in made]
+    for upto in range(1, len(gs) + 1):
+        for g, r, h in zip(gs[:upto], rays, gpu.GpuBatch(gs[:upto]).find_intersection(rays[:upto])):
+            _same(g.find_intersection(r), h)
