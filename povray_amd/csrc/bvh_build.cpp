@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstring>
 #include <future>
+#include <system_error>
 #include <thread>
 
 namespace pvx {
@@ -48,6 +49,23 @@ struct Box3 {
     }
 };
 
+// work(0) ... work(n - 1) on threads of their own, or here where the system
+// gives no more threads (an exception past the C interface would end the
+// caller's program).
+template <class Work>
+void on_threads(size_t n, Work &&work) {
+    std::vector<std::thread> pool;
+    pool.reserve(n);
+    for (uint32_t k = 0; k < n; k++) {
+        try {
+            pool.emplace_back([&work, k]() { work(k); });
+        } catch (const std::system_error &) {
+            work(k);
+        }
+    }
+    for (auto &t : pool) t.join();
+}
+
 class Builder {
   public:
     Builder(const float *lo, const float *hi, uint32_t n, int max_leaf, int bins)
@@ -80,7 +98,7 @@ class Builder {
         std::vector<int> sub_depth(tasks.size(), 0);
         unsigned hw = std::max(1u, std::thread::hardware_concurrency());
         std::atomic_size_t next(0);
-        auto worker = [&]() {
+        on_threads(std::min<size_t>(hw, tasks.size()), [&](uint32_t) {
             for (;;) {
                 size_t t = next.fetch_add(1);
                 if (t >= tasks.size()) break;
@@ -88,10 +106,7 @@ class Builder {
                 sub_root[t] = build_rec(tasks[t].b, tasks[t].e, tasks[t].depth, sub[t], md);
                 sub_depth[t] = md;
             }
-        };
-        std::vector<std::thread> pool;
-        for (unsigned i = 0; i < std::min<size_t>(hw, tasks.size()); i++) pool.emplace_back(worker);
-        for (auto &th : pool) th.join();
+        });
         // Phase 3: concatenate in task order and patch links.
         res.nodes = std::move(top);
         auto fix = [](int32_t link, int32_t off) { return link >= 0 ? link + off : link; };
@@ -187,13 +202,10 @@ class Builder {
         const uint32_t parts =
             std::min({16u, std::max(1u, std::thread::hardware_concurrency()), (e - b) / kMaxGrain});
         std::vector<T> res(parts, out);
-        std::vector<std::thread> pool;
-        for (uint32_t k = 0; k < parts; k++)
-            pool.emplace_back([&, k]() {
-                work(b + (uint32_t)((uint64_t)(e - b) * k / parts), b + (uint32_t)((uint64_t)(e - b) * (k + 1) / parts),
-                     res[k]);
-            });
-        for (auto &t : pool) t.join();
+        on_threads(parts, [&](uint32_t k) {
+            work(b + (uint32_t)((uint64_t)(e - b) * k / parts), b + (uint32_t)((uint64_t)(e - b) * (k + 1) / parts),
+                 res[k]);
+        });
         for (const T &r : res) merge(out, r);
     }
 

@@ -91,3 +91,21 @@ def test_wide_difference_is_linear(prep):
             best = min(best, t)
         ms.append(best)
     assert ms[1] < 24.0 * ms[0]
+
+
+def test_no_threads_left(prep):
+    # a stack size that no thread can have: std::thread throws, the tree is
+    # built all the same
+    s = scenes.sphere_scene(n=100000)
+    want = prep(s)[3]
+
+    def starved():
+        attr, L = C.create_string_buffer(64), C.CDLL(None)
+        L.pthread_attr_setstacksize.argtypes = [C.c_void_p, C.c_size_t]
+        L.pthread_attr_init(attr)
+        assert L.pthread_attr_setstacksize(attr, 1 << 46) == 0
+        assert L.pthread_setattr_default_np(attr) == 0
+        rc, msg, _, sizes = prep(s)
+        return rc, sizes
+
+    _in_child(starved, (0, want))
