@@ -1,7 +1,8 @@
 """Light rays followed through glass in the walk, the bounces of a frame
-together: frames against the oracle's TraceRay, with area lights (several
-light rays a hit), supersampling (more hits wait), and many layers in a row;
-the light-ray count is the layer-by-layer one."""
+together: frames against the oracle's TraceRay and against light rays followed
+a layer a launch (the kd-tree's frames), image and light-ray count, with area
+lights (several light rays a hit), supersampling, more layers in a row than
+are followed, and light rays followed in the middle of a frame."""
 import ctypes as C
 
 import numpy as np
@@ -48,15 +49,23 @@ AREA = [dict(kind="area", position=np.array([0.0, 12.0, 0.0]), axis1=np.array([2
              axis2=np.array([0.0, 0.0, 2.0]), size=(3, 4), colour=np.ones(3))]
 
 
-@pytest.mark.parametrize("n,lights", [(1, POINT), (20, POINT), (40, POINT), (6, AREA), (3, POINT + AREA)])
+# a light ray meets two surfaces a box and is followed through at most 64: 33
+# boxes and more end it on the way
+@pytest.mark.parametrize("n,lights", [(1, POINT), (20, POINT), (31, POINT), (32, POINT), (33, POINT), (40, POINT),
+                                      (70, POINT), (6, AREA), (3, POINT + AREA)])
 def test_layers(gpu, n, lights):
     s = _layers(n, lights)
-    g = gpu.GpuScene(s)
+    g, steps = gpu.GpuScene(s), gpu.GpuScene(s, accel=A.PVX_ACCEL_BSP)
     g.set_shading()
+    steps.set_shading()
     img, st = g.render()
-    ref, rst = OracleScene(s).render(s)
+    ref, _ = OracleScene(s).render(s)
     _close(img, ref)
-    assert st["shadow_rays"] >= st["closest_rays"] // 4  # the layers' rays are counted
+    by_layer, sst = steps.render()  # light rays followed a layer a launch
+    assert np.array_equal(img, by_layer)
+    assert st["shadow_rays"] == sst["shadow_rays"] and st["closest_rays"] == sst["closest_rays"]
+    if lights is POINT and n >= 33:  # some light rays of the floor were followed to the limit
+        assert st["shadow_rays"] > 64 * 96
     again, st2 = g.render()
     assert np.array_equal(img, again) and st2["shadow_rays"] == st["shadow_rays"]
 
