@@ -1,10 +1,11 @@
 // pvx: MI355X (gfx950) closest-hit / per-shape / camera kernels and the C-ABI.
 //
 // Closest hit (replaces Trace::FindIntersection, core/render/trace.cpp:285-344):
-//   * one lane per ray, persistent grid sized to the device (wave64);
+//   * one lane per ray, blocks of one wavefront, a launch over all rays (on a
+//     persistent grid where the tree can outgrow the stack in LDS);
 //   * FP32 traversal of a BVH2 (64 B nodes): slab test in FMA form against
 //     conservative boxes, near child first, far child pushed on a per-lane
-//     LDS stack (32 entries, [depth][lane] so lanes never share a bank) that
+//     LDS stack (25 entries, [depth][lane] so lanes never share a bank) that
 //     overflows into a per-lane global spill area;
 //   * leaves hold 64 B primitive records: mesh triangles and spheres inline,
 //     boxes/tori/CSG by reference.  Each candidate is decided with the
@@ -461,8 +462,9 @@ static bool whole_grid(const pvx_scene *s, uint32_t variant) {
 
 // One closest-hit launch with an explicit traversal variant and grid.
 // variant: PVX_TRAVERSAL_DEFAULT (by scene content and ray kind), _WIDE_WW,
-// _WIDE_STEP (4-wide tree; triangle/sphere scenes) or _BINARY (binary tree,
-// scenes without tori/CSG); every variant gives the same hits.
+// _WIDE_STEP (4-wide tree; triangle/sphere scenes), _BINARY (binary tree,
+// scenes of triangles, spheres and boxes) or _BINARY_WW (triangle/sphere
+// scenes); every variant gives the same hits.
 template <bool kCount>
 static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_depth, uint32_t ray_kind,
                           const uint8_t *kinds, size_t n, pvx_hit *hits, uint32_t *nv, uint32_t *pt,
@@ -476,7 +478,6 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
         return r;
     const bool few = !s->use_kd && !wide && variant != PVX_TRAVERSAL_BINARY_WW;
     const uint32_t wave_rays = few ? rays_per_wave(n, s->grid) : 64u;
-    const uint32_t nblocks = launch_units(n, wave_rays, grid);
     const bool flags = s->view.any_flags != 0 && (ray_kind != PVX_RAY_PRIMARY || kinds);
     TraceKernel k{kWalkStep4, flags, kCount, false};
     if (s->use_kd)
@@ -490,17 +491,19 @@ static int launch_variant(pvx_scene *s, const pvx_ray *rays, const double *max_d
     TraceArgs ta{};
     ta.sv = s->view;
     ta.kd = s->kd;
-    ta.rays = rays;
-    ta.max_depth = max_depth;
     ta.kind = ray_kind;
-    ta.kinds = kinds;
-    ta.n = (uint32_t)n;
     ta.wave_rays = wave_rays;
-    ta.hits = hits;
     ta.spill = spill;
-    ta.node_visits = nv;
-    ta.prim_tests = pt;
-    HIP_TRY(trace_launch(k, ta, nblocks, st));
+    for (size_t at = 0; at < n; at += kMaxLaunch) {
+        ta.n = (uint32_t)std::min<size_t>(n - at, kMaxLaunch);
+        ta.rays = rays + at;
+        ta.max_depth = max_depth ? max_depth + at : nullptr;
+        ta.kinds = kinds ? kinds + at : nullptr;
+        ta.hits = hits + at;
+        ta.node_visits = nv ? nv + at : nullptr;
+        ta.prim_tests = pt ? pt + at : nullptr;
+        HIP_TRY(trace_launch(k, ta, launch_units(ta.n, wave_rays, grid), st));
+    }
     return PVX_OK;
 }
 
@@ -520,8 +523,8 @@ static int launch_closest(pvx_scene *s, const pvx_ray *rays, const double *max_d
                                   static_cast<hipStream_t>(stream), variant, grid);
 }
 
-// Variants a scene admits: the kd-tree and tori/CSG scenes have one walk;
-// box/triangle scenes the binary tree; triangle/sphere scenes all three.
+// Variants a scene admits: triangle/sphere scenes all four; box and
+// stand-alone-triangle scenes the binary tree; the others have one walk.
 static std::vector<uint32_t> scene_variants(const pvx_scene *s) {
     const uint32_t level = kernel_level(s->view);
     if (s->use_kd || level >= 2) return {PVX_TRAVERSAL_DEFAULT};
@@ -555,8 +558,8 @@ extern "C" int pvx_scene_set_traversal(pvx_scene *s, uint32_t ray_kind, uint32_t
     return PVX_OK;
 }
 
-// Times every traversal variant the scene admits, on persistent grids of
-// one and two times the resident blocks, over the caller's rays (1 warm-up +
+// Times every traversal variant the scene admits (on persistent grids of one
+// and two times the resident blocks where it takes one), over the caller's rays (1 warm-up +
 // 3 timed launches each), and keeps the fastest for rays of this class
 // (light rays, or camera / bounce / radiosity rays).
 int pvx::autotune_internal(pvx_scene *s, const pvx_ray *rays, const double *max_depth, size_t n,
@@ -633,6 +636,7 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     int r;
     int32_t *spill = nullptr;
     if (!stack_in_lds(s->host, !binary) && (r = scene_spill(s, st, &spill))) return r;
+    if (n_rays > kMaxLaunch) next = nullptr; // its counter is for one launch
     // the fixed-stride walks on twice the resident blocks (the light rays of
     // one shaded point differ little in length, the tail of a launch more:
     // 19.3 ms against 21.8 ms on the resident grid for the 1.3M-triangle
@@ -640,16 +644,12 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     // to fill; the binary walk over all rays when its stack fits in LDS
     uint32_t grid = grid_blocks ? grid_blocks : next ? s->grid : 2 * s->grid;
     if (!next && binary && stack_in_lds(s->host, false)) grid = kWholeGrid;
-    const uint32_t nb = launch_units(n_rays, 64, grid);
     TraceArgs ta{};
     ta.wave_rays = 64;
     ta.sv = s->view;
-    ta.n = n_rays;
     ta.spill = spill;
-    ta.gen_groups = groups;
     ta.gen_lights = lights;
     ta.gen_S = S;
-    ta.gen_vis = vis;
     ta.gen_next = next;
     ta.gen_count = count;
     // refill a wavefront once no more than 16 of its lanes hold rays: new
@@ -658,9 +658,16 @@ int pvx::light_rays_internal(pvx_scene *s, const LightGroup *groups, const Light
     // free lane at once mixes rays of distant points and is slower (the
     // 1.3M-triangle frame: 27.5 ms against 18.0 ms at 16 and 18.5 ms at 0)
     ta.gen_refill_below = 16;
-    HIP_TRY(trace_launch(TraceKernel{next ? (binary ? kWalkLightDynBin : kWalkLightDyn) : binary ? kWalkLightBin : kWalkLightWW,
-                                     s->view.any_flags != 0, false, false},
-                         ta, nb, st));
+    const TraceKernel k{next ? (binary ? kWalkLightDynBin : kWalkLightDyn) : binary ? kWalkLightBin : kWalkLightWW,
+                        s->view.any_flags != 0, false, false};
+    const uint32_t most = kMaxLaunch / S * S; // rays of whole groups
+    for (size_t at = 0; at < n_rays; at += most) {
+        ta.n = (uint32_t)std::min<size_t>(n_rays - at, most);
+        ta.gen_first = (uint32_t)(at / S);
+        ta.gen_groups = groups + ta.gen_first;
+        ta.gen_vis = vis + at;
+        HIP_TRY(trace_launch(k, ta, launch_units(ta.n, 64, grid), st));
+    }
     return PVX_OK;
 }
 
@@ -867,7 +874,7 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     // with per-scene clocks the persistent grid: every wavefront's start is an
     // atomic on one word (64 scenes, 45 M rays, one wavefront per chunk: 9.4 ms
     // instead of 7.1 ms in 64 launches)
-    const uint32_t nblocks = launch_units(n, 64, b->whole && !clk ? kWholeGrid : b->grid);
+    const uint32_t grid = b->whole && !clk ? kWholeGrid : b->grid;
     const SceneView *views = static_cast<const SceneView *>(b->views.p);
     const uint4 *chunks = static_cast<const uint4 *>(b->chunks.p);
     int32_t *spill = static_cast<int32_t *>(b->spill.p);
@@ -875,17 +882,19 @@ static int launch_batch(pvx_batch *b, const pvx_ray *rays, const uint64_t *first
     TraceArgs ta{};
     ta.wave_rays = 64;
     ta.views = views;
-    ta.chunks = chunks;
     ta.clocks = clk;
     ta.rays = rays;
     ta.max_depth = max_depth;
     ta.kind = ray_kind;
-    ta.n = n;
     ta.hits = hits;
     ta.spill = spill;
     ta.node_visits = nv;
     ta.prim_tests = pt;
-    HIP_TRY(trace_launch(k, ta, nblocks, st));
+    for (size_t at = 0; at < n; at += kMaxLaunch) { // the chunks say which rays are theirs
+        ta.n = (uint32_t)std::min<size_t>(n - at, kMaxLaunch);
+        ta.chunks = chunks + at / 64;
+        HIP_TRY(trace_launch(k, ta, launch_units(ta.n, 64, grid), st));
+    }
     return PVX_OK;
 }
 

@@ -980,13 +980,15 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
 
     // t0, t1: a bounce's own launches; w0, w1: the waiting light rays', which
     // may be followed between a bounce's records and their read-back
-    hipEvent_t e0, e1, t0, t1, w0, w1;
+    hipEvent_t e0, e1, t0, t1, w0 = nullptr, w1 = nullptr;
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventCreate(&t0));
     HIP_TRY(hipEventCreate(&t1));
-    HIP_TRY(hipEventCreate(&w0));
-    HIP_TRY(hipEventCreate(&w1));
+    if (chain) {
+        HIP_TRY(hipEventCreate(&w0));
+        HIP_TRY(hipEventCreate(&w1));
+    }
     double trace_ms = 0.0, shadow_ms = 0.0;
     uint64_t n_closest = 0, n_shadow = 0;
     uint32_t bounces = 0;
@@ -1375,8 +1377,8 @@ static int render_frame(pvx_scene *s, const pvx_camera *cam, uint32_t S, const d
     (void)hipEventDestroy(e1);
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
-    (void)hipEventDestroy(w0);
-    (void)hipEventDestroy(w1);
+    if (w0) (void)hipEventDestroy(w0);
+    if (w1) (void)hipEventDestroy(w1);
     if (stats) {
         stats->closest_rays = n_closest;
         stats->shadow_rays = n_shadow;

@@ -246,7 +246,7 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
     if (part && lane >= wave_rays) return;
     const uint32_t i0 = xcd_block() * (part ? wave_rays : (uint32_t)kWaveBlock) + lane;
     const uint32_t istep = gridDim.x * (part ? wave_rays : (uint32_t)kWaveBlock);
-    for (uint32_t i = i0; i < n; i = next_ray(i, istep, n)) {
+    for (uint32_t i = i0; i < n; i += istep) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
             const uint4 ch = chunks[__builtin_amdgcn_readfirstlane(i >> 6)];
@@ -307,11 +307,10 @@ __device__ __forceinline__ void trace_closest_body(const SceneView &sv0, const S
         int32_t node = (occl && bo >= 0 && bt < occl_lim) ? kEmpty : (kLevel == 0 && !kBin) ? sv.root4 : sv.root;
         int sp = 0;
         uint32_t cnt_nodes = 0, cnt_prims = 0;
-        // Triangle / sphere scenes traverse the 4-wide tree; camera and
-        // bounce rays with while-while passes (the lanes of a wavefront visit
-        // inner nodes together, then leaves together), light rays one node or
-        // leaf per pass.  Scenes with boxes, tori and CSG, whose leaf tests
-        // are long, take the binary tree one step per pass.
+        // Without kBin, level 0 walks the 4-wide tree: in while-while passes
+        // (kWW: the lanes of a wavefront visit inner nodes together, then
+        // leaves together) or one node or leaf a pass.  All others walk the
+        // binary tree, kNodeSteps nodes, then a leaf, a pass.
 #define PVX_POP()                                                                       \
     do {                                                                                \
         if (sp == 0) {                                                                  \
@@ -697,7 +696,7 @@ __device__ __forceinline__ void trace_ref_body(const TraceArgs &a, int32_t *s_st
     bool on = false;         // kChain: the ray goes on behind a blocker
     uint32_t more = 0;       // kChain: continued rays
     for (uint32_t i = kChain && wl >= per_wave ? n : (kMulti ? blockIdx.x : xcd_block()) * per_wave + wl; i < n;
-         i = kChain && on ? i : next_ray(i, step, n)) {
+         i += kChain && on ? 0u : step) {
         uint32_t ri = i, scene = 0;
         if constexpr (kMulti) {
             const uint4 ch = a.chunks[__builtin_amdgcn_readfirstlane(i >> 6)];

@@ -42,8 +42,8 @@ __global__ __launch_bounds__(kWaveBlock, 4) void k_trace_ref_multi(TraceArgs a) 
 }
 
 // Level-0 scenes (triangles, spheres, planes) through the binary tree.
-// 92 VGPRs, 5 wavefronts per SIMD (the level-1 binary kernel, with box
-// leaves, needs 108 and spills; forcing 6 here spills and is slower).
+// 80 VGPRs, 6 wavefronts per SIMD (82 and 5 with object flags and counters;
+// the level-1 kernel, with box leaves, takes 104 and 4, without spills).
 // kWW: while-while passes (inner nodes, then leaves, lane by lane).
 template <bool kWW, bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock) void k_trace_closest_bin0(TraceArgs a) {
@@ -54,9 +54,8 @@ __global__ __launch_bounds__(kWaveBlock) void k_trace_closest_bin0(TraceArgs a) 
                                                                     nullptr, nullptr, 1, nullptr, a.wave_rays);
 }
 
-// Triangle scenes, camera and bounce rays: while-while traversal (78 VGPRs
-// and a 24 KB LDS stack per block: 6 wavefronts per SIMD; forcing 7 or 8
-// costs more in register pressure than it gains).
+// Triangle scenes, 4-wide tree: while-while traversal (80 VGPRs and a 6.4 KB
+// LDS stack per wavefront: 6 wavefronts per SIMD).
 template <bool kFlags, bool kCount>
 __global__ __launch_bounds__(kWaveBlock) void k_trace_closest_ww(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
@@ -64,14 +63,22 @@ __global__ __launch_bounds__(kWaveBlock) void k_trace_closest_ww(TraceArgs a) {
                                                 a.kinds, a.n, a.hits, a.spill, a.node_visits, a.prim_tests, s_stack);
 }
 
+// Rays of a launch of light rays made in the kernel: a.n, or, with a group
+// count on the device, what this part of the launch has of them.
+__device__ __forceinline__ uint32_t gen_rays(const TraceArgs &a) {
+    if (!a.gen_count) return a.n;
+    const uint32_t groups = a.gen_count[0];
+    return min(groups > a.gen_first ? (groups - a.gen_first) * a.gen_S : 0u, a.n);
+}
+
 // Light rays of pvx_render made in the kernel (triangle / sphere scenes,
 // every material opaque): occlusion test, while-while walk, a visibility
-// byte per ray.  5 wavefronts per SIMD: held to 80 VGPRs for 6 it was
+// byte per ray.  84 VGPRs, 5 wavefronts per SIMD: held to 80 for 6 it was
 // slower (18.7 against 18.3 ms of light passes on the 1.3M-triangle frame).
 template <bool kFlags>
 __global__ __launch_bounds__(kWaveBlock, 5) void k_light_ww(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
-    const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
+    const uint32_t n = gen_rays(a);
     trace_closest_body<0, kFlags, false, true, false, true>(a.sv, nullptr, nullptr, nullptr, nullptr, nullptr,
                                                             PVX_RAY_SHADOW | kRayOcclusion, nullptr, n, nullptr,
                                                             a.spill, nullptr, nullptr, s_stack, a.gen_groups,
@@ -82,7 +89,7 @@ __global__ __launch_bounds__(kWaveBlock, 5) void k_light_ww(TraceArgs a) {
 template <bool kFlags>
 __global__ __launch_bounds__(kWaveBlock) void k_light_bin(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
-    const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
+    const uint32_t n = gen_rays(a);
     trace_closest_body<0, kFlags, false, false, false, true, true>(
         a.sv, nullptr, nullptr, nullptr, nullptr, nullptr, PVX_RAY_SHADOW | kRayOcclusion, nullptr, n, nullptr, a.spill,
         nullptr, nullptr, s_stack, a.gen_groups, a.gen_lights, a.gen_S, a.gen_vis);
@@ -101,7 +108,7 @@ template <bool kFlags, bool kBin>
 __global__ __launch_bounds__(kWaveBlock, 5) void k_light_dyn(TraceArgs a) {
     __shared__ int32_t s_stack[kStackLds * kWaveBlock];
     const SceneView &sv = a.sv;
-    const uint32_t n = a.gen_count ? a.gen_count[0] * a.gen_S : a.n;
+    const uint32_t n = gen_rays(a);
     const uint32_t lane = threadIdx.x;
     const uint32_t gtid = blockIdx.x * kWaveBlock + lane;
     int32_t *my_spill = a.spill + (size_t)gtid * kStackSpill;
@@ -343,7 +350,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_closest_kd(TraceArgs a) {
     };
     kind &= 0xFFu; // closest hits only (the occlusion bit is a hint)
     const bool shadow = (kind == PVX_RAY_SHADOW);
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i = next_ray(i, gridDim.x * kBlock, n)) {
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
         const pvx_ray r = rays[i];
         const uint32_t rk = (kFlags && kinds) ? (uint32_t)kinds[i] : kind;
         const D3 o = d3(r.o[0], r.o[1], r.o[2]), d = d3(r.d[0], r.d[1], r.d[2]);

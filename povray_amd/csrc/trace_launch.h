@@ -87,7 +87,8 @@ struct TraceArgs {
     uint32_t gen_S;
     uint8_t *gen_vis;
     uint32_t *gen_next; // kWalkLightDyn: next ray to hand out (zero at launch)
-    const uint32_t *gen_count; // when set: n = gen_count[0] * gen_S, read on the device
+    const uint32_t *gen_count; // when set, read on the device: the groups of the whole launch
+    uint32_t gen_first;        // of them, those before this part of the launch
     // kWalkChain: ray k's colour is chain_col[3 * k]; the number of continued
     // rays is added to chain_more
     const MatRec *chain_mats;

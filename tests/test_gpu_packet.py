@@ -1,9 +1,10 @@
 """Light rays made in the traversal kernel (pvx_render on triangle / sphere
 scenes whose materials are all opaque): from the shaded points and the
-light's grid, tested for occlusion only, with the 4-wide tree walked per lane
-(PVX_TRAVERSAL_FUSED, the default; PVX_TRAVERSAL_REFILL, lanes taking new
-rays as theirs end) or by each wavefront as one packet with a shared stack
-(PVX_TRAVERSAL_PACKET).  Both give the visibility of the light
+light's grid, tested for occlusion only, through the binary tree per lane
+(PVX_TRAVERSAL_LIGHT_BINARY, the default; PVX_TRAVERSAL_REFILL_BINARY, lanes
+taking new rays as theirs end), the 4-wide tree (PVX_TRAVERSAL_FUSED and
+_REFILL) or by each wavefront as one packet with a shared stack
+(PVX_TRAVERSAL_PACKET).  All give the visibility of the light
 rays written out and traced one by one (a per-ray walk chosen with
 pvx_scene_set_traversal), so the frames are identical bit for bit, and they
 match the oracle."""
@@ -51,3 +52,25 @@ def test_packet_light_rays_equal_per_ray_walk(gpu, name):
     ok = float(np.mean(np.abs(_q(img) - _q(orc)).max(-1) <= 1))
     print(f"[packet {name}] {ok * 100:.4f}% of pixels within 1/255 of the oracle", flush=True)
     assert ok >= 0.999
+
+
+def test_more_light_rays_than_one_launch_takes(gpu):
+    # 2.07 M hits, eight lights of 16 x 16: more than 2^31 light rays, which the
+    # per-lane walks make in several launches and the packet walk in one
+    s = scenes.sphere_scene(n=60, width=1920, height=1080)
+    s.sphere_center[0], s.sphere_radius[0] = [0.0, -212.0, 0.0], 200.0  # the ground
+    s.camera = scenes.look_at_camera((0.1, 30.0, 0.0), (0.0, 0.0, 0.0), 1920, 1080)
+    s.materials["reflection"] = np.zeros_like(s.materials["reflection"])
+    s.lights = [dict(kind="area", position=np.array([8.0 * np.cos(k), 35.0, 8.0 * np.sin(k)]),
+                     axis1=np.array([3.0, 0.0, 0.0]), axis2=np.array([0.0, 0.0, 3.0]), size=(16, 16),
+                     colour=np.full(3, 0.125)) for k in range(8)]
+    gs = gpu.GpuScene(s)
+    gs.set_shading()
+    frames = []
+    for v in (A.PVX_TRAVERSAL_DEFAULT, A.PVX_TRAVERSAL_REFILL_BINARY, A.PVX_TRAVERSAL_PACKET):
+        gs.set_traversal(v, 0, A.PVX_RAY_SHADOW)
+        img, st = gs.render()
+        print(f"[light rays] walk {v}: {st['shadow_rays']} in {st['shadow_ms']:.0f} ms", flush=True)
+        assert 2**31 < st["shadow_rays"] < 2**32
+        frames.append(img)
+    assert np.array_equal(frames[0], frames[2]) and np.array_equal(frames[1], frames[2])
