@@ -15,8 +15,10 @@ this host's cores on the same rays).
 """
 import argparse
 import ctypes
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 
@@ -378,13 +380,54 @@ def bounce_leg(scene, gs, gpu_hits, host_rays, stream, steps, node_bytes):
                          "node_visits_per_ray": round(vis, 2), "prim_tests_per_ray": round(tst, 2)}}
 
 
+TRAVERSAL_SOURCES = ("trace_body.h", "trace_kernels.hip", "shapes_device.h", "poly_device.h", "pvx_types.h",
+                     "trace_launch.h", "ray_grid.h")
+
+
+def traversal_digest():
+    """Digest of the traversal kernels' code, without comments and spaces."""
+    h = hashlib.sha256()
+    for name in TRAVERSAL_SOURCES:
+        with open(os.path.join(ROOT, "povray_amd", "csrc", name)) as f:
+            text = re.sub(r"//[^\n]*|/\*.*?\*/", "", f.read(), flags=re.S)
+        h.update("".join(text.split()).encode())
+    return h.hexdigest()[:16]
+
+
+def launch_of(st, n, kernel, grid_blocks=0):
+    """What a counter summary must agree on to be of this launch: the kernel
+    and its code, the wavefronts and the tree.  Trees of depth up to 24 are
+    launched over all rays, deeper ones on grid_blocks."""
+    units = (n + 255) // 256
+    if st["bvh_depth"] + 1 > 25:
+        units = min(units, grid_blocks)
+    return {"kernel": kernel, "code": traversal_digest(), "SQ_WAVES": 4 * units, "bvh_nodes": st["n_nodes"],
+            "bvh_depth": st["bvh_depth"]}
+
+
+def counter_summary(name, launch):
+    """The committed counter summary `name`, or None where it is missing or of
+    another launch: figures made of its counts and this run's time would be
+    of neither."""
+    path = os.path.join(ROOT, "profiles", name)
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        prof = json.load(f)
+    other = [k for k, v in launch.items() if prof.get(k) != v]
+    if other:
+        log(f"profiles/{name} is of another launch ({', '.join(other)}): not used")
+        return None
+    return prof
+
+
 def configs_leg(stream, steps):
     """Closest-hit throughput of the other two single-GPU workloads: the
     1,000-sphere frame (640x480, 1 spp) and the 10,000-leaf CSG field
     (1280x720, 4 spp: four passes of camera rays at seeded sub-pixel
     offsets, one 2x2-stratified jitter per pass), plus their shaded frames.
     The CSG field's FP64 work per launch comes from the committed PMC
-    summary (profiles/fp64_csg10000.json) when present."""
+    summary (profiles/fp64_csg10000.json) when it is of this launch."""
     from povray_amd import hip, pvx, scenes
 
     out = []
@@ -413,11 +456,9 @@ def configs_leg(stream, steps):
              "frame_1spp_ms": round(fr["total_ms"], 3), "frame_closest_rays": fr["closest_rays"],
              "frame_shadow_rays": fr["shadow_rays"],
              "frame_all_rays_mrays_s": round((fr["closest_rays"] + fr["shadow_rays"]) / (fr["total_ms"] * 1e3), 1)}
-        pf = os.path.join(ROOT, "profiles", "fp64_csg10000.json")
-        if "csg" in name and os.path.exists(pf):
-            with open(pf) as f:
-                prof = json.load(f)
-            if prof.get("rays_per_launch") == n:
+        if "csg" in name:
+            prof = counter_summary("fp64_csg10000.json", launch_of(gs.stats(), n, "k_trace_ref<2, true, false, false>"))
+            if prof:
                 tf = prof["fp64_flop_per_launch"] / (ms * 1e-3) / 1e12
                 e["fp64_roofline"] = {"bound": "fp64 valu", "achieved": round(tf, 3), "peak": 78.6,
                                       "unit": "TFLOP/s", "frac": round(tf / 78.6, 4),
@@ -679,12 +720,15 @@ def main():
     multi_rad = None if (args.no_batch or args.no_batch_radiosity) else batch_radiosity_leg()
     configs = None if args.no_configs else configs_leg(stream, args.steps)
 
-    # measured HBM traffic per launch from the committed rocprofv3 PMC summary
-    traffic = None
-    tfile = os.path.join(ROOT, "profiles", f"traffic_{scene.name}.json")
-    if os.path.exists(tfile):
-        with open(tfile) as f:
-            traffic = json.load(f).get("bytes_per_launch")
+    # measured HBM traffic per launch and where the time goes instead, from
+    # the committed rocprofv3 PMC summaries of this very launch
+    walk = {A.PVX_TRAVERSAL_WIDE_WW: "k_trace_closest_ww<false, false>",
+            A.PVX_TRAVERSAL_WIDE_STEP: "k_trace_closest<0, false, false>",
+            A.PVX_TRAVERSAL_BINARY: "k_trace_closest_bin0<false, false, false>",
+            A.PVX_TRAVERSAL_BINARY_WW: "k_trace_closest_bin0<true, false, false>"}
+    launch = launch_of(st, n, walk.get(tune["variant"]), tune["grid_blocks"])
+    traffic = (counter_summary(f"traffic_{scene.name}.json", launch) or {}).get("bytes_per_launch")
+    counters = counter_summary(f"counters_{scene.name}.json", launch)
 
     cpu = None
     if not args.no_cpu:
@@ -720,14 +764,6 @@ def main():
     image_parity = None
     if not (args.no_cpu or args.no_image_parity) and scene.lights:
         image_parity = image_parity_leg(scene, gs, orc, args.cpu_threads or min(os.cpu_count() or 1, 64))
-
-    # what the hardware counters say about the same launch (committed PMC
-    # summaries): bytes that reached HBM, and where the time goes instead
-    counters = None
-    cfile = os.path.join(ROOT, "profiles", f"counters_{scene.name}.json")
-    if os.path.exists(cfile):
-        with open(cfile) as f:
-            counters = json.load(f)
 
     out = {
         "metric": "closest-hit Mrays/s",
@@ -766,9 +802,9 @@ def main():
             "hbm_measured_gbs": None if traffic is None else round(traffic / (mean_launch_ms * 1e-3) / 1e9, 1),
             "hbm_measured_frac": None if traffic is None else
             round(traffic / (mean_launch_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-            "note": "achieved counts each node and primitive fetch of every ray once (no cache credit); the "
-                    "scene fits the 256 MB Infinity Cache, so HBM sees far less (hbm_measured_*) and the "
-                    "launch is bound by issue and latency, not HBM bandwidth (counters)",
+            "note": "achieved counts each node and primitive fetch of every ray once (no cache credit), so it "
+                    "may exceed the HBM peak; the scene fits the 256 MB Infinity Cache, so HBM sees far less "
+                    "(hbm_measured_*) and the launch is bound by issue and latency, not HBM bandwidth (counters)",
             "counters": counters,
         },
         "bounce_rays": bounce,
