@@ -504,8 +504,8 @@ struct FusedArgs {
 // kOwnParams parameters or fewer a thread (a batch of 1,344 points or more)
 // the weights and moments stay in its registers for the whole run.  100 steps
 // of 2,048 points: 3.35 ms with fences and polls by every wavefront, 256
-// threads and the weights in memory; 2.0 ms so (load 1.1, forward + backward
-// 5.9, gradient tiles 2.1, barrier 3.8, reduction + Adam 3.1, barrier 3.8 us
+// threads and the weights in memory; 2.1 ms so (load 1.1, forward + backward
+// 5.9, gradient tiles 2.1, barrier 4.4, reduction + Adam 3.1, barrier 4.4 us
 // a step).
 template <bool kOwn>
 __global__ __launch_bounds__(kTrainThreads) void k_mlp_train(FusedArgs a) {
